@@ -17,10 +17,8 @@ import sys
 
 import numpy as np
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-for _p in (ROOT, os.path.join(ROOT, "autodiff-ir-rust_amd")):
-    if _p not in sys.path:
-        sys.path.insert(0, _p)
+# the package's folder, in the tree that is the working folder
+sys.path.insert(0, os.path.join(os.getcwd(), "autodiff-ir-rust_amd"))
 
 from adhip import autodiff, ir as IR, nn, workloads  # noqa: E402
 from adhip.core import concat, constant  # noqa: E402
