@@ -1,4 +1,5 @@
-// FP32 matrix product for gfx950 on the matrix cores (v_mfma_f32_32x32x2_f32), LDS-tiled.
+// FP32 matrix product for gfx950 on the FP32 matrix cores (v_mfma_f32_32x32x2_f32), LDS-tiled: the kernel of products
+// whose k is shorter than 32.  Longer ones run on the bf16 matrix cores (gemm_split.cpp), which share its interface.
 //
 // The reference multiplies with one work-item per output element, a sequential k loop and two
 // global loads per multiply-add (reference src/devices/opencl/kernels/dotprod.rs:23-53); transposed
@@ -16,7 +17,16 @@
 
 namespace adhip {
 
-std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue) {
+int gemm_tile_columns(const GemmConfig& cfg) { return cfg.bn ? cfg.bn : (cfg.bm == 64 ? 64 : 128); }
+
+// 32x32 blocks of a wavefront's sub-tile, in rows and columns
+static int wave_rows(const GemmConfig& cfg) { return cfg.bm == 256 && cfg.bf16_parts ? 4 : cfg.bm == 64 ? 1 : 2; }
+static int wave_columns(const GemmConfig& cfg) { return gemm_tile_columns(cfg) == 64 ? 1 : 2; }
+unsigned gemm_threads(const GemmConfig& cfg) {
+    return 64u * (unsigned)((cfg.bm / (32 * wave_rows(cfg))) * (gemm_tile_columns(cfg) / (32 * wave_columns(cfg))) * cfg.k_waves);
+}
+
+std::string gemm_kernel_head(const GemmConfig& cfg, const GemmEpilogue* epilogue) {
     std::string s;
     if (epilogue) s += epilogue->prelude;
     s += strf("#define STORE_C %d\n#define EPI_PARAMS %s\n", (!epilogue || epilogue->store_c) ? 1 : 0,
@@ -45,12 +55,18 @@ std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, 
         }
         s += "#define GROUP_PARAMS " + params + "\n#define GROUP_PICK " + pick + " default: return; }\n";
     }
+    return s;
+}
+
+std::string gemm_tile_head(const GemmConfig& cfg, const std::string& entry) {
+    return strf("#define KERNEL_NAME %s\n#define BM %d\n#define BN %d\n#define TM %d\n#define TN %d\n#define NT %u\n", entry.c_str(), cfg.bm,
+                gemm_tile_columns(cfg), wave_rows(cfg), wave_columns(cfg), gemm_threads(cfg));
+}
+
+std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue) {
+    std::string s = gemm_kernel_head(cfg, epilogue);
     // tile geometry: BM x BN block tile, TM x TN MFMA blocks per wave, WGN waves along n
-    const int bn = cfg.bn ? cfg.bn : (cfg.bm == 64 ? 64 : 128);
-    const int tm = cfg.bm == 64 ? 1 : 2, tn = (bn == 64) ? 1 : 2;
-    const int waves = (cfg.bm / (32 * tm)) * (bn / (32 * tn));
-    s += strf("#define KERNEL_NAME %s\n#define BM %d\n#define BN %d\n#define TM %d\n#define TN %d\n#define NT %d\n", entry.c_str(),
-              cfg.bm, bn, tm, tn, waves * 64);
+    s += gemm_tile_head(cfg, entry);
     {
         // diagnostic: ADHIP_GEMM_AHEAD=1 keeps the global loads one k-tile ahead of the MFMAs instead of two
         int ahead = 2;
@@ -110,20 +126,14 @@ static __device__ __forceinline__ float4_t edge_load4(const float* p, long long 
 // EDGE: M, N or K is not a multiple of the tile, or an operand is not 16-byte aligned.  Stores are bounds-checked;
 // loads go through edge_load4 where an element may not exist (all of them without EDGE_VEC; with it, only the last
 // ragged k-tile and quads that straddle the end of M or N).
-// SPLITK: the block at blockIdx.y multiplies only k in [y*k_chunk, (y+1)*k_chunk) and writes slice y of a
-// [gridDim.y][M][N] buffer; the caller adds the slices in a fixed order.  For products whose output alone gives
-// too few blocks to hide the latency of the operand loads.
 // GROUPED: several independent products of one shape and one set of strides in a single launch; the block row
 // blockIdx.y works on problem y, whose three base pointers (operand offsets already applied) are parameters
 // c<y>, a<y>, b<y>.  For the same kind of product when there are many of them (the per-head projections of
-// multi-head attention).  With SPLITK the range of k is picked by blockIdx.z.
+// multi-head attention).
 extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
 #if GROUPED
     const int* __restrict__ guard, GROUP_PARAMS long long M, long long N, long long K, long long a_sm, long long a_sk,
     long long b_sk, long long b_sn
-#if SPLITK
-    , long long k_chunk
-#endif
     ) {
     if (guard && *guard == 0) return;
     float* __restrict__ C;
@@ -135,24 +145,10 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     const int* __restrict__ guard, float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ B,
     long long M, long long N, long long K, long long a_off, long long a_sm, long long a_sk, long long b_off,
     long long b_sk, long long b_sn
-#if SPLITK
-    , long long k_chunk
-#endif
     EPI_PARAMS) {
     if (guard && *guard == 0) return;
 #endif
-#if SPLITK
-#if GROUPED
-    const unsigned slice = blockIdx.z;  // c<y> points at problem y's own [gridDim.z][M][N] slices
-#else
-    const unsigned slice = blockIdx.y;
-#endif
-    const long long k_lo = (long long)slice * k_chunk;
-    const long long k_hi = min(K, k_lo + k_chunk);
-    C += (long long)slice * M * N;
-#else
     const long long k_lo = 0, k_hi = K;
-#endif
     __shared__ __attribute__((aligned(16))) float As[2][BK][LDA];
     __shared__ __attribute__((aligned(16))) float Bs[2][BK][LDB];
 

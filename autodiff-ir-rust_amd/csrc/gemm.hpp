@@ -12,6 +12,9 @@ struct GemmConfig {
     int bm = 128;           // block tile: 256 (256x128, 8 waves), 128 (128x128, 4 waves) or 64 (64x64, 4 waves); k depth 16
     int bn = 0;             // block tile columns; 0 = the default for bm (128, or 64 for bm 64).  128x64 is the only other shape
     bool split_k = false;   // blockIdx.y picks a range of k (extra argument k_chunk); slice y of the product goes to C + y*M*N
+    bool bf16_parts = false;  // the kernel on the bf16 matrix cores (gemm_split.cpp); needs K >= bk
+    int bk = 16;            // k depth of its tiles (16, 32 or 64)
+    int k_waves = 1;        // of that kernel: 2 = a tile's k is shared between two sets of wavefronts, whose sums are added at the end
     bool grouped = false;   // blockIdx.y picks one of kGemmGroupSlots products of the same shape (parameters c<i>, a<i>, b<i>)
 };
 
@@ -28,6 +31,14 @@ struct GemmEpilogue {
     bool store_c = true;
 };
 
+// What both kernels of a configuration share: the epilogue as a macro, the switches, the choice among grouped problems.
+std::string gemm_kernel_head(const GemmConfig& cfg, const GemmEpilogue* epilogue);
+std::string gemm_tile_head(const GemmConfig& cfg, const std::string& entry);
+int gemm_tile_columns(const GemmConfig& cfg);
+unsigned gemm_threads(const GemmConfig& cfg);
+
 std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr);
+// The same product on the bf16 matrix cores, every operand split into three bf16 parts (gemm_split.cpp).
+std::string gemm_split_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr);
 
 }  // namespace adhip

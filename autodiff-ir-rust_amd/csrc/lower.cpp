@@ -3174,41 +3174,11 @@ struct Lowerer {
         }
     }
 
-    // Tile and k ranges of a grouped launch of `cnt` products shaped like `first`: by the number of blocks the whole
-    // launch has, as plan_dot does for a single product.
     static DotLaunchPlan plan_dot_group(const Node* first, int cnt) {
         std::array<int64_t, 8> key{};
         ADHIP_CHECK(dot_group_key(first, key), "internal: grouped launch of a product that does not qualify");
-        const int64_t M = key[0], N = key[1], K = key[2];
-        DotLaunchPlan pl;
-        GemmConfig& cfg = pl.cfg;
-        cfg.a_kcontig = key[4] == 1;
-        cfg.b_kcontig = key[5] == 1;
-        cfg.grouped = true;
-        const int64_t blocks128 = ((M + 127) / 128) * ((N + 127) / 128) * cnt;
-        const int64_t max_splits = std::min<int64_t>(K / 256, 32);
-        auto splits_for = [&](int64_t blocks) {
-            if (blocks >= 256 || max_splits < 2) return (int64_t)1;
-            return std::max<int64_t>(std::min<int64_t>((512 + blocks - 1) / blocks, max_splits), 1);
-        };
-        // three 64x64 blocks per CU without cutting k beat 128x128 blocks with k cut and the slice sum that follows
-        // (12 x 2048x128x1024: 66 us against 77 + 8); with two per CU it is the other way round (8 x 2048x128x2048:
-        // 105-118 us against 80 + 7)
-        const int64_t blocks64 = ((M + 63) / 64) * ((N + 63) / 64) * cnt;
-        const bool small_whole = blocks128 < 256 && blocks64 >= 768;
-        cfg.bm = (!small_whole && blocks128 * splits_for(blocks128) >= 256) ? 128 : 64;
-        pl.bn_tile = cfg.bm == 64 ? 64 : 128;
-        if (cfg.bm == 128 && blocks128 < 512 && splits_for(blocks128) == 1) { pl.bn_tile = 64; cfg.bn = 64; }
-        cfg.edge = key[7] || (M % cfg.bm) || (N % pl.bn_tile);
-        cfg.edge_vec = key[7] != 2;
-        const int64_t blocks = ((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile) * cnt;
-        const int64_t want = small_whole ? 1 : splits_for(blocks);
-        if (want > 1) {
-            pl.k_chunk = (((K + want - 1) / want) + 15) / 16 * 16;
-            pl.splits = (K + pl.k_chunk - 1) / pl.k_chunk;
-            cfg.split_k = pl.splits > 1;
-            if (!cfg.split_k) pl.splits = 1;
-        }
+        DotLaunchPlan pl = plan_product(key[0], key[1], key[2], cnt, key[4] == 1, key[5] == 1, (int)key[7]);
+        pl.cfg.grouped = true;
         return pl;
     }
 
@@ -3225,11 +3195,10 @@ struct Lowerer {
         const GemmConfig& cfg = pl.cfg;
         ADHIP_CHECK(cfg.split_k == (partial != nullptr), "internal: split grouped product and its slice buffer disagree");
         ADHIP_CHECK(!partial || numel(partial->shape) == (int64_t)cnt * pl.splits * M * N, "internal: slice buffer of the wrong size");
-        std::string entry = strf("adhip_gemm_%c%c_%d%s%s%s_grouped", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', cfg.bm,
-                                 cfg.bn == 64 && cfg.bm != 64 ? "x64" : "", cfg.edge ? (cfg.edge_vec ? "_rim" : "_edge") : "", cfg.split_k ? "_splitk" : "");
+        const std::string entry = dot_kernel_name(cfg) + "_grouped";
         Launch l;
-        l.kernel = add_kernel(entry, gemm_kernel_source(cfg, entry), "dot_mfma");
-        l.block[0] = cfg.bm == 64 ? 256u : (unsigned)(cfg.bm * 2);
+        l.kernel = add_kernel(entry, gemm_source(cfg, entry), "dot_mfma");
+        l.block[0] = gemm_threads(cfg);
         l.grid[0] = (unsigned)(((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile));
         l.grid[1] = (unsigned)cnt;
         l.grid[2] = (unsigned)pl.splits;
@@ -3354,56 +3323,97 @@ struct Lowerer {
         tref_affine2d(n->in[0], a);
         tref_affine2d(n->in[1], b);
         const int64_t M = n->shape[0], N = n->shape[1], K = n->in[0].shape[1];
+        return plan_product(M, N, K, 1, a.s1 == 1, b.s0 == 1, dot_alignment(a, b, M, N, K));
+    }
+
+    // Tile and k ranges of a launch of `cnt` products of one shape (`alignment` as dot_alignment gives it).
+    static DotLaunchPlan plan_product(int64_t M, int64_t N, int64_t K, int64_t cnt, bool a_kcontig, bool b_kcontig, int alignment) {
         DotLaunchPlan pl;
         GemmConfig& cfg = pl.cfg;
-        cfg.a_kcontig = a.s1 == 1;
-        cfg.b_kcontig = b.s0 == 1;
-        const int alignment = dot_alignment(a, b, M, N, K);
-        const bool unaligned = alignment != 0;
-        // the largest block tile that still puts enough blocks on the chip's 256 CUs: 256x128 (8 waves) with at
-        // least two blocks per CU, 128x128 with at least one -- counting the ranges k can be cut into (each at
-        // least 256 deep; the slices are added afterwards) -- else 64x64, cut the same way.  A block that has a CU
-        // to itself cannot hide the latency of its operand loads, hence the target of about 512 blocks.
-        const int64_t blocks128 = ((M + 127) / 128) * ((N + 127) / 128);
+        cfg.a_kcontig = a_kcontig;
+        cfg.b_kcontig = b_kcontig;
+        auto blocks = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * cnt; };
+        const int64_t blocks128 = blocks(128, 128), blocks64 = blocks(64, 64);
+        cfg.bf16_parts = K >= 32;
+        if (!cfg.bf16_parts) {
+            // a tile of k or less: a launch that stores, on the FP32 matrix cores (below k = 8 the parts' six roundings
+            // are more than the k / 2 of an FP32 chain)
+            if (!alignment && M % 256 == 0 && N % 128 == 0 && blocks(256, 128) >= 512) cfg.bm = 256;
+            else cfg.bm = blocks128 >= 256 ? 128 : 64;
+            if (cfg.bm == 128 && blocks128 < 512) cfg.bn = 64;
+            pl.bn_tile = gemm_tile_columns(cfg);
+            cfg.edge = alignment || (M % cfg.bm) || (N % pl.bn_tile);
+            cfg.edge_vec = alignment != 2;
+            return pl;
+        }
         const int64_t max_splits = std::min<int64_t>(K / 256, 32);
-        auto splits_for = [&](int64_t blocks) {
-            if (blocks >= 256 || max_splits < 2) return (int64_t)1;
-            return std::max<int64_t>(std::min<int64_t>((512 + blocks - 1) / blocks, max_splits), 1);
+        auto tile = [&](int bm, int bn, int bk, int k_waves) {
+            cfg.bm = bm;
+            cfg.bn = bn;
+            cfg.bk = bk;
+            cfg.k_waves = k_waves;
         };
-        // An output of 512 and more 64x64 tiles but fewer than 256 of 128x128, with k up to 2048: the small tile, whole,
-        // beats the large one with k cut in four and the slices added afterwards (2048 x 1024 x 1024: 38.5 us against
-        // 39.1 + 6.4; at k = 4096 the large tile's better rate has made up for the slice sum: 139.6 against 131.3 + 6.4).
-        const int64_t blocks64 = ((M + 63) / 64) * ((N + 63) / 64);
-        const bool small_whole = blocks128 < 256 && blocks64 >= 512 && K <= 2048;
-        if (!unaligned && M % 256 == 0 && N % 128 == 0 && (M / 256) * (N / 128) >= 512) cfg.bm = 256;
-        else if (!small_whole && blocks128 * splits_for(blocks128) >= 256) cfg.bm = 128;
-        else cfg.bm = 64;
-        pl.bn_tile = cfg.bm == 64 ? 64 : 128;
-        // one 128x128 block per CU is too few to hide its own latencies: halve the tile's width for two per CU
-        if (cfg.bm == 128 && blocks128 < 512 && splits_for(blocks128) == 1) { pl.bn_tile = 64; cfg.bn = 64; }
-        // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits> forces tile and k ranges of every aligned product the tile divides
-        int64_t forced_splits = 0;
+        int64_t want = 1;
+        // Time of a launch in whole rounds of the chip's 256 CUs: 256x256 blocks one per CU at 215 TFLOP/s, 128x128 ones
+        // two per CU at 180 (4096^3: 640 and 770 us, against 1090 on the FP32 matrix cores).
+        const int64_t blocks256 = blocks(256, 256);
+        const double t256 = (double)((blocks256 + 255) / 256) * 65536 / 215, t128 = (double)((blocks128 + 511) / 512) * 32768 / 180;
+        if (blocks256 >= 200 && t256 <= t128) tile(256, 256, 16, 1);
+        else if (blocks128 >= 512) tile(128, 128, 16, 1);
+        else if (blocks128 >= 256 && K < 512) tile(128, 64, 32, 1);   // (2048 x 2048 x 512: 38 us against 31; at k = 260 both 35)
+        else if (blocks128 >= 256) tile(128, 128, 32, 2);
+        // Two 64x64 blocks and more per CU without cutting k beat the large tile with k cut and the slice sum behind it
+        // while k is short (2048 x 1024 x 1024: 40 us against 33 + 6, and it keeps the epilogue; at 2048 80 against 50 + 6).
+        else if (blocks64 >= 512 && K <= 1024) tile(64, 64, 32, 1);
+        else if (blocks128 * max_splits >= 256) {
+            // one block per CU: as many ranges as fill whole rounds best, each at least 256 deep; the slice sum is
+            // worth some 6 us, a round of the whole k 0.045 us per k
+            tile(128, 128, 32, 2);
+            double best = 0;
+            for (int64_t c = 1; c <= max_splits; ++c) {
+                const double t = (double)((blocks128 * c + 255) / 256) * (0.045 * (double)K / (double)c + 3) + (c > 1 ? 6 : 0);
+                if (c == 1 || t < best) { best = t; want = c; }
+            }
+        } else {
+            // few small tiles: a tile's time is the latency of its chain of k-tiles.  Cut from k = 1024 on (at 784
+            // 1000 x 500 takes 22 us whole against 15 + 5 and keeps its epilogue)
+            if (K >= 1024 && blocks64 < 256) want = std::max<int64_t>(std::min<int64_t>((512 + blocks64 - 1) / blocks64, max_splits), 1);
+            if (want == 1 && blocks64 <= 256 && K >= 64) tile(64, 64, 64, 2);
+            else tile(64, 64, 32, 1);
+        }
+        // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits> forces tile and k ranges of every product with k of 64 and more
         if (const char* e = getenv("ADHIP_DOT_PLAN")) {
             long fbm = 0, fbn = 0, fs = 0;
-            if (sscanf(e, "%ld,%ld,%ld", &fbm, &fbn, &fs) == 3 && !unaligned && (fbm == 256 || fbm == 128 || fbm == 64) &&
-                (fbn == 128 || fbn == 64) && M % fbm == 0 && N % fbn == 0 && fs >= 1 && !(fbm == 256 && fbn != 128) && !(fbm == 64 && fbn != 64)) {
-                cfg.bm = (int)fbm;
-                pl.bn_tile = (int)fbn;
-                cfg.bn = (fbm == 128 && fbn == 64) ? 64 : 0;
-                forced_splits = fs;
+            if (sscanf(e, "%ld,%ld,%ld", &fbm, &fbn, &fs) == 3 && K >= 64 && fs >= 1) {
+                const bool known = (fbm == 256 && fbn == 256) || (fbm == 128 && (fbn == 128 || fbn == 64)) || (fbm == 64 && fbn == 64);
+                if (known) {
+                    tile((int)fbm, (int)fbn, fbm == 256 ? 16 : 32, fbm == 128 && fbn == 128 ? 2 : 1);
+                    want = std::min<int64_t>(fs, K / 64);
+                }
             }
         }
-        cfg.edge = unaligned || (M % cfg.bm) || (N % pl.bn_tile);
-        cfg.edge_vec = alignment != 2;
-        const int64_t blocks = ((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile);
-        const int64_t want = forced_splits ? std::min<int64_t>(forced_splits, std::max<int64_t>(K / 64, 1)) : (cfg.bm == 256 || small_whole ? 1 : splits_for(blocks));
+        pl.bn_tile = cfg.bn;
         if (want > 1) {
-            pl.k_chunk = (((K + want - 1) / want) + 15) / 16 * 16;
+            pl.k_chunk = (((K + want - 1) / want) + cfg.bk - 1) / cfg.bk * cfg.bk;
             pl.splits = (K + pl.k_chunk - 1) / pl.k_chunk;
             cfg.split_k = pl.splits > 1;
             if (!cfg.split_k) pl.splits = 1;
         }
+        cfg.edge = alignment || (M % cfg.bm) || (N % cfg.bn) || (K % cfg.bk);
         return pl;
+    }
+
+    static std::string dot_kernel_name(const GemmConfig& cfg) {
+        std::string s = strf("adhip_gemm_%c%c_%d", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', cfg.bm);
+        if (cfg.bm != 64 && gemm_tile_columns(cfg) == 64) s += "x64";
+        if (cfg.edge) s += cfg.bf16_parts || cfg.edge_vec ? "_rim" : "_edge";
+        if (cfg.split_k) s += "_splitk";
+        else if (cfg.k_waves == 2) s += "_pair";
+        if (!cfg.bf16_parts) s += "_f32";
+        return s;
+    }
+    static std::string gemm_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr) {
+        return cfg.bf16_parts ? gemm_split_kernel_source(cfg, entry, epilogue) : gemm_kernel_source(cfg, entry, epilogue);
     }
 
     void emit_dot(Node* n, std::vector<Step>& out, const DotEpilogueCode* epi = nullptr, bool store_c = true,
@@ -3421,8 +3431,7 @@ struct Lowerer {
             GemmConfig cfg = pl.cfg;
             const int bn_tile = pl.bn_tile;
             ADHIP_CHECK(!cfg.split_k || (partial && !epi), "internal: split product without its slice buffer");
-            std::string entry = strf("adhip_gemm_%c%c_%d%s%s%s", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', cfg.bm,
-                                     cfg.bn == 64 && cfg.bm != 64 ? "x64" : "", cfg.edge ? (cfg.edge_vec ? "_rim" : "_edge") : "", cfg.split_k ? "_splitk" : "");
+            std::string entry = dot_kernel_name(cfg);
             Launch l;
             if (epi) {
                 // the element-wise group that followed the product runs on the accumulators; every distinct
@@ -3433,11 +3442,11 @@ struct Lowerer {
                 ge.params = epi->params;
                 ge.code = epi->code;
                 ge.store_c = store_c;
-                l.kernel = add_kernel(entry, gemm_kernel_source(cfg, entry, &ge), "dot_mfma");
+                l.kernel = add_kernel(entry, gemm_source(cfg, entry, &ge), "dot_mfma");
             } else {
-                l.kernel = add_kernel(entry, gemm_kernel_source(cfg, entry), "dot_mfma");
+                l.kernel = add_kernel(entry, gemm_source(cfg, entry), "dot_mfma");
             }
-            l.block[0] = cfg.bm == 64 ? 256u : (unsigned)(cfg.bm * 2);
+            l.block[0] = gemm_threads(cfg);
             l.grid[0] = (unsigned)(((M + cfg.bm - 1) / cfg.bm) * ((N + bn_tile - 1) / bn_tile));
             // a product that is not stored has no buffer; the kernel never touches C then
             Node* c_arg = cfg.split_k ? partial : (store_c ? n : (epi ? epi->buffer_args[0] : n));
