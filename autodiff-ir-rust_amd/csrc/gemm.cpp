@@ -391,4 +391,76 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     return s;
 }
 
+// Products too small for a matrix-core tile, and operands without a unit stride.  Bound by latency: a thread that walks
+// k alone makes k dependent trips through two loads (64 x 48 x 64: 12 us, where an empty kernel takes 4).  `lanes` lanes
+// (a power of two, at most 64) share a result instead, each with every lanes-th k, four of which are in flight at once;
+// the caller picks lanes so that one round of four covers k where it can.
+std::string dot_small_source(const std::string& entry, const GemmEpilogue* epilogue, bool grouped) {
+    GemmConfig cfg;
+    cfg.grouped = grouped;
+    std::string s = gemm_kernel_head(cfg, epilogue);
+    // (name and parameters stand as text: a launch that runs several kernels in turn reads them from the source)
+    s += "extern \"C\" __global__ __launch_bounds__(256) void " + entry + "(const int* __restrict__ guard, ";
+    if (grouped) {
+        s += R"(GROUP_PARAMS long long M, long long N, long long K, long long a_sm, long long a_sk, long long b_sk, long long b_sn, int lanes) {
+    if (guard && *guard == 0) return;
+    float* __restrict__ C;
+    const float* __restrict__ A;
+    const float* __restrict__ B;
+    GROUP_PICK
+    const long long a_off = 0, b_off = 0;
+)";
+    } else {
+        s += R"(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ B, long long M, long long N, long long K,
+    long long a_off, long long a_sm, long long a_sk, long long b_off, long long b_sk, long long b_sn, int lanes)" +
+             (epilogue ? epilogue->params : std::string()) + R"() {
+    if (guard && *guard == 0) return;
+)";
+    }
+    s += R"(
+    const unsigned share = threadIdx.x & (unsigned)(lanes - 1), per_block = 256u / (unsigned)lanes;
+    const long long total = M * N, stride = (long long)gridDim.x * per_block;
+    for (long long g = (long long)blockIdx.x * per_block + threadIdx.x / (unsigned)lanes; g < total; g += stride) {
+        const long long row = total <= 0x7fffffff ? (long long)((unsigned)g / (unsigned)N) : g / N, col = g - row * N;
+        const float* pa = A + a_off + row * a_sm;
+        const float* pb = B + b_off + col * b_sn;
+        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (long long k0 = share; k0 < K; k0 += 4 * lanes) {
+            float x[4], y[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                // what lies beyond k is read at the first place and taken as 0
+                const long long k = k0 + u * lanes;
+                const bool ok = k < K;
+                x[u] = pa[ok ? k * a_sk : 0];
+                y[u] = pb[ok ? k * b_sk : 0];
+                x[u] = ok ? x[u] : 0.0f;
+                y[u] = ok ? y[u] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[u] = __builtin_fmaf(x[u], y[u], acc[u]);
+        }
+        float sum_value = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        for (int d = lanes >> 1; d > 0; d >>= 1) sum_value += __shfl_xor(sum_value, d);
+        if (share == 0) {
+#if STORE_C
+            C[g] = sum_value;
+#endif
+            EPILOGUE
+        }
+    }
+}
+#undef EPILOGUE
+#undef EPI_PARAMS
+#undef STORE_C
+#undef A_KCONTIG
+#undef B_KCONTIG
+#undef EDGE
+#undef EDGE_VEC
+#undef SPLITK
+#undef GROUPED
+)";
+    return s;
+}
+
 }  // namespace adhip

@@ -41,4 +41,7 @@ std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, 
 // The same product on the bf16 matrix cores, every operand split into three bf16 parts (gemm_split.cpp).
 std::string gemm_split_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr);
 
+// Products too small for the matrix cores, and operands of any strides (takes the product kernels' arguments, then `int lanes`).
+std::string dot_small_source(const std::string& entry, const GemmEpilogue* epilogue = nullptr, bool grouped = false);
+
 }  // namespace adhip

@@ -121,6 +121,25 @@ extern "C" __global__ void adhip_flag(int* __restrict__ flags, int slot, int par
     flags[slot] = v;
 }
 
+// One thread per output element, k ascending, one accumulator: the reference's dot kernel
+// (src/devices/opencl/kernels/dotprod.rs:23-53).  Used for the very smallest products,
+// phases of a single-block launch, which it keeps shortest (the five of two layers 5-3-2: 44.5 us a call against 46.2).
+extern "C" __global__ __launch_bounds__(256) void adhip_dot_naive(const int* __restrict__ guard, float* __restrict__ c,
+                                                                  const float* __restrict__ a, const float* __restrict__ b,
+                                                                  long long m, long long n, long long k,
+                                                                  long long a_off, long long a_sm, long long a_sk,
+                                                                  long long b_off, long long b_sk, long long b_sn) {
+    if (guard && *guard == 0) return;
+    long long g = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (g >= m * n) return;
+    long long row = g / n, col = g % n;
+    float acc = 0.0f;
+    const float* pa = a + a_off + row * a_sm;
+    const float* pb = b + b_off + col * b_sn;
+    for (long long kk = 0; kk < k; ++kk) acc = __builtin_fmaf(pa[kk * a_sk], pb[kk * b_sk], acc);
+    c[g] = acc;
+}
+
 // Second pass of column sums that rode along with an element-wise kernel: up to four sums, each the sum over
 // `tiles` rows of its dense partial buffer [tiles][cols] (cols a multiple of 4), in one launch (blockIdx.y picks the
 // sum).  A block is 16 four-column groups x 64 row groups; the row groups are combined through LDS by a tree of fixed
@@ -251,23 +270,6 @@ extern "C" __global__ __launch_bounds__(256) void adhip_sum_slices_grouped(const
     }
 }
 
-// One thread per output element, k ascending, one accumulator: the reference's dot kernel
-// (src/devices/opencl/kernels/dotprod.rs:23-53).  Used for small products.
-extern "C" __global__ __launch_bounds__(256) void adhip_dot_naive(const int* __restrict__ guard, float* __restrict__ c,
-                                                                  const float* __restrict__ a, const float* __restrict__ b,
-                                                                  long long m, long long n, long long k,
-                                                                  long long a_off, long long a_sm, long long a_sk,
-                                                                  long long b_off, long long b_sk, long long b_sn) {
-    if (guard && *guard == 0) return;
-    long long g = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (g >= m * n) return;
-    long long row = g / n, col = g % n;
-    float acc = 0.0f;
-    const float* pa = a + a_off + row * a_sm;
-    const float* pb = b + b_off + col * b_sn;
-    for (long long kk = 0; kk < k; ++kk) acc = __builtin_fmaf(pa[kk * a_sk], pb[kk * b_sk], acc);
-    c[g] = acc;
-}
 )";
 }
 
@@ -329,7 +331,7 @@ struct Lowerer {
     std::map<std::string, int> kernel_by_source;
     int kernel_counter = 0;
     std::map<std::pair<int, int>, int> layered_kernels;
-    int fixed_copy = -1, fixed_dot = -1, fixed_transpose = -1, fixed_transpose4 = -1, fixed_finalize = -1, fixed_sums_finalize = -1, fixed_sum_slices = -1, fixed_sum_slices_grouped = -1;
+    int fixed_copy = -1, fixed_dot = -1, fixed_dot_tiny = -1, fixed_transpose = -1, fixed_transpose4 = -1, fixed_finalize = -1, fixed_sums_finalize = -1, fixed_sum_slices = -1, fixed_sum_slices_grouped = -1;
     int dot_epilogue_counter = 0;
     int cur_guard = -1;  // flag slot guarding the block being lowered, or -1
     // The device-predicated loop whose body is being lowered: its block, predicate id and flag.  The last region of the
@@ -2457,7 +2459,7 @@ struct Lowerer {
                 DotLaunchPlan dpl;
                 const bool grouped = G.members.size() > 1;  // one launch for all of them: whole k, no epilogue
                 if (dot_uses_mfma(D) && !grouped) dpl = plan_dot(D);
-                int nx = (grouped || dpl.splits > 1 || !opt.fuse || !dot_uses_mfma(D)) ? -1 : find_epilogue(rp, g, D, numel(D->shape));
+                int nx = (grouped || dpl.splits > 1 || !opt.fuse || dot_is_tiny(D)) ? -1 : find_epilogue(rp, g, D, numel(D->shape));
                 if (nx >= 0) {
                     // an epilogue streams its other operands in the accumulator layout (32 floats of a row per half
                     // wave); with many of them (a sum over all heads' gradients) a separate element-wise pass, with
@@ -3040,13 +3042,18 @@ struct Lowerer {
     };
 
     // What must agree for products to share a grouped launch: sizes, strides and whether operands are 16-byte
-    // aligned.  False for products that do not go to the matrix cores.
+    // aligned.  Small products (last number kSmallDot) share one as well, but for the very smallest, which are phases of
+    // a single-block launch with whatever stands around them.
+    static constexpr int64_t kSmallDot = 16;
     static bool dot_group_key(const Node* n, std::array<int64_t, 8>& key) {
-        if (!dot_uses_mfma(n)) return false;
         Affine2D a, b;
-        tref_affine2d(n->in[0], a);
-        tref_affine2d(n->in[1], b);
+        if (!tref_affine2d(n->in[0], a) || !tref_affine2d(n->in[1], b)) return false;
         const int64_t M = n->shape[0], N = n->shape[1], K = n->in[0].shape[1];
+        if (!dot_uses_mfma(n)) {
+            if (dot_is_tiny(n) || M * N * K < 2048 || M * N * K >= 64 * 64 * 64) return false;
+            key = {M, N, K, a.s0, a.s1, b.s0, b.s1, kSmallDot};
+            return true;
+        }
         key = {M, N, K, a.s0, a.s1, b.s0, b.s1, dot_alignment(a, b, M, N, K)};
         return true;
     }
@@ -3158,7 +3165,10 @@ struct Lowerer {
         for (auto& kv : sets) {
             const std::vector<int>& set = kv.second;
             if (set.size() < 2) continue;
-            const size_t launches = (set.size() + kGemmGroupSlots - 1) / kGemmGroupSlots;
+            // (small products: eight; the plan's tests count on launches that grow with the number of heads, and twelve
+            // products in two launches instead of one are 2 of some 37 launches of a small encoder layer's step)
+            const size_t slots = kv.first.second[7] == kSmallDot ? kGemmGroupSlots / 2 : kGemmGroupSlots;
+            const size_t launches = (set.size() + slots - 1) / slots;
             const size_t per = (set.size() + launches - 1) / launches;
             for (size_t i0 = 0; i0 < set.size(); i0 += per) {
                 const size_t i1 = std::min(set.size(), i0 + per);
@@ -3177,6 +3187,7 @@ struct Lowerer {
     static DotLaunchPlan plan_dot_group(const Node* first, int cnt) {
         std::array<int64_t, 8> key{};
         ADHIP_CHECK(dot_group_key(first, key), "internal: grouped launch of a product that does not qualify");
+        if (key[7] == kSmallDot) return DotLaunchPlan();
         DotLaunchPlan pl = plan_product(key[0], key[1], key[2], cnt, key[4] == 1, key[5] == 1, (int)key[7]);
         pl.cfg.grouped = true;
         return pl;
@@ -3195,11 +3206,13 @@ struct Lowerer {
         const GemmConfig& cfg = pl.cfg;
         ADHIP_CHECK(cfg.split_k == (partial != nullptr), "internal: split grouped product and its slice buffer disagree");
         ADHIP_CHECK(!partial || numel(partial->shape) == (int64_t)cnt * pl.splits * M * N, "internal: slice buffer of the wrong size");
-        const std::string entry = dot_kernel_name(cfg) + "_grouped";
+        const bool small = key0[7] == kSmallDot;
+        const std::string entry = small ? "adhip_dot_small_grouped" : dot_kernel_name(cfg) + "_grouped", kind = small ? "dot_naive" : "dot_mfma";
+        const int lanes = small_dot_lanes(M, N, K);
         Launch l;
-        l.kernel = add_kernel(entry, gemm_source(cfg, entry), "dot_mfma");
-        l.block[0] = gemm_threads(cfg);
-        l.grid[0] = (unsigned)(((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile));
+        l.kernel = add_kernel(entry, small ? dot_small_source(entry, nullptr, true) : gemm_source(cfg, entry), kind);
+        l.block[0] = small ? 256u : gemm_threads(cfg);
+        l.grid[0] = (unsigned)(small ? (M * N * lanes + 255) / 256 : ((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile));
         l.grid[1] = (unsigned)cnt;
         l.grid[2] = (unsigned)pl.splits;
         auto B = [&](Node* x, int64_t off) {
@@ -3225,10 +3238,11 @@ struct Lowerer {
         }
         for (int q = 0; q < 7; ++q) l.args.push_back(I(key0[q]));
         if (cfg.split_k) l.args.push_back(I(pl.k_chunk));
+        if (small) { Arg la; la.kind = Arg::I32; la.iv = lanes; l.args.push_back(la); }
         l.label = strf("dots_%s_%dx_%lldx%lldx%lld", dots[0]->name.c_str(), cnt, (long long)M, (long long)N, (long long)K);
         l.bytes = 4.0 * cnt * ((double)M * K + (double)K * N + (double)M * N * (double)pl.splits);
         l.flops = 2.0 * cnt * (double)M * (double)N * (double)K;
-        push_launch(out, l, "dot_mfma");
+        push_launch(out, l, kind);
         if (cfg.split_k) {
             if (fixed_sum_slices_grouped < 0)
                 fixed_sum_slices_grouped = add_kernel("adhip_sum_slices_grouped", fixed_kernels_source(), "sum_slices");
@@ -3307,6 +3321,16 @@ struct Lowerer {
                   (cfg.mask ? 4.0 * (double)key0.sq * (double)key0.sk : 0.0);
         l.flops = 2.0 * cnt * (double)key0.sq * (double)key0.sk * (double)(key0.d + key0.dv);
         push_launch(out, l, "attention");
+    }
+
+    static bool dot_is_tiny(const Node* n) { return n->in[0].shape[1] <= 8 && n->shape[0] * n->shape[1] * n->in[0].shape[1] < 2048; }
+
+    // Lanes that share a result of a small product: k / 4 of them, so that one round of four loads each covers k; one (and
+    // the lanes of a wavefront on neighbouring columns) where there are results enough to fill the chip.
+    static int small_dot_lanes(int64_t M, int64_t N, int64_t K) {
+        int lanes = 1;
+        while (lanes < 64 && 4 * lanes < K && M * N < 65536) lanes *= 2;
+        return lanes;
     }
 
     // whether a product goes to the matrix-core kernel (else the one-thread-per-output kernel)
@@ -3424,7 +3448,6 @@ struct Lowerer {
         auto B = [&](Node* x) { Arg q; q.kind = Arg::BUF; ADHIP_CHECK(x->buffer >= 0, "internal: matmul operand without buffer"); q.buf = x->buffer; return q; };
         auto I = [&](int64_t v) { Arg q; q.kind = Arg::I64; q.iv = v; return q; };
         const bool a_unit = a.s1 == 1 || a.s0 == 1, b_unit = b.s0 == 1 || b.s1 == 1;
-        ADHIP_CHECK(!epi || dot_uses_mfma(n), "internal: product epilogue on the small-product kernel");
         if (M * N * K >= 64 * 64 * 64 && a_unit && b_unit) {
             // matrix-core kernel; operands keep their strides (x^T, W^T are never copied)
             DotLaunchPlan pl = plan_dot(n);
@@ -3481,15 +3504,45 @@ struct Lowerer {
             }
             return;
         }
-        if (fixed_dot < 0) fixed_dot = add_kernel("adhip_dot_naive", fixed_kernels_source(), "dot_naive");
+        // (a product of up to 64 multiplications per thread of one block stays in one, which can share a launch with its
+        // neighbours)
+        const bool tiny = dot_is_tiny(n);
+        const int lanes = small_dot_lanes(M, N, K);
+        const int64_t blocks = tiny ? (M * N + 255) / 256 : M * N * K <= 16384 ? 1 : (M * N * lanes + 255) / 256;
         Launch l;
-        l.kernel = fixed_dot;
+        if (epi) {
+            const std::string entry = strf("adhip_dot_small_e%d", dot_epilogue_counter++);
+            GemmEpilogue ge;
+            ge.prelude = kernel_prelude();
+            ge.params = epi->params;
+            ge.code = epi->code;
+            ge.store_c = store_c;
+            l.kernel = add_kernel(entry, dot_small_source(entry, &ge), "dot_naive");
+        } else if (tiny) {
+            if (fixed_dot_tiny < 0) fixed_dot_tiny = add_kernel("adhip_dot_naive", fixed_kernels_source(), "dot_naive");
+            l.kernel = fixed_dot_tiny;
+        } else {
+            if (fixed_dot < 0) fixed_dot = add_kernel("adhip_dot_small", dot_small_source("adhip_dot_small"), "dot_naive");
+            l.kernel = fixed_dot;
+        }
         l.block[0] = 256;
-        l.grid[0] = (unsigned)((M * N + 255) / 256);
-        l.args = {B(n), B(a.base), B(b.base), I(M), I(N), I(K), I(a.offset), I(a.s0), I(a.s1), I(b.offset), I(b.s0), I(b.s1)};
+        ADHIP_CHECK(blocks <= 0x7fffffff, "internal: small product grid too large");
+        l.grid[0] = (unsigned)blocks;
+        l.args = {B(store_c ? n : epi->buffer_args[0]), B(a.base), B(b.base), I(M), I(N), I(K), I(a.offset), I(a.s0), I(a.s1), I(b.offset), I(b.s0), I(b.s1)};
+        Arg la;
+        la.kind = Arg::I32;
+        la.iv = lanes;
+        if (!tiny) l.args.push_back(la);
         l.label = strf("dot_%s_%lldx%lldx%lld", n->name.c_str(), (long long)M, (long long)N, (long long)K);
-        l.bytes = 4.0 * ((double)M * K + (double)K * N + (double)M * N);
+        l.bytes = 4.0 * ((double)M * K + (double)K * N + (store_c ? (double)M * N : 0.0));
         l.flops = 2.0 * (double)M * (double)N * (double)K;
+        if (epi) {
+            for (Node* x : epi->buffer_args) {
+                l.args.push_back(B(x));
+                l.bytes += 4.0 * (double)std::min<int64_t>(numel(x->shape), M * N);
+            }
+            l.flops += epi->flops * (double)M * (double)N;
+        }
         push_launch(out, l, "dot_naive");
     }
 
