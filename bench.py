@@ -22,6 +22,8 @@ for p in (ROOT, os.path.join(ROOT, "autodiff-ir-rust_amd")):
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, published
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix, published
+# FP32 products on the bf16 matrix cores: six products of bf16 parts each (dense bf16, published, over six)
+BF16_PARTS_PEAK_TFLOPS = 2500.0 / 6
 # Bytes per launch between the L2 caches and the memory fabric, from rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by a plain
 # copy kernel of known size (the summaries under profiles/ give the runs).  These counters sit in front of the 256 MiB
 # last-level cache, so they bound HBM traffic from above.  Valid for the full-size workloads only.
@@ -154,8 +156,8 @@ def measure_mlp(dev, iters):
            "flops_per_train_step": wl4.flops / iters}
     if tf:
         # all matrix-product launches of the run together: flops over the sum of their durations
-        out["roofline"] = {"bound": "mfma", "achieved": tf, "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                           "frac": tf / FP32_MFMA_PEAK_TFLOPS, "traffic": None, "kernel": "dot_mfma (all launches)",
+        out["roofline"] = {"bound": "mfma", "achieved": tf, "peak": BF16_PARTS_PEAK_TFLOPS, "unit": "TFLOP/s",
+                           "frac": tf / BF16_PARTS_PEAK_TFLOPS, "traffic": None, "kernel": "dot_mfma (all launches)",
                            "avg_ms": dot_ms / sum(k["launches_per_run"] for k in k4 if k["kernel"].startswith("dot"))}
     return out
 
