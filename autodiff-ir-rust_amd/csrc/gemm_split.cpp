@@ -1,8 +1,10 @@
 // FP32 matrix product for gfx950 on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16), LDS-tiled.
 //
-// An FP32 number is exactly the sum of three bf16 ones (8 + 8 + 8 bits, each rounded to nearest, of the same exponent
-// range), so a product of two is nine products of parts, each exact in FP32.  The six with a weight of 2^-16 and more
-// are summed, smallest first; the three left out come to some 2^-27 of the product, a fraction of the rounding of one
+// An FP32 number times 2^16 is exactly the sum of three bf16 ones (8 + 8 + 8 bits, each rounded to nearest; without the
+// factor the last of them would fall below bf16's range where the number is below 2^-110), so a product of two is nine
+// products of parts, each exact in FP32 (the method: Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", ARITH 2019).  The six with a weight of 2^-16 and more are
+// summed, smallest first, and the sum is taken back by 2^-32; the three left out come to some 2^-27 of the product, a fraction of the rounding of one
 // FP32 addition.  A step of 16 k costs 6 x 32 matrix cycles per 32 x 32 block where the FP32 matrix cores take 512, and,
 // other than theirs, vector instructions of one wavefront run under the matrix instructions of another: the bound is the
 // bf16 matrix rate over six (2.0 PFLOP/s sustained: 330 TFLOP/s), shared with the LDS (a k-tile of parts is one and a
@@ -38,6 +40,7 @@ std::string gemm_split_kernel_source(const GemmConfig& cfg, const std::string& e
 #define LDA (BM + 4)                    /* rows of a k group in LDS: the next group starts a quarter of the banks on */
 #define LDB (BN + 4)
 #define WGN (BN / (32 * TN))            /* waves along n */
+#define SCALE 65536.0f                  /* what the parts of an operand are larger by: its third part is then above bf16's smallest number */
 #define SETS (KW == 1 && BK == 32 ? 2 : 1)   /* of accumulators: for the first and second half of a tile's k */
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
@@ -53,14 +56,15 @@ typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
 typedef float4_t float4_g UNALIGNED;
 
 
-// Two neighbours of an operand, times sign (1 or -1), as three pairs of bf16 whose sums are exactly the two.
+// Two neighbours of an operand, times scale (2^16 or -2^16), as three pairs of bf16 whose sums are exactly the two: the
+// last bit of the smallest FP32 number, 2^-149, becomes the last bit of the smallest bf16 one.
 static __device__ __forceinline__ unsigned pack(float x, float y) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x, y}), bf16x2_t));
 }
-static __device__ __forceinline__ void split(float x, float y, float sign, unsigned& p0, unsigned& p1, unsigned& p2) {
-    p0 = pack(x, y) ^ (__builtin_bit_cast(unsigned, sign) & 0x80000000u) ^ ((__builtin_bit_cast(unsigned, sign) & 0x80000000u) >> 16);
-    x = __builtin_fmaf(x, sign, -__builtin_bit_cast(float, p0 << 16));
-    y = __builtin_fmaf(y, sign, -__builtin_bit_cast(float, p0 & 0xffff0000u));
+static __device__ __forceinline__ void split(float x, float y, float scale, unsigned& p0, unsigned& p1, unsigned& p2) {
+    p0 = pack(x * scale, y * scale);
+    x = __builtin_fmaf(x, scale, -__builtin_bit_cast(float, p0 << 16));
+    y = __builtin_fmaf(y, scale, -__builtin_bit_cast(float, p0 & 0xffff0000u));
     p1 = pack(x, y);
     x -= __builtin_bit_cast(float, p1 << 16);
     y -= __builtin_bit_cast(float, p1 & 0xffff0000u);
@@ -247,12 +251,12 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     // second half of each tile where it has accumulators of its own, else runs of tiles in the order + - - + - + + -
     // ..., which also cancels what grows with the sum; the accumulators change sign where a run ends.
 #if KW == 2 || BK == 32
-    const float a_sign = ga >= KG / 2 ? -1.0f : 1.0f;
-#define SIGN_OF(t) a_sign
+    const float a_scale = ga >= KG / 2 ? -SCALE : SCALE;
+#define SCALE_OF(t) a_scale
 #else
     const int run = 31 - __builtin_clz((unsigned)max(KT >> 3, 1));
     auto minus = [&](int t) { return (__builtin_popcount((unsigned)t >> run) & 1) != 0; };
-#define SIGN_OF(t) (minus(t) ? -1.0f : 1.0f)
+#define SCALE_OF(t) (minus(t) ? -SCALE : SCALE)
     auto negate = [&] {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -262,12 +266,12 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = -acc[i][j][r];
     };
 #endif
-    auto park_one = [&](uint4_t* to, int plane, const float* r, float sign) {
+    auto park_one = [&](uint4_t* to, int plane, const float* r, float scale) {
         uint4_t p0, p1, p2;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             unsigned u0, u1, u2;
-            split(r[2 * q], r[2 * q + 1], sign, u0, u1, u2);
+            split(r[2 * q], r[2 * q + 1], scale, u0, u1, u2);
             p0[q] = u0;
             p1[q] = u1;
             p2[q] = u2;
@@ -279,9 +283,9 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     // tile t, which has been loaded, goes to LDS in parts
     auto park = [&](int buf, int t, const float (*ra)[8], const float (*rb)[8]) {
 #pragma unroll
-        for (int i = 0; i < RA; ++i) park_one(&As[buf][0][ga][ROW_A(i)], KG * LDA, ra[i], SIGN_OF(t));
+        for (int i = 0; i < RA; ++i) park_one(&As[buf][0][ga][ROW_A(i)], KG * LDA, ra[i], SCALE_OF(t));
 #pragma unroll
-        for (int i = 0; i < RB; ++i) park_one(&Bs[buf][0][gb][ROW_B(i)], KG * LDB, rb[i], 1.0f);
+        for (int i = 0; i < RB; ++i) park_one(&Bs[buf][0][gb][ROW_B(i)], KG * LDB, rb[i], SCALE);
     };
     // ... and if it is the last and has k that the tile before had, A is parked once more with zeros there.  (B keeps
     // its values: zero times what is finite is zero, and a sum that is not finite is computed again anyway.)
@@ -293,7 +297,7 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
                 float r[8];
 #pragma unroll
                 for (int q = 0; q < 8; ++q) r[q] = (int)(8 * ga + q) < again ? 0.0f : ra[i][q];
-                park_one(&As[buf][0][ga][ROW_A(i)], KG * LDA, r, SIGN_OF(t));
+                park_one(&As[buf][0][ga][ROW_A(i)], KG * LDA, r, SCALE_OF(t));
             }
         }
 #endif
@@ -368,7 +372,7 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
 #define INTERLEAVE                                                                                          \
     _Pragma("unroll") for (int q = 0; q < MATRIX_OPS; ++q) {                                                \
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                  \
-        __builtin_amdgcn_sched_group_barrier(0x002, (48 * RA + 44 * RB + MATRIX_OPS - 1) / (MATRIX_OPS) + 1, 0); \
+        __builtin_amdgcn_sched_group_barrier(0x002, (48 * RA + 48 * RB + MATRIX_OPS - 1) / (MATRIX_OPS) + 1, 0); \
     }
 #else
 #define INTERLEAVE
@@ -447,10 +451,9 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     }
 #endif
 
-    // What the parts cannot represent -- infinities, values near the end of the range, NaN -- ends in a sum that is
-    // not finite, and what they represent with fewer bits (magnitudes of 2^-110 and less) in a sum that is tiny: such
-    // a wavefront's sub-tile is multiplied again on the FP32 matrix cores.
-    unsigned largest = 0u, smallest = 0x7f000000u;
+    // What the parts cannot represent -- infinities, NaN, operands from 2^111 and sums from 2^95 on -- ends in a sum that
+    // is not finite: such a wavefront's sub-tile is multiplied again on the FP32 matrix cores.
+    unsigned largest = 0u;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -458,11 +461,10 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float x = acc[i][j][r];   // (a bit cast of a vector's element itself reads the vector's first)
-                const unsigned u = __builtin_bit_cast(unsigned, x) & 0x7fffffffu;
-                largest = max(largest, u);
-                smallest = min(smallest, u - 1u);   // (zero wraps: it is as good as any)
+                largest = max(largest, __builtin_bit_cast(unsigned, x) & 0x7fffffffu);
             }
-    const bool again_f32 = __builtin_amdgcn_ballot_w64(largest >= 0x7f800000u || smallest < 0x17800000u) != 0ull;   // not finite, or below 2^-80
+    const bool again_f32 = __builtin_amdgcn_ballot_w64(largest >= 0x7f800000u) != 0ull;
+    const float unscale = again_f32 ? 1.0f : 1.0f / SCALE / SCALE;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         if (again_f32) {
@@ -499,7 +501,7 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
                     if (row < M && col < N)
 #endif
                     {
-                        const float sum_value = acc[i][j][4 * g + r];
+                        const float sum_value = acc[i][j][4 * g + r] * unscale;
 #if STORE_C
                         C[row * N + col] = sum_value;
 #endif

@@ -3,6 +3,7 @@ the smallest k, k beside a multiple of every tile depth, outputs beside the tile
 and operands the parts cannot represent, which are multiplied again on the FP32 matrix cores.  Tolerance: 1e-5 * sqrt(k)
 of the largest |a|.|b| dot product, as for every other product; the summation error of k FP32 terms stays below it."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -71,3 +72,52 @@ def test_operands_that_the_parts_cannot_represent(layout, shape, hip_device):
     assert_close(got[rows].reshape(-1), (a64[rows] @ b64).reshape(-1), RED_RTOL * math.sqrt(k), "c", scale=float((np.abs(a64[rows]) @ np.abs(b64)).max()))
     assert_close(got[11] * 2.0 ** 118, (a64[11] @ b64) * 2.0 ** 118, RED_RTOL * math.sqrt(k), "tiny row",
                  scale=float((np.abs(a64[11]) @ np.abs(b64)).max() * 2.0 ** 118))
+
+
+@pytest.mark.parametrize("shape,layout", [((130, 70, 77), "kn"), ((300, 200, 256), "mk"), ((300, 200, 1100), "kk"), ((2000, 1900, 1030), "mn")])
+@pytest.mark.parametrize("ea,eb", [(-118, 60), (-122, 90), (-126, 100), (-130, 110), (-140, 115), (-140, 90), (90, -122), (-62, -64)])
+def test_operands_at_the_bottom_of_the_range(shape, layout, ea, eb, hip_device):
+    """Operands down into FP32's subnormals beside large ones: the result is an ordinary number, and as precise as any
+    other.  Bound: an operand is held to the bit it has, so the error is that of the sum alone, for which 2^-24 sqrt(k)
+    of the root mean square is what k roundings of partial sums no larger than the result add up to; where the result
+    is itself subnormal, half of its last bit (one for each of the few ranges that k is cut into) comes on top."""
+    m, n, k = shape
+    print(f"[case] small operands {m}x{n}x{k} layout {layout} 2^{ea} x 2^{eb}", flush=True)
+    rng = np.random.default_rng(m + 1000 + ea)
+    a = rng.standard_normal((m, k), dtype=np.float32) * np.float32(2.0 ** ea)
+    b = rng.standard_normal((k, n), dtype=np.float32) * np.float32(2.0 ** eb)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = (a64 @ b64).reshape(-1)
+    got = _product(hip_device, layout, a, b).reshape(-1).astype(np.float64)
+    rms = math.sqrt(float(np.mean(want ** 2)))
+    err = math.sqrt(float(np.mean((got - want) ** 2)))
+    assert err <= 2.0 ** -24 * math.sqrt(k) * rms + 4 * 2.0 ** -149, (err / rms, rms)
+
+
+def _time(hip_device, a, b):
+    (m, k), n = a.shape, b.shape[1]
+    cmds = [IR.CreateMat(a.reshape(-1), [m, k], "a"), IR.CreateMat(b.reshape(-1), [k, n], "b"), IR.DotProduct(a="a", b="b", res="c"), IR.EX()]
+    prog = hip_device.compile(IR.IRProcedure("main", cmds), {"c"})
+    prog.upload()
+    best = math.inf
+    for _ in range(5):
+        t0 = time.perf_counter()
+        for _ in range(20):
+            prog.enqueue()
+        prog.sync()
+        best = min(best, time.perf_counter() - t0)
+    prog.close()
+    return best
+
+
+@pytest.mark.parametrize("shape", [(4096, 4096, 1024), (4096, 1024, 4096)])
+def test_tiny_results_cost_nothing(shape, hip_device):
+    """Rows of results around 2^-105 in every tile take the time of any others."""
+    m, n, k = shape
+    print(f"[case] time of tiny results {m}x{n}x{k}", flush=True)
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    plain = _time(hip_device, a, b)
+    tiny = a.copy()
+    tiny[5::32] *= np.float32(2.0 ** -110)
+    assert _time(hip_device, tiny, b) < 1.25 * plain
