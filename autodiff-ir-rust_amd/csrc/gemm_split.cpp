@@ -452,7 +452,10 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
 #endif
 
     // What the parts cannot represent -- infinities, NaN, operands from 2^111 and sums from 2^95 on -- ends in a sum that
-    // is not finite: such a wavefront's sub-tile is multiplied again on the FP32 matrix cores.
+    // is not finite: such a wavefront's sub-tile is multiplied again on the FP32 matrix cores, straight from memory.  A
+    // lane takes four consecutive k at a time, and two rows of blocks share what is loaded (all four at once spill):
+    // 4096^3 with an infinity in every wavefront's rows 1.8-2.2 ms in all, where one k and one row at a time took 3.8-5.9
+    // (FP32 matrix cores alone, staged through LDS: 1.1).
     unsigned largest = 0u;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -465,30 +468,83 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
             }
     const bool again_f32 = __builtin_amdgcn_ballot_w64(largest >= 0x7f800000u) != 0ull;
     const float unscale = again_f32 ? 1.0f : 1.0f / SCALE / SCALE;
+#define ROWS (TM < 2 ? TM : 2)
+#define KEEP(x) asm volatile("" : "+v"(x));   /* step by step: the addresses of all steps at once cost the 256x256 tile its last registers */
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i0 = 0; i0 < TM; i0 += ROWS) {
         if (again_f32) {
-            const float* qa = A + CLAMP_A(wm * (32 * TM) + 32 * i + li) * a_sm;
-            const float* qb[TN];
+            long long qa[ROWS], qb[TN];   // where its next four k begin
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                qb[j] = B + CLAMP_B(wn * (32 * TN) + 32 * j + li) * b_sn;
+            for (int i = 0; i < ROWS; ++i) {
+                qa[i] = CLAMP_A(wm * (32 * TM) + 32 * (i0 + i) + li) * a_sm + (k_lo + 4 * lh) * a_sk;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i0 + i][j][r] = 0.0f;
             }
-#pragma unroll 2
-            for (long long k0 = k_lo; k0 < k_hi; k0 += 2) {
-                const long long k = min(k0 + lh, k_hi - 1);
-                const bool in = k0 + lh < k_hi;
-                const float x = qa[k * a_sk], xa = in ? x : 0.0f;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) qb[j] = CLAMP_B(wn * (32 * TN) + 32 * j + li) * b_sn + (k_lo + 4 * lh) * b_sk;
+            auto multiply_f32 = [&](const float* x, const float* y, int stride) {   // one k of a lane
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i0 + i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i * stride], y[j * stride], acc[i0 + i][j], 0, 0, 0);
+            };
+            long long k0 = k_lo;
+#pragma unroll 1
+            for (; k0 + 8 <= k_hi; k0 += 8) {
+                float x[ROWS][4], y[TN][4];
+#if A_KCONTIG
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i) {
+                    *(float4_t*)x[i] = *(const float4_g*)(A + qa[i]);
+                    qa[i] += 8;
+                }
+#else
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < ROWS; ++i) {
+                        x[i][q] = A[qa[i]];
+                        qa[i] += (q < 3 ? 1 : 5) * a_sk;
+                        KEEP(qa[i])
+                    }
+#endif
+#if B_KCONTIG
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    const float y = qb[j][k * b_sk], xb = in ? y : 0.0f;
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, xb, acc[i][j], 0, 0, 0);
+                    *(float4_t*)y[j] = *(const float4_g*)(B + qb[j]);
+                    qb[j] += 8;
                 }
+#else
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        y[j][q] = B[qb[j]];
+                        qb[j] += (q < 3 ? 1 : 5) * b_sk;
+                        KEEP(qb[j])
+                    }
+#endif
+#pragma unroll
+                for (int q = 0; q < 4; ++q) multiply_f32(&x[0][q], &y[0][q], 4);
+            }
+#pragma unroll 1
+            for (int q = 0; q < 4 && k0 + q < k_hi; ++q) {
+                const bool in = k0 + 4 * lh + q < k_hi;   // (beyond: the last k again, as zero)
+                const long long at = in ? q : k_hi - 1 - (k0 + 4 * lh);
+                float x[ROWS], y[TN];
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i) x[i] = in ? A[qa[i] + at * a_sk] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) y[j] = in ? B[qb[j] + at * b_sk] : 0.0f;
+                multiply_f32(x, y, 1);
             }
         }
         // acc[i][j][4g + r] holds C[row = 32i + 8g + 4*lh + r][col = 32j + li] of the wave's sub-tile
+#pragma unroll
+        for (int i = i0; i < i0 + ROWS; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
