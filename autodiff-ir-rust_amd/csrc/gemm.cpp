@@ -419,8 +419,8 @@ std::string dot_small_source(const std::string& entry, const GemmEpilogue* epilo
     }
     s += R"(
     const unsigned share = threadIdx.x & (unsigned)(lanes - 1), per_block = 256u / (unsigned)lanes;
-    const long long total = M * N, stride = (long long)gridDim.x * per_block;
-    for (long long g = (long long)blockIdx.x * per_block + threadIdx.x / (unsigned)lanes; g < total; g += stride) {
+    const long long total = M * N, g = (long long)blockIdx.x * per_block + threadIdx.x / (unsigned)lanes;
+    if (g < total) {
         const long long row = total <= 0x7fffffff ? (long long)((unsigned)g / (unsigned)N) : g / N, col = g - row * N;
         const float* pa = A + a_off + row * a_sm;
         const float* pb = B + b_off + col * b_sn;

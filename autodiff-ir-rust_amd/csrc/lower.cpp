@@ -3352,9 +3352,15 @@ struct Lowerer {
     static bool dot_is_tiny(const Node* n) { return n->in[0].shape[1] <= 8 && n->shape[0] * n->shape[1] * n->in[0].shape[1] < 2048; }
 
     // Lanes that share a result of a small product: k / 4 of them, so that one round of four loads each covers k; one (and
-    // the lanes of a wavefront on neighbouring columns) where there are results enough to fill the chip.
+    // the lanes of a wavefront on neighbouring columns) where there are results enough to fill the chip.  Up to 256
+    // results take the lanes that one block has for them if these need no more than four rounds: a launch of one block can
+    // share it with its neighbours (a perceptron 16-16-16-4 at batch 16, a hundred steps: 2.71 ms; 3.50 with k / 4 lanes and
+    // so four blocks, 3.49 with these in one block, one after the other; eight rounds gain nothing, sixteen lose again).
     static int small_dot_lanes(int64_t M, int64_t N, int64_t K) {
         int lanes = 1;
+        while (lanes < 64 && 2 * lanes * M * N <= 256) lanes *= 2;
+        if (M * N <= 256 && K <= 4 * 4 * lanes) return lanes;
+        lanes = 1;
         while (lanes < 64 && 4 * lanes < K && M * N < 65536) lanes *= 2;
         return lanes;
     }
@@ -3530,11 +3536,11 @@ struct Lowerer {
             }
             return;
         }
-        // (a product of up to 64 multiplications per thread of one block stays in one, which can share a launch with its
-        // neighbours)
+        // (as many blocks as cover the results at once: one block that walks over them pays a trip to memory for every 256
+        // lanes, 0.4 us each -- 128 x 128 x 1 24.8 us against 3.1, 16 x 16 x 64 13.2 against 3.4 -- and saves 2 to 3 us at most)
         const bool tiny = dot_is_tiny(n);
         const int lanes = small_dot_lanes(M, N, K);
-        const int64_t blocks = tiny ? (M * N + 255) / 256 : M * N * K <= 16384 ? 1 : (M * N * lanes + 255) / 256;
+        const int64_t blocks = (M * N * (tiny ? 1 : lanes) + 255) / 256;
         Launch l;
         if (epi) {
             const std::string entry = strf("adhip_dot_small_e%d", dot_epilogue_counter++);
