@@ -3234,7 +3234,7 @@ struct Lowerer {
         ADHIP_CHECK(!partial || numel(partial->shape) == (int64_t)cnt * pl.splits * M * N, "internal: slice buffer of the wrong size");
         const bool small = key0[7] == kSmallDot;
         const std::string entry = small ? "adhip_dot_small_grouped" : dot_kernel_name(cfg) + "_grouped", kind = small ? "dot_naive" : "dot_mfma";
-        const int lanes = small_dot_lanes(M, N, K);
+        const int lanes = small_dot_lanes(M, N, K, key0[4] <= key0[3] && key0[5] <= key0[6]);
         Launch l;
         l.kernel = add_kernel(entry, small ? dot_small_source(entry, nullptr, true) : gemm_source(cfg, entry), kind);
         l.block[0] = small ? 256u : gemm_threads(cfg);
@@ -3351,17 +3351,22 @@ struct Lowerer {
 
     static bool dot_is_tiny(const Node* n) { return n->in[0].shape[1] <= 8 && n->shape[0] * n->shape[1] * n->in[0].shape[1] < 2048; }
 
-    // Lanes that share a result of a small product: k / 4 of them, so that one round of four loads each covers k; one (and
-    // the lanes of a wavefront on neighbouring columns) where there are results enough to fill the chip.  Up to 256
+    // Lanes that share a result of a small product: k / 4 of them, so that one round of four loads each covers k; fewer
+    // (and the lanes of a wavefront on neighbouring columns) where there are results enough to give every SIMD of the chip
+    // three wavefronts.  That line only concerns larger products of operands without a unit stride, where more lanes read
+    // more lines at once than the caches hold (255 x 255 x 1000: 38-137 us by layout with 2 lanes, 159-205 with 64, 107-188
+    // with one thread per result; 300 x 300 x 300 19 with 2, 24 with one) -- unless both operands lie along k, whose lines
+    // the lanes then share (the same: 58 us with 64, 117 with 2).  Up to 256
     // results take the lanes that one block has for them if these need no more than four rounds: a launch of one block can
     // share it with its neighbours (a perceptron 16-16-16-4 at batch 16, a hundred steps: 2.71 ms; 3.50 with k / 4 lanes and
     // so four blocks, 3.49 with these in one block, one after the other; eight rounds gain nothing, sixteen lose again).
-    static int small_dot_lanes(int64_t M, int64_t N, int64_t K) {
+    static int small_dot_lanes(int64_t M, int64_t N, int64_t K, bool along_k) {
         int lanes = 1;
         while (lanes < 64 && 2 * lanes * M * N <= 256) lanes *= 2;
         if (M * N <= 256 && K <= 4 * 4 * lanes) return lanes;
+        const int64_t most = along_k && M * N < 65536 ? 64 : 3 * 256 * 4 * 64 / std::max<int64_t>(M * N, 1);
         lanes = 1;
-        while (lanes < 64 && 4 * lanes < K && M * N < 65536) lanes *= 2;
+        while (lanes < 64 && 4 * lanes < K && 2 * lanes <= most) lanes *= 2;
         return lanes;
     }
 
@@ -3539,7 +3544,7 @@ struct Lowerer {
         // (as many blocks as cover the results at once: one block that walks over them pays a trip to memory for every 256
         // lanes, 0.4 us each -- 128 x 128 x 1 24.8 us against 3.1, 16 x 16 x 64 13.2 against 3.4 -- and saves 2 to 3 us at most)
         const bool tiny = dot_is_tiny(n);
-        const int lanes = small_dot_lanes(M, N, K);
+        const int lanes = small_dot_lanes(M, N, K, a.s1 <= a.s0 && b.s0 <= b.s1);
         const int64_t blocks = (M * N * (tiny ? 1 : lanes) + 255) / 256;
         Launch l;
         if (epi) {
