@@ -58,9 +58,10 @@ struct Module {
     }
 };
 
-// A kept tensor on the host.  Small ones live in a vector and arrive through the staging area; large ones live in
-// pinned memory of their own, which the copy engine writes directly (about five times the rate of a copy into
-// pageable memory) and which is kept for the next read-back of the same id.
+// A kept tensor on the host.  Those of up to kStageMaxItem live in a vector and arrive through the staging area; larger
+// ones live in pinned memory of their own, which the copy engine writes directly (about five times the rate of a copy into
+// pageable memory, which also holds the host up and behind it the next copy: 24 of 512 KB beside an encoder layer's larger
+// gradients cost 0.7 of 3.6 ms a pass) and which is kept for the next read-back of the same id.
 struct HostResult {
     std::vector<float> data;
     float* pinned = nullptr;
@@ -90,10 +91,52 @@ struct HostResult {
     }
     ~HostResult() { release(); }
 };
-// Results at least this large get pinned memory: all that are too large for the staging area (kStageMaxItem).  A copy into
-// pageable memory holds the host up, and behind it the next copy (24 of 512 KB beside an encoder layer's larger
-// gradients: 3.6 ms a pass, of which 0.7 ms was spent so).
-constexpr size_t kPinnedResultBytes = (size_t(64) << 10) + 1;
+constexpr size_t kStageBytes = 1 << 20;        // pinned staging area
+constexpr size_t kStageMaxItem = 64 << 10;     // larger transfers go directly
+
+// Pinned blocks of results whose ids did not come back, for the ids that come: two programs that take turns would
+// otherwise pin and unpin every result of theirs at every call, some 100 us each (24 of 512 KiB: 2.8 ms a call, of which the
+// same program again takes 0.5).  At most kParkedBytes in blocks of up to kParkedBlockBytes (larger ones are as quickly
+// allocated as found), the oldest given up first, all of them with the context.
+struct PinnedBlocks {
+    static constexpr size_t kParkedBytes = size_t(32) << 20, kParkedBlockBytes = size_t(1) << 20;
+    std::vector<std::pair<float*, size_t>> parked;   // memory, elements
+    size_t bytes = 0;
+    // takes over r's block
+    void park(HostResult& r) {
+        if (r.pinned && r.pinned_elems * sizeof(float) <= kParkedBlockBytes) {
+            parked.push_back({r.pinned, r.pinned_elems});
+            bytes += r.pinned_elems * sizeof(float);
+            r.pinned = nullptr;
+            r.pinned_elems = 0;
+            while (bytes > kParkedBytes) drop(0);
+        }
+        r.release();
+    }
+    // gives r, which has none, a block of at least `elems` elements: the smallest parked one, if at most twice as large
+    void provide(HostResult& r, size_t elems) {
+        size_t best = parked.size();
+        for (size_t i = 0; i < parked.size(); ++i)
+            if (parked[i].second >= elems && parked[i].second <= 2 * elems && (best == parked.size() || parked[i].second < parked[best].second)) best = i;
+        if (best < parked.size()) {
+            r.pinned = parked[best].first;
+            r.pinned_elems = parked[best].second;
+            bytes -= r.pinned_elems * sizeof(float);
+            parked.erase(parked.begin() + (std::ptrdiff_t)best);
+            return;
+        }
+        HIP_OK(hipHostMalloc((void**)&r.pinned, elems * sizeof(float), hipHostMallocDefault));
+        r.pinned_elems = elems;
+    }
+    void drop(size_t i) {
+        bytes -= parked[i].second * sizeof(float);
+        (void)hipHostFree(parked[i].first);
+        parked.erase(parked.begin() + (std::ptrdiff_t)i);
+    }
+    ~PinnedBlocks() {
+        while (!parked.empty()) drop(parked.size() - 1);
+    }
+};
 
 }  // namespace
 
@@ -104,6 +147,7 @@ struct adhip_ctx {
     std::string last_error;
     std::map<std::string, std::shared_ptr<Module>> modules;  // by source text
     std::map<std::string, HostResult> results;
+    PinnedBlocks blocks;
     float* pinned = nullptr;  // small pinned area for predicate read-back
     char* stage = nullptr;    // pinned staging area for small uploads and read-backs
     unsigned char* static_scratch = nullptr;  // this device's copy of adhip_static_scratch (device address)
@@ -114,8 +158,6 @@ struct adhip_ctx {
     struct CachedExec { std::string key; adhip_program* prog; size_t bytes; };
     std::vector<CachedExec> exec_cache;
 };
-constexpr size_t kStageBytes = 1 << 20;        // pinned staging area
-constexpr size_t kStageMaxItem = 64 << 10;     // larger transfers go directly
 constexpr size_t kExecCacheEntries = 4;        // programs kept per context
 constexpr size_t kExecCacheBytes = size_t(4) << 30;  // device memory the kept programs may hold together
 
@@ -847,6 +889,8 @@ void program_readback(adhip_program* p) {
     // result cost more than the copy itself
     std::map<std::string, HostResult> previous;
     previous.swap(ctx->results);
+    for (auto& kv : previous)
+        if (!p->plan->results.count(kv.first)) ctx->blocks.park(kv.second);
     struct Staged { HostResult* r; size_t off, nb; };
     std::vector<Staged> staged;
     size_t used = 0;
@@ -879,31 +923,26 @@ void program_readback(adhip_program* p) {
         for (auto d : kv.second.shape) r.dims.push_back((uint64_t)d);
         const int64_t ne = numel(kv.second.shape);
         const size_t nb = (size_t)std::max<int64_t>(ne, 0) * sizeof(float);
-        if (nb >= kPinnedResultBytes) {
+        if (nb > kStageMaxItem) {
             if (r.pinned_elems < (size_t)ne) {
-                r.release();
-                HIP_OK(hipHostMalloc((void**)&r.pinned, nb, hipHostMallocDefault));
-                r.pinned_elems = (size_t)ne;
+                ctx->blocks.park(r);
+                ctx->blocks.provide(r, (size_t)ne);
             }
             r.data.clear();
             HIP_OK(hipMemcpyAsync(r.pinned, p->buf_ptr[kv.second.buf], nb, hipMemcpyDeviceToHost, ctx->stream));
             continue;
         }
-        r.release();
+        ctx->blocks.park(r);
         r.data.resize((size_t)std::max<int64_t>(ne, 0));
         if (ne <= 0) continue;
         if (span && p->arena_off[(size_t)kv.second.buf] != SIZE_MAX) {
             staged.push_back({&r, p->arena_off[(size_t)kv.second.buf] - span_lo, nb});
             continue;
         }
-        if (nb <= kStageMaxItem) {
-            if (used + nb > kStageBytes) drain();
-            HIP_OK(hipMemcpyAsync(ctx->stage + used, p->buf_ptr[kv.second.buf], nb, hipMemcpyDeviceToHost, ctx->stream));
-            staged.push_back({&r, used, nb});
-            used += (nb + 255) & ~size_t(255);
-        } else {
-            HIP_OK(hipMemcpyAsync(r.data.data(), p->buf_ptr[kv.second.buf], nb, hipMemcpyDeviceToHost, ctx->stream));
-        }
+        if (used + nb > kStageBytes) drain();
+        HIP_OK(hipMemcpyAsync(ctx->stage + used, p->buf_ptr[kv.second.buf], nb, hipMemcpyDeviceToHost, ctx->stream));
+        staged.push_back({&r, used, nb});
+        used += (nb + 255) & ~size_t(255);
     }
     drain();
 }
