@@ -3191,10 +3191,7 @@ struct Lowerer {
         for (auto& kv : sets) {
             const std::vector<int>& set = kv.second;
             if (set.size() < 2) continue;
-            // (small products: eight; the plan's tests count on launches that grow with the number of heads, and twelve
-            // products in two launches instead of one are 2 of some 37 launches of a small encoder layer's step)
-            const size_t slots = kv.first.second[7] == kSmallDot ? kGemmGroupSlots / 2 : kGemmGroupSlots;
-            const size_t launches = (set.size() + slots - 1) / slots;
+            const size_t launches = (set.size() + kGemmGroupSlots - 1) / kGemmGroupSlots;
             const size_t per = (set.size() + launches - 1) / launches;
             for (size_t i0 = 0; i0 < set.size(); i0 += per) {
                 const size_t i1 = std::min(set.size(), i0 + per);

@@ -489,7 +489,8 @@ def test_kernels_differing_only_in_name_are_compiled_once():
         text = lower_describe(proc, deps)
         counts.append((int(re.search(r"kernels: (\d+)", text).group(1)), len(re.findall(r"^\s*launch", text, re.M))))
     assert counts[0][0] == counts[1][0] == counts[2][0], counts
-    assert counts[0][1] < counts[1][1] < counts[2][1], counts
+    # (products of one shape share launches of up to sixteen, so two heads more need not be a launch more)
+    assert counts[0][1] <= counts[1][1] <= counts[2][1] and counts[0][1] < counts[2][1], counts
 
 
 def test_training_loop_body_groups_per_head_products():
