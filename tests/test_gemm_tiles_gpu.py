@@ -1,6 +1,6 @@
-"""Every variant of the 256x128 block tile of the matrix-core kernel, value-checked.
+"""Every variant of the 256x256 block tile of the kernel on the bf16 matrix cores, value-checked.
 
-The lowering picks that tile only for outputs of at least 4096 x 4096 (512 tiles), so these cases use such an output
+The lowering picks that tile only for outputs of at least 200 such tiles, so these cases use 4096 x 4096 (256 tiles)
 with a short inner dimension (k = 256 keeps the float64 reference cheap): the four operand layouts (k- or m-contiguous
 A, k- or n-contiguous B: the forward product and the two backward products of reference
 src/graph/ops/dot_product.rs:34-42 read their operands that way), each plain and with an element-wise epilogue on the
@@ -50,7 +50,7 @@ def _kernels(proc, keep):
 @pytest.mark.parametrize("layout", ["kn", "kk", "mn", "mk"])
 @pytest.mark.parametrize("k", [256, 272])
 def test_256_tile_plain(layout, k, hip_device):
-    print(f"[case] 256x128 tile, layout {layout}, k {k}", flush=True)
+    print(f"[case] 256x256 tile, layout {layout}, k {k}", flush=True)
     rng = np.random.default_rng(100 + k + sum(map(ord, layout)))
     cmds, a64, b64 = _operands(layout, k, rng)
     cmds += [IR.DotProduct(a="a", b="b", res="c"), IR.EX()]
@@ -69,7 +69,7 @@ def test_256_tile_plain(layout, k, hip_device):
 def test_256_tile_epilogue(layout, kind, hip_device):
     """`update`: W += -0.01 * (A.B), the product itself never stored (the SGD step on a weight gradient);
     `activation`: y = sigmoid-like 1 / (1 + exp2(-(A.B + bias))) with the product also kept."""
-    print(f"[case] 256x128 tile epilogue, layout {layout}, {kind}", flush=True)
+    print(f"[case] 256x256 tile epilogue, layout {layout}, {kind}", flush=True)
     k = 256
     rng = np.random.default_rng(200 + sum(map(ord, layout + kind)))
     cmds, a64, b64 = _operands(layout, k, rng)

@@ -1,7 +1,8 @@
 """Products on the bf16 matrix cores (operands split into three bf16 parts), value-checked where the kernel can go wrong:
-the smallest k, k beside a multiple of every tile depth, outputs beside the tiles, every tile of the planner, ranges of k,
-and operands the parts cannot represent, which are multiplied again on the FP32 matrix cores.  Tolerance: 1e-5 * sqrt(k)
-of the largest |a|.|b| dot product, as for every other product; the summation error of k FP32 terms stays below it."""
+the smallest k, k beside a multiple of every tile depth, outputs beside the tiles, ranges of k, operands of every magnitude,
+and what does not come out finite, which is multiplied again on the FP32 matrix cores.  Tolerance: 1e-5 * sqrt(k) of the
+largest |a|.|b| dot product, as for every other product: it sees a wrong element, not a lost part of one, for which there
+is test_product_bits.py, on every tile of the planner."""
 import math
 import time
 
