@@ -64,6 +64,7 @@ std::string gemm_tile_head(const GemmConfig& cfg, const std::string& entry) {
 }
 
 std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue) {
+    ADHIP_CHECK(!cfg.bf16_parts && !cfg.split_k && cfg.bk == 16 && cfg.k_waves == 1, "internal: configuration of the kernel on the bf16 matrix cores");
     std::string s = gemm_kernel_head(cfg, epilogue);
     // tile geometry: BM x BN block tile, TM x TN MFMA blocks per wave, WGN waves along n
     s += gemm_tile_head(cfg, entry);
@@ -296,9 +297,9 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     // of tile kt + 2 are issued into the set that held tile kt (parked in LDS during tile kt - 1), and the set that
     // holds tile kt + 1, issued a whole tile earlier, is parked.  A load then has a k-tile and a half of MFMAs to
     // arrive instead of half a tile (which is some 500 cycles where a wavefront owns 64x32, less than a trip to
-    // memory): 4096 x 1024 x 4096 in 276 / 268 / 251 us instead of 289 / 274 / 257, the MLP workload's step 1.2 % and
-    // the encoder layer's 1.3 % shorter.  The loop is unrolled by two so that the sets and the LDS buffers are named,
-    // not indexed.
+    // memory).  Measured when products of any k ran here, of which there are one or two tiles left: 4096 x 1024 x 4096 in
+    // 276 / 268 / 251 us instead of 289 / 274 / 257.  The loop is unrolled by two so that the sets and the LDS buffers are
+    // named, not indexed.
     // Loads and parkings stand under no condition: beyond the last tile the loads fetch the last tile again and the
     // parking writes a tile nobody reads.  (Under a condition, the wait in front of a parking also waits for the
     // newest loads, or the compiler moves the loads down to the parking that consumes them.)

@@ -1,4 +1,5 @@
-// Source generator for the FP32 MFMA matrix-product kernel (see gemm.cpp).
+// Source generators for the matrix-product kernels: on the bf16 matrix cores (gemm_split.cpp), on the FP32 ones and for small
+// products (gemm.cpp).
 #pragma once
 #include <string>
 
@@ -9,11 +10,12 @@ struct GemmConfig {
     bool b_kcontig = false; // B[k,n]: k has unit stride (else n has)
     bool edge = false;      // bounds-checked accesses (odd sizes or unaligned operands)
     bool edge_vec = false;  // with edge: both operands' contiguous extents are at least 4, so threads load 128 bits where all four exist
-    int bm = 128;           // block tile: 256 (256x128, 8 waves), 128 (128x128, 4 waves) or 64 (64x64, 4 waves); k depth 16
-    int bn = 0;             // block tile columns; 0 = the default for bm (128, or 64 for bm 64).  128x64 is the only other shape
-    bool split_k = false;   // blockIdx.y picks a range of k (extra argument k_chunk); slice y of the product goes to C + y*M*N
+    // block tile: on the bf16 matrix cores 256x256, 128x128, 128x64 or 64x64; on the FP32 ones 256x128, 128x128, 128x64 or 64x64
+    int bm = 128;
+    int bn = 0;             // its columns; 0 = the FP32 kernel's for bm (128, or 64 for bm 64)
     bool bf16_parts = false;  // the kernel on the bf16 matrix cores (gemm_split.cpp); needs K >= bk
-    int bk = 16;            // k depth of its tiles (16, 32 or 64)
+    bool split_k = false;   // of that kernel: blockIdx.y picks a range of k (extra argument k_chunk); slice y of the product goes to C + y*M*N
+    int bk = 16;            // k depth of a tile: 16, 32 or 64, on the FP32 matrix cores 16
     int k_waves = 1;        // of that kernel: 2 = a tile's k is shared between two sets of wavefronts, whose sums are added at the end
     bool grouped = false;   // blockIdx.y picks one of kGemmGroupSlots products of the same shape (parameters c<i>, a<i>, b<i>)
 };

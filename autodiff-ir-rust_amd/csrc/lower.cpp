@@ -3367,7 +3367,8 @@ struct Lowerer {
         return lanes;
     }
 
-    // whether a product goes to the matrix-core kernel (else the one-thread-per-output kernel)
+    // whether a product goes to a matrix-core kernel (else the one whose lanes share a result, or the very smallest to the
+    // one-thread-per-output kernel)
     static bool dot_uses_mfma(const Node* n) {
         Affine2D a, b;
         if (!tref_affine2d(n->in[0], a) || !tref_affine2d(n->in[1], b)) return false;
