@@ -152,3 +152,22 @@ def test_error_of_sums(tile, layout, hip_device):
     exact = a.astype(np.float64) @ b.astype(np.float64)
     err = math.sqrt(float(np.mean((_run(hip_device, layout, a, b, kernel) - exact) ** 2) / np.mean(exact ** 2)))
     assert err <= _bound(k), (err, _bound(k))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,m,n,k,kernel", [(16, 2048, 512, 16, "kn_256_f32"), (5, 500, 500, 64, "kn_64_rim"), (5, 500, 64, 500, "kn_64_rim_pair"),
+                                                (8, 2048, 128, 1024, "kn_64"), (8, 2048, 128, 2048, "kn_128_splitk"), (4, 1000, 132, 2050, "kn_128_rim_splitk"), (8, 2000, 132, 2050, "kn_128_rim_pair"), (6, 1536, 1536, 96, "kn_256"),
+                                                (7, 1500, 1500, 50, "kn_256_rim"), (16, 100, 100, 31, "kn_64_rim_f32")])
+def test_exact_products_grouped(count, m, n, k, kernel, hip_device):
+    print(f"[case] {count} exact products {m}x{n}x{k}", flush=True)
+    rng = np.random.default_rng(count + m + n + k)
+    cmds, wants = [], []
+    for i in range(count):
+        a, b, want = list(_exact_programs(m, n, k, rng))[i % 3]
+        cmds += [IR.CreateMat(a.reshape(-1), [m, k], f"a{i}"), IR.CreateMat(b.reshape(-1), [k, n], f"b{i}"), IR.DotProduct(a=f"a{i}", b=f"b{i}", res=f"c{i}")]
+        wants.append(want)
+    proc, keep = IR.IRProcedure("main", cmds + [IR.EX()]), {f"c{i}" for i in range(count)}
+    assert re.findall(r"launch dots_\w+ \[dot_mfma\] kernel=(\w+)", lower_describe(proc, keep)) == [f"adhip_gemm_{kernel}_grouped"]
+    hip_device.execute(proc, keep)
+    for i, want in enumerate(wants):
+        assert np.array_equal(np.asarray(hip_device.get_tensor(f"c{i}").data).reshape(m, n), want), i
