@@ -4,12 +4,14 @@
 // factor the last of them would fall below bf16's range where the number is below 2^-110), so a product of two is nine
 // products of parts, each exact in FP32 (the method: Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial
 // Intelligence Datatype For Higher-Precision Computations", ARITH 2019).  The six with a weight of 2^-16 and more are
-// summed, smallest first, and the sum is taken back by 2^-32; the three left out come to some 2^-27 of the product, a fraction of the rounding of one
-// FP32 addition.  A step of 16 k costs 6 x 32 matrix cycles per 32 x 32 block where the FP32 matrix cores take 512, and,
-// other than theirs, vector instructions of one wavefront run under the matrix instructions of another: the bound is the
-// bf16 matrix rate over six (2.0 PFLOP/s sustained: 330 TFLOP/s), shared with the LDS (a k-tile of parts is one and a
-// half times its FP32 bytes) and the splitting.  The sums are rounded twice per 8 k and product instead of once per k:
-// errors against 64 bits are no larger (normal operands, k = 4096: 1.0e-6 against 1.1e-6 of the root mean square; k = 1024:
+// summed, smallest first, and the sum is taken back by 2^-32; the three left out come to some 2^-27 of the product, a
+// fraction of the rounding of one FP32 addition.  A step of 16 k costs 6 x 32 matrix cycles per 32 x 32 block where the
+// FP32 matrix cores take 512, and, other than theirs, vector instructions of one wavefront run under the matrix
+// instructions of another: the bound is the bf16 matrix rate over six (2.0 PFLOP/s sustained: 330 TFLOP/s).  The matrix
+// cores are busy 62-78 % of the time at 4096^3; the splitting takes a quarter of the vector pipes' and the parts a fifth
+// of the LDS's, and the rest is time in which no wavefront of a SIMD multiplies.  The sums are rounded twice per 8 k and
+// product instead of once per k: errors against 64 bits are no larger (normal operands, k = 4096: 1.0e-6 against 1.1e-6 of
+// the root mean square; k = 1024:
 // 3.4-4.8e-7 against 5.8e-7; k = 64: 0.7e-7 against 1.4e-7).
 //
 // The operands are described by strides and split on their way from registers to LDS, where a part's eight consecutive
@@ -18,10 +20,10 @@
 //   256x256x16  8 wavefronts of 128x64 in two sets that take turns between multiplying and everything else: 600-650 us
 //   128x128x16  4 wavefronts of 64x64, two blocks per CU: 710-770 us
 //   128x128x32  8 wavefronts, two per 64x64 sub-tile with half of the k-tile each: one block per CU does what two of
-//               the former do (4096 x 1024 x 4096: 177 us against 326 on 128x64 FP32 tiles)
+//               the former do (4096 x 1024 x 4096: 181-188 us against 326 on 128x64 FP32 tiles)
 //   128x64x32, 64x64x32, 64x64x64 (two sets): small outputs
 // Ragged sizes cost little: rows beyond the product repeat its last row, and the last k-tile starts inside the one
-// before it, with zeros for the k it shares (4000 x 4011 x 4001: 613 us against 1567).
+// before it, with zeros for the k it shares (4000 x 4011 x 4001: 615-665 us against 1567).
 #include "gemm.hpp"
 
 #include "common.hpp"
@@ -57,7 +59,8 @@ typedef float4_t float4_g UNALIGNED;
 
 
 // Two neighbours of an operand, times scale (2^16 or -2^16), as three pairs of bf16 whose sums are exactly the two: the
-// last bit of the smallest FP32 number, 2^-149, becomes the last bit of the smallest bf16 one.
+// last bit of the smallest FP32 number, 2^-149, becomes the last bit of the smallest bf16 one.  (Without the factor the
+// products take 0-4 % less, 4096 x 1024 x 4096 180.6 us for 184.5, and are wrong for operands below 2^-110.)
 static __device__ __forceinline__ unsigned pack(float x, float y) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x, y}), bf16x2_t));
 }
