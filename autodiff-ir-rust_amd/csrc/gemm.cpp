@@ -23,14 +23,14 @@ int gemm_tile_columns(const GemmConfig& cfg) { return cfg.bn ? cfg.bn : (cfg.bm 
 static int wave_rows(const GemmConfig& cfg) { return cfg.bm == 256 && cfg.bf16_parts ? 4 : cfg.bm == 64 ? 1 : 2; }
 static int wave_columns(const GemmConfig& cfg) { return gemm_tile_columns(cfg) == 64 ? 1 : 2; }
 unsigned gemm_threads(const GemmConfig& cfg) {
+    if (cfg.k_waves == kDirectWaves) return 64u * (unsigned)cfg.k_waves;
     return 64u * (unsigned)((cfg.bm / (32 * wave_rows(cfg))) * (gemm_tile_columns(cfg) / (32 * wave_columns(cfg))) * cfg.k_waves);
 }
 
 std::string gemm_kernel_head(const GemmConfig& cfg, const GemmEpilogue* epilogue) {
     std::string s;
     if (epilogue) s += epilogue->prelude;
-    s += strf("#define STORE_C %d\n#define EPI_PARAMS %s\n", (!epilogue || epilogue->store_c) ? 1 : 0,
-              epilogue ? epilogue->params.c_str() : "");
+    s += strf("#define STORE_C %d\n", (!epilogue || epilogue->store_c) ? 1 : 0);
     {
         // the epilogue statements become one macro (line continuations), expanded where an element is finished
         std::string body = epilogue ? epilogue->code : std::string();
@@ -46,28 +46,42 @@ std::string gemm_kernel_head(const GemmConfig& cfg, const GemmEpilogue* epilogue
     }
     s += strf("#define A_KCONTIG %d\n#define B_KCONTIG %d\n#define EDGE %d\n#define EDGE_VEC %d\n#define SPLITK %d\n#define GROUPED %d\n", cfg.a_kcontig ? 1 : 0,
               cfg.b_kcontig ? 1 : 0, cfg.edge ? 1 : 0, cfg.edge && cfg.edge_vec ? 1 : 0, cfg.split_k ? 1 : 0, cfg.grouped ? 1 : 0);
-    if (cfg.grouped) {
-        // one parameter triple per problem slot, and the (wave-uniform) choice among them by blockIdx.y
-        std::string params, pick = "switch (blockIdx.y) {";
-        for (int i = 0; i < kGemmGroupSlots; ++i) {
-            params += strf("float* c%d, const float* a%d, const float* b%d, ", i, i, i);
-            pick += strf(" case %d: C = c%d; A = a%d; B = b%d; break;", i, i, i, i);
-        }
-        s += "#define GROUP_PARAMS " + params + "\n#define GROUP_PICK " + pick + " default: return; }\n";
-    }
     return s;
 }
 
-std::string gemm_tile_head(const GemmConfig& cfg, const std::string& entry) {
-    return strf("#define KERNEL_NAME %s\n#define BM %d\n#define BN %d\n#define TM %d\n#define TN %d\n#define NT %u\n", entry.c_str(), cfg.bm,
-                gemm_tile_columns(cfg), wave_rows(cfg), wave_columns(cfg), gemm_threads(cfg));
+std::string gemm_tile_head(const GemmConfig& cfg) {
+    return strf("#define BM %d\n#define BN %d\n#define TM %d\n#define TN %d\n#define NT %u\n", cfg.bm, gemm_tile_columns(cfg), wave_rows(cfg),
+                wave_columns(cfg), gemm_threads(cfg));
+}
+
+std::string gemm_entry(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue, unsigned threads, const char* more) {
+    std::string s = strf("extern \"C\" __global__ __launch_bounds__(%u) void %s(const int* __restrict__ guard, ", threads, entry.c_str());
+    const char* sizes = "long long M, long long N, long long K, ";
+    if (cfg.grouped) {
+        // one parameter triple per problem slot, and the (wave-uniform) choice among them by blockIdx.y
+        std::string pick;
+        for (int i = 0; i < kGemmGroupSlots; ++i) {
+            s += strf("float* c%d, const float* a%d, const float* b%d, ", i, i, i);
+            pick += strf("    case %d: C = c%d; A = a%d; B = b%d; break;\n", i, i, i, i);
+        }
+        return s + sizes + "long long a_sm, long long a_sk, long long b_sk, long long b_sn" + (cfg.split_k ? ", long long k_chunk" : "") + more + R"() {
+    if (guard && *guard == 0) return;
+    float* __restrict__ C;
+    const float* __restrict__ A;
+    const float* __restrict__ B;
+    switch (blockIdx.y) {
+)" + pick + "    default: return;\n    }\n    const long long a_off = 0, b_off = 0;\n";
+    }
+    return s + "float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ B, " + sizes +
+           "long long a_off, long long a_sm, long long a_sk, long long b_off, long long b_sk, long long b_sn" + (cfg.split_k ? ", long long k_chunk" : "") + more +
+           (epilogue ? epilogue->params : std::string()) + ") {\n    if (guard && *guard == 0) return;\n";
 }
 
 std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue) {
     ADHIP_CHECK(!cfg.bf16_parts && !cfg.split_k && cfg.bk == 16 && cfg.k_waves == 1, "internal: configuration of the kernel on the bf16 matrix cores");
     std::string s = gemm_kernel_head(cfg, epilogue);
     // tile geometry: BM x BN block tile, TM x TN MFMA blocks per wave, WGN waves along n
-    s += gemm_tile_head(cfg, entry);
+    s += gemm_tile_head(cfg);
     {
         // diagnostic: ADHIP_GEMM_AHEAD=1 keeps the global loads one k-tile ahead of the MFMAs instead of two
         int ahead = 2;
@@ -131,25 +145,7 @@ static __device__ __forceinline__ float4_t edge_load4(const float* p, long long 
 // blockIdx.y works on problem y, whose three base pointers (operand offsets already applied) are parameters
 // c<y>, a<y>, b<y>.  For the same kind of product when there are many of them (the per-head projections of
 // multi-head attention).
-extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
-#if GROUPED
-    const int* __restrict__ guard, GROUP_PARAMS long long M, long long N, long long K, long long a_sm, long long a_sk,
-    long long b_sk, long long b_sn
-    ) {
-    if (guard && *guard == 0) return;
-    float* __restrict__ C;
-    const float* __restrict__ A;
-    const float* __restrict__ B;
-    GROUP_PICK
-    const long long a_off = 0, b_off = 0;
-#else
-    const int* __restrict__ guard, float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ B,
-    long long M, long long N, long long K, long long a_off, long long a_sm, long long a_sk, long long b_off,
-    long long b_sk, long long b_sn
-    EPI_PARAMS) {
-    if (guard && *guard == 0) return;
-#endif
-    const long long k_lo = 0, k_hi = K;
+)" + gemm_entry(cfg, entry, epilogue, gemm_threads(cfg)) + R"(    const long long k_lo = 0, k_hi = K;
     __shared__ __attribute__((aligned(16))) float As[2][BK][LDA];
     __shared__ __attribute__((aligned(16))) float Bs[2][BK][LDB];
 
@@ -400,24 +396,7 @@ std::string dot_small_source(const std::string& entry, const GemmEpilogue* epilo
     GemmConfig cfg;
     cfg.grouped = grouped;
     std::string s = gemm_kernel_head(cfg, epilogue);
-    // (name and parameters stand as text: a launch that runs several kernels in turn reads them from the source)
-    s += "extern \"C\" __global__ __launch_bounds__(256) void " + entry + "(const int* __restrict__ guard, ";
-    if (grouped) {
-        s += R"(GROUP_PARAMS long long M, long long N, long long K, long long a_sm, long long a_sk, long long b_sk, long long b_sn, int lanes) {
-    if (guard && *guard == 0) return;
-    float* __restrict__ C;
-    const float* __restrict__ A;
-    const float* __restrict__ B;
-    GROUP_PICK
-    const long long a_off = 0, b_off = 0;
-)";
-    } else {
-        s += R"(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ B, long long M, long long N, long long K,
-    long long a_off, long long a_sm, long long a_sk, long long b_off, long long b_sk, long long b_sn, int lanes)" +
-             (epilogue ? epilogue->params : std::string()) + R"() {
-    if (guard && *guard == 0) return;
-)";
-    }
+    s += gemm_entry(cfg, entry, epilogue, 256, ", int lanes");
     s += R"(
     const unsigned share = threadIdx.x & (unsigned)(lanes - 1), per_block = 256u / (unsigned)lanes;
     const long long total = M * N, g = (long long)blockIdx.x * per_block + threadIdx.x / (unsigned)lanes;
@@ -452,7 +431,6 @@ std::string dot_small_source(const std::string& entry, const GemmEpilogue* epilo
     }
 }
 #undef EPILOGUE
-#undef EPI_PARAMS
 #undef STORE_C
 #undef A_KCONTIG
 #undef B_KCONTIG

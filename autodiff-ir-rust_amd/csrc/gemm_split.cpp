@@ -21,7 +21,7 @@
 //   128x128x16  4 wavefronts of 64x64, two blocks per CU: 710-770 us
 //   128x128x32  8 wavefronts, two per 64x64 sub-tile with half of the k-tile each: one block per CU does what two of
 //               the former do (4096 x 1024 x 4096: 181-188 us against 326 on 128x64 FP32 tiles)
-//   128x64x32, 64x64x32, 64x64x64 (two sets): small outputs
+//   128x64x32, 64x64x32: outputs of a few hundred blocks with a short k (smaller ones: gemm_direct.cpp)
 // Ragged sizes cost little: rows beyond the product repeat its last row, and the last k-tile starts inside the one
 // before it, with zeros for the k it shares (4000 x 4011 x 4001: 615-665 us against 1567).
 #include "gemm.hpp"
@@ -30,21 +30,8 @@
 
 namespace adhip {
 
-std::string gemm_split_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue) {
-    std::string s = gemm_kernel_head(cfg, epilogue) + gemm_tile_head(cfg, entry);
-    const int per_thread = 8 * (int)gemm_threads(cfg);   // elements of an operand's tile that a thread's unit of eight k covers
-    s += strf("#define BK %d\n#define KW %d\n#define PINGPONG %d\n#define KS %d\n#define RA_VALUE %d\n#define RB_VALUE %d\n", cfg.bk, cfg.k_waves,
-              cfg.bm == 256 ? 1 : 0, cfg.bm == 256 ? cfg.bk / 16 : 1, cfg.bm * cfg.bk / per_thread, gemm_tile_columns(cfg) * cfg.bk / per_thread);
-    s += R"(
-#define KG (BK / 8)                     /* groups of eight k of a tile */
-#define RA RA_VALUE                     /* rows of A (with their eight k) that a thread carries from memory to LDS */
-#define RB RB_VALUE
-#define LDA (BM + 4)                    /* rows of a k group in LDS: the next group starts a quarter of the banks on */
-#define LDB (BN + 4)
-#define WGN (BN / (32 * TN))            /* waves along n */
-#define SCALE 65536.0f                  /* what the parts of an operand are larger by: its third part is then above bf16's smallest number */
-#define SETS (KW == 1 && BK == 32 ? 2 : 1)   /* of accumulators: for the first and second half of a tile's k */
-typedef float float4_t __attribute__((ext_vector_type(4)));
+std::string split_types() {
+    return R"(typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -64,41 +51,155 @@ typedef float4_t float4_g UNALIGNED;
 static __device__ __forceinline__ unsigned pack(float x, float y) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x, y}), bf16x2_t));
 }
+// part p (0, 1, 2 in turn) of two neighbours, which become what is left of them
+static __device__ __forceinline__ unsigned split_part(int p, float& x, float& y, float scale) {
+    const unsigned u = p == 0 ? pack(x * scale, y * scale) : pack(x, y);
+    if (p == 2) return u;
+    x = __builtin_fmaf(x, p == 0 ? scale : 1.0f, -__builtin_bit_cast(float, u << 16));
+    y = __builtin_fmaf(y, p == 0 ? scale : 1.0f, -__builtin_bit_cast(float, u & 0xffff0000u));
+    return u;
+}
 static __device__ __forceinline__ void split(float x, float y, float scale, unsigned& p0, unsigned& p1, unsigned& p2) {
-    p0 = pack(x * scale, y * scale);
-    x = __builtin_fmaf(x, scale, -__builtin_bit_cast(float, p0 << 16));
-    y = __builtin_fmaf(y, scale, -__builtin_bit_cast(float, p0 & 0xffff0000u));
-    p1 = pack(x, y);
-    x -= __builtin_bit_cast(float, p1 << 16);
-    y -= __builtin_bit_cast(float, p1 & 0xffff0000u);
-    p2 = pack(x, y);
+    p0 = split_part(0, x, y, scale);
+    p1 = split_part(1, x, y, scale);
+    p2 = split_part(2, x, y, scale);
 }
 
-extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
-#if GROUPED
-    const int* __restrict__ guard, GROUP_PARAMS long long M, long long N, long long K, long long a_sm, long long a_sk,
-    long long b_sk, long long b_sn
-#if SPLITK
-    , long long k_chunk
-#endif
-    ) {
-    if (guard && *guard == 0) return;
-    float* __restrict__ C;
-    const float* __restrict__ A;
-    const float* __restrict__ B;
-    GROUP_PICK
-    const long long a_off = 0, b_off = 0;
+)";
+}
+
+std::string split_tail() {
+    return R"(    // What the parts cannot represent -- infinities, NaN, operands from 2^111 and sums from 2^95 on -- ends in a sum that
+    // is not finite: such a wavefront's sub-tile is multiplied again on the FP32 matrix cores, straight from memory.  A
+    // lane takes four consecutive k at a time, and two rows of blocks share what is loaded (all four at once spill):
+    // 4096^3 with an infinity in every wavefront's rows 1.8-2.2 ms in all, where one k and one row at a time took 3.8-5.9
+    // (FP32 matrix cores alone, staged through LDS: 1.1).
+    unsigned largest = 0u;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float x = acc[i][j][r];   // (a bit cast of a vector's element itself reads the vector's first)
+                largest = max(largest, __builtin_bit_cast(unsigned, x) & 0x7fffffffu);
+            }
+    const bool again_f32 = __builtin_amdgcn_ballot_w64(largest >= 0x7f800000u) != 0ull;
+    const float unscale = again_f32 ? 1.0f : 1.0f / SCALE / SCALE;
+#define ROWS (TM < 2 ? TM : 2)
+#define KEEP(x) asm volatile("" : "+v"(x));   /* step by step: the addresses of all steps at once cost the 256x256 tile its last registers */
+#pragma unroll
+    for (int i0 = 0; i0 < TM; i0 += ROWS) {
+        if (again_f32) {
+            long long qa[ROWS], qb[TN];   // where its next four k begin
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i) {
+                qa[i] = CLAMP_A(wm * (32 * TM) + 32 * (i0 + i) + li) * a_sm + (k_lo + 4 * lh) * a_sk;
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i0 + i][j][r] = 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < TN; ++j) qb[j] = CLAMP_B(wn * (32 * TN) + 32 * j + li) * b_sn + (k_lo + 4 * lh) * b_sk;
+            auto multiply_f32 = [&](const float* x, const float* y, int stride) {   // one k of a lane
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i0 + i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i * stride], y[j * stride], acc[i0 + i][j], 0, 0, 0);
+            };
+            long long k0 = k_lo;
+#pragma unroll 1
+            for (; k0 + 8 <= k_hi; k0 += 8) {
+                float x[ROWS][4], y[TN][4];
+#if A_KCONTIG
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i) {
+                    *(float4_t*)x[i] = *(const float4_g*)(A + qa[i]);
+                    qa[i] += 8;
+                }
 #else
-    const int* __restrict__ guard, float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ B,
-    long long M, long long N, long long K, long long a_off, long long a_sm, long long a_sk, long long b_off,
-    long long b_sk, long long b_sn
-#if SPLITK
-    , long long k_chunk
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int i = 0; i < ROWS; ++i) {
+                        x[i][q] = A[qa[i]];
+                        qa[i] += (q < 3 ? 1 : 5) * a_sk;
+                        KEEP(qa[i])
+                    }
 #endif
-    EPI_PARAMS) {
-    if (guard && *guard == 0) return;
+#if B_KCONTIG
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    *(float4_t*)y[j] = *(const float4_g*)(B + qb[j]);
+                    qb[j] += 8;
+                }
+#else
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        y[j][q] = B[qb[j]];
+                        qb[j] += (q < 3 ? 1 : 5) * b_sk;
+                        KEEP(qb[j])
+                    }
 #endif
-#if SPLITK
+#pragma unroll
+                for (int q = 0; q < 4; ++q) multiply_f32(&x[0][q], &y[0][q], 4);
+            }
+#pragma unroll 1
+            for (int q = 0; q < 4 && k0 + q < k_hi; ++q) {
+                const bool in = k0 + 4 * lh + q < k_hi;   // (beyond: the last k again, as zero)
+                const long long at = in ? q : k_hi - 1 - (k0 + 4 * lh);
+                float x[ROWS], y[TN];
+#pragma unroll
+                for (int i = 0; i < ROWS; ++i) x[i] = in ? A[qa[i] + at * a_sk] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) y[j] = in ? B[qb[j] + at * b_sk] : 0.0f;
+                multiply_f32(x, y, 1);
+            }
+        }
+        // acc[i][j][4g + r] holds C[row = 32i + 8g + 4*lh + r][col = 32j + li] of the wave's sub-tile
+#pragma unroll
+        for (int i = i0; i < i0 + ROWS; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const long long row = bm + wm * (32 * TM) + 32 * i + 8 * g + 4 * lh + r;
+                    const long long col = bn + wn * (32 * TN) + 32 * j + li;
+                    if (IN_RESULT(row, col))
+                    {
+                        const float sum_value = acc[i][j][4 * g + r] * unscale;
+#if STORE_C
+                        C[row * N + col] = sum_value;
+#endif
+                        EPILOGUE
+                    }
+                }
+    }
+}
+)";
+}
+
+std::string gemm_split_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue) {
+    std::string s = gemm_kernel_head(cfg, epilogue) + gemm_tile_head(cfg);
+    const int per_thread = 8 * (int)gemm_threads(cfg);   // elements of an operand's tile that a thread's unit of eight k covers
+    s += strf("#define BK %d\n#define KW %d\n#define PINGPONG %d\n#define KS %d\n#define RA_VALUE %d\n#define RB_VALUE %d\n", cfg.bk, cfg.k_waves,
+              cfg.bm == 256 ? 1 : 0, cfg.bm == 256 ? cfg.bk / 16 : 1, cfg.bm * cfg.bk / per_thread, gemm_tile_columns(cfg) * cfg.bk / per_thread);
+    s += R"(
+#define KG (BK / 8)                     /* groups of eight k of a tile */
+#define RA RA_VALUE                     /* rows of A (with their eight k) that a thread carries from memory to LDS */
+#define RB RB_VALUE
+#define LDA (BM + 4)                    /* rows of a k group in LDS: the next group starts a quarter of the banks on */
+#define LDB (BN + 4)
+#define WGN (BN / (32 * TN))            /* waves along n */
+#define SCALE 65536.0f                  /* what the parts of an operand are larger by: its third part is then above bf16's smallest number */
+#define SETS (KW == 1 && BK == 32 ? 2 : 1)   /* of accumulators: for the first and second half of a tile's k */
+)" + split_types() + R"()" + gemm_entry(cfg, entry, epilogue, gemm_threads(cfg)) + R"(#if SPLITK
 #if GROUPED
     const unsigned slice = blockIdx.z;  // c<y> points at problem y's own [gridDim.z][M][N] slices
 #else
@@ -157,9 +258,11 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     // rows beyond the product read its last row: what they contribute to is never stored
 #define CLAMP_A(r) min(bm + (long long)(r), M - 1)
 #define CLAMP_B(r) min(bn + (long long)(r), N - 1)
+#define IN_RESULT(row, col) ((row) < M && (col) < N)
 #else
 #define CLAMP_A(r) (bm + (long long)(r))
 #define CLAMP_B(r) (bn + (long long)(r))
+#define IN_RESULT(row, col) true
 #endif
     const int KT = __builtin_amdgcn_readfirstlane((int)((k_hi - k_lo + BK - 1) / BK));
 #if EDGE
@@ -454,122 +557,7 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     }
 #endif
 
-    // What the parts cannot represent -- infinities, NaN, operands from 2^111 and sums from 2^95 on -- ends in a sum that
-    // is not finite: such a wavefront's sub-tile is multiplied again on the FP32 matrix cores, straight from memory.  A
-    // lane takes four consecutive k at a time, and two rows of blocks share what is loaded (all four at once spill):
-    // 4096^3 with an infinity in every wavefront's rows 1.8-2.2 ms in all, where one k and one row at a time took 3.8-5.9
-    // (FP32 matrix cores alone, staged through LDS: 1.1).
-    unsigned largest = 0u;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float x = acc[i][j][r];   // (a bit cast of a vector's element itself reads the vector's first)
-                largest = max(largest, __builtin_bit_cast(unsigned, x) & 0x7fffffffu);
-            }
-    const bool again_f32 = __builtin_amdgcn_ballot_w64(largest >= 0x7f800000u) != 0ull;
-    const float unscale = again_f32 ? 1.0f : 1.0f / SCALE / SCALE;
-#define ROWS (TM < 2 ? TM : 2)
-#define KEEP(x) asm volatile("" : "+v"(x));   /* step by step: the addresses of all steps at once cost the 256x256 tile its last registers */
-#pragma unroll
-    for (int i0 = 0; i0 < TM; i0 += ROWS) {
-        if (again_f32) {
-            long long qa[ROWS], qb[TN];   // where its next four k begin
-#pragma unroll
-            for (int i = 0; i < ROWS; ++i) {
-                qa[i] = CLAMP_A(wm * (32 * TM) + 32 * (i0 + i) + li) * a_sm + (k_lo + 4 * lh) * a_sk;
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i0 + i][j][r] = 0.0f;
-            }
-#pragma unroll
-            for (int j = 0; j < TN; ++j) qb[j] = CLAMP_B(wn * (32 * TN) + 32 * j + li) * b_sn + (k_lo + 4 * lh) * b_sk;
-            auto multiply_f32 = [&](const float* x, const float* y, int stride) {   // one k of a lane
-#pragma unroll
-                for (int i = 0; i < ROWS; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i0 + i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i * stride], y[j * stride], acc[i0 + i][j], 0, 0, 0);
-            };
-            long long k0 = k_lo;
-#pragma unroll 1
-            for (; k0 + 8 <= k_hi; k0 += 8) {
-                float x[ROWS][4], y[TN][4];
-#if A_KCONTIG
-#pragma unroll
-                for (int i = 0; i < ROWS; ++i) {
-                    *(float4_t*)x[i] = *(const float4_g*)(A + qa[i]);
-                    qa[i] += 8;
-                }
-#else
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-#pragma unroll
-                    for (int i = 0; i < ROWS; ++i) {
-                        x[i][q] = A[qa[i]];
-                        qa[i] += (q < 3 ? 1 : 5) * a_sk;
-                        KEEP(qa[i])
-                    }
-#endif
-#if B_KCONTIG
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    *(float4_t*)y[j] = *(const float4_g*)(B + qb[j]);
-                    qb[j] += 8;
-                }
-#else
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        y[j][q] = B[qb[j]];
-                        qb[j] += (q < 3 ? 1 : 5) * b_sk;
-                        KEEP(qb[j])
-                    }
-#endif
-#pragma unroll
-                for (int q = 0; q < 4; ++q) multiply_f32(&x[0][q], &y[0][q], 4);
-            }
-#pragma unroll 1
-            for (int q = 0; q < 4 && k0 + q < k_hi; ++q) {
-                const bool in = k0 + 4 * lh + q < k_hi;   // (beyond: the last k again, as zero)
-                const long long at = in ? q : k_hi - 1 - (k0 + 4 * lh);
-                float x[ROWS], y[TN];
-#pragma unroll
-                for (int i = 0; i < ROWS; ++i) x[i] = in ? A[qa[i] + at * a_sk] : 0.0f;
-#pragma unroll
-                for (int j = 0; j < TN; ++j) y[j] = in ? B[qb[j] + at * b_sk] : 0.0f;
-                multiply_f32(x, y, 1);
-            }
-        }
-        // acc[i][j][4g + r] holds C[row = 32i + 8g + 4*lh + r][col = 32j + li] of the wave's sub-tile
-#pragma unroll
-        for (int i = i0; i < i0 + ROWS; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const long long row = bm + wm * (32 * TM) + 32 * i + 8 * g + 4 * lh + r;
-                    const long long col = bn + wn * (32 * TN) + 32 * j + li;
-#if EDGE
-                    if (row < M && col < N)
-#endif
-                    {
-                        const float sum_value = acc[i][j][4 * g + r] * unscale;
-#if STORE_C
-                        C[row * N + col] = sum_value;
-#endif
-                        EPILOGUE
-                    }
-                }
-    }
-}
-)";
+)" + split_tail();
     return s;
 }
 

@@ -3094,7 +3094,8 @@ struct Lowerer {
         // (the kernel without bounds checks addresses a tile by 32-bit offsets from its corner: lines of 2^22 elements
         // and more take the checked variant, whose index arithmetic is 64 bits wide)
         const int64_t widest = int64_t(1) << 22;
-        return ((a.offset % 4) || (b.offset % 4) || (a_ld % 4) || (b_ld % 4) || (K % 16) || a_ld >= widest || b_ld >= widest) ? 1 : 0;
+        if (a_ld >= widest || b_ld >= widest) return 3;
+        return ((a.offset % 4) || (b.offset % 4) || (a_ld % 4) || (b_ld % 4) || (K % 16)) ? 1 : 0;
     }
 
     template <class ReadsNode, class KeepsEpilogue>
@@ -3433,12 +3434,30 @@ struct Lowerer {
                 const double t = (double)((blocks128 * c + 255) / 256) * (0.045 * (double)K / (double)c + 3) + (c > 1 ? 6 : 0);
                 if (c == 1 || t < best) { best = t; want = c; }
             }
+        } else if (K < 64 || (blocks64 > 256 && K < 512)) {
+            // too short for eight wavefronts to share: more than a round of blocks, or no gain at all (65 x 63 x 33: 7.2 us, 7.4
+            // without a staging buffer, and 7.4e-8 off instead of 5.5e-8, the halves of a tile's k being summed apart)
+            tile(64, 64, 32, 1);
         } else {
-            // few small tiles: a tile's time is the latency of its chain of k-tiles.  Cut from k = 1024 on (at 784
-            // 1000 x 500 takes 22 us whole against 15 + 5 and keeps its epilogue)
-            if (K >= 1024 && blocks64 < 256) want = std::max<int64_t>(std::min<int64_t>((512 + blocks64 - 1) / blocks64, max_splits), 1);
-            if (want == 1 && blocks64 <= 256 && K >= 64) tile(64, 64, 64, 2);
-            else tile(64, 64, 32, 1);
+            // Small outputs: the kernel without a staging buffer, whose blocks take 1.5 us and, per k of 64x64, 64x32 and
+            // 32x32 tiles, 8.6, 6.2 and 4.3 ns, one block per CU at a time.  So the smallest tile of which there are at most 256
+            // (1000 x 500 x 784: 18.2 us on 128 of 64x64, 15.2 on 256 of 32x64, 17.3 on 512 of 32x32; 500 x 320 x 1000 18.6, 14.6,
+            // 12.0), and 64x64 beyond (1000 x 784 x 500: 15.9, 19.8, 20.6).  k is cut from 1280 on, where the slice sum's 5 us pay.
+            double best = 0;
+            for (int64_t c = 1; c <= (K >= 1280 ? max_splits : 1); ++c)
+                for (int form = 0; form < 4; ++form) {
+                    const int bm = form & 1 ? 32 : 64, bn = form & 2 ? 32 : 64;
+                    const double per_k = bm + bn == 128 ? 0.0086 : bm + bn == 96 ? 0.0062 : 0.0043, n_blocks = (double)(blocks(bm, bn) * c);
+                    const double t = std::ceil(n_blocks / 256) * (1.5 + (double)K / (double)c * per_k) + 1e-3 * n_blocks + (c > 1 ? 5 : 0);
+                    if ((c == 1 && form == 0) || t < best) {
+                        best = t;
+                        want = c;
+                        tile(bm, bn, 32, kDirectWaves);
+                    }
+                }
+            cfg.narrow_m = M < cfg.bm;
+            cfg.narrow_n = N < cfg.bn;
+            cfg.wide_lines = alignment == 3;
         }
         // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits> forces tile and k ranges of every product with k of 64 and more
         if (const char* e = getenv("ADHIP_DOT_PLAN")) {
@@ -3463,15 +3482,16 @@ struct Lowerer {
     }
 
     static std::string dot_kernel_name(const GemmConfig& cfg) {
-        std::string s = strf("adhip_gemm_%c%c_%d", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', cfg.bm);
-        if (cfg.bm != 64 && gemm_tile_columns(cfg) == 64) s += "x64";
+        std::string s = strf("adhip_gemm_%c%c_%d", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', std::max(cfg.bm, 64));
+        if (cfg.bm > 64 && gemm_tile_columns(cfg) == 64) s += "x64";
         if (cfg.edge) s += cfg.bf16_parts || cfg.edge_vec ? "_rim" : "_edge";
         if (cfg.split_k) s += "_splitk";
-        else if (cfg.k_waves == 2) s += "_pair";
+        else if (cfg.k_waves > 1) s += "_pair";
         if (!cfg.bf16_parts) s += "_f32";
         return s;
     }
     static std::string gemm_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr) {
+        if (cfg.k_waves == kDirectWaves) return gemm_direct_kernel_source(cfg, entry, epilogue);
         return cfg.bf16_parts ? gemm_split_kernel_source(cfg, entry, epilogue) : gemm_kernel_source(cfg, entry, epilogue);
     }
 
