@@ -1,5 +1,7 @@
 #include "lower.hpp"
 
+#include "../../include/adhip.h"
+
 #include <algorithm>
 #include <array>
 #include <cctype>
@@ -236,9 +238,8 @@ extern "C" __global__ __launch_bounds__(256) void adhip_sum_slices(const int* __
 
 // The same for up to 16 products that shared one launch: blockIdx.y picks the product, whose slices are
 // slices[y][count][n] and whose result goes to o<y>.
-#define ADHIP_O16 float* o0, float* o1, float* o2, float* o3, float* o4, float* o5, float* o6, float* o7, float* o8, float* o9, \
-                  float* o10, float* o11, float* o12, float* o13, float* o14, float* o15
-extern "C" __global__ __launch_bounds__(256) void adhip_sum_slices_grouped(const int* __restrict__ guard, ADHIP_O16,
+extern "C" __global__ __launch_bounds__(256) void adhip_sum_slices_grouped(const int* __restrict__ guard, float* o0, float* o1, float* o2,
+    float* o3, float* o4, float* o5, float* o6, float* o7, float* o8, float* o9, float* o10, float* o11, float* o12, float* o13, float* o14, float* o15,
                                                                            const float* __restrict__ slices, long long count,
                                                                            long long n) {
     if (guard && *guard == 0) return;
@@ -329,7 +330,7 @@ struct Lowerer {
     std::map<RegionKey, IdSet> region_live;
     std::vector<std::unique_ptr<Node>> arena;
     std::map<std::string, int> kernel_by_source;
-    int kernel_counter = 0;
+    int kernel_counter = 0, shared_counter = 0;
     std::map<std::pair<int, int>, int> layered_kernels;
     int fixed_copy = -1, fixed_dot = -1, fixed_dot_tiny = -1, fixed_transpose = -1, fixed_transpose4 = -1, fixed_finalize = -1, fixed_sums_finalize = -1, fixed_sum_slices = -1, fixed_sum_slices_grouped = -1;
     int dot_epilogue_counter = 0;
@@ -357,6 +358,8 @@ struct Lowerer {
 
     Lowerer(const Proc& p, const std::vector<std::string>& d, const LowerOptions& o) : prog(p), opt(o) {
         for (auto& s : d) deps.insert(s);
+        pool_packed.packed = true;
+        pool.packed = opt.pack_slots;
     }
 
     // -----------------------------------------------------------------------------------
@@ -599,32 +602,58 @@ struct Lowerer {
         return it->second;
     }
 
-    std::vector<std::pair<int64_t, bool>> slots;  // (elems, in use)
-    int alloc_temp(int64_t elems, const std::string& name) {
-        elems = std::max<int64_t>(elems, 1);
-        int best = -1;
-        for (size_t i = 0; i < slots.size(); ++i) {
-            if (slots[i].second) continue;
-            if (best < 0) { best = (int)i; continue; }
-            const int64_t cur = slots[best].first, cand = slots[i].first;
-            const bool cur_fits = cur >= elems, cand_fits = cand >= elems;
-            if (cand_fits && (!cur_fits || cand < cur)) best = (int)i;
-            else if (!cand_fits && !cur_fits && cand > cur) best = (int)i;
+    struct SlotPool {
+        bool packed = false;   // any free slot will do
+        std::vector<std::pair<int64_t, bool>> slots;  // (elems, in use)
+        int take(int64_t elems) {
+            int best = -1;
+            for (size_t i = 0; i < slots.size(); ++i) {
+                // (a small temporary would only keep a large slot from its like)
+                if (slots[i].second || (!packed && slots[i].first > 8 * elems + 256)) continue;
+                if (best < 0) { best = (int)i; continue; }
+                const int64_t cur = slots[best].first, cand = slots[i].first;
+                const bool cur_fits = cur >= elems, cand_fits = cand >= elems;
+                if (cand_fits && (!cur_fits || cand < cur)) best = (int)i;
+                else if (!cand_fits && !cur_fits && cand > cur) best = (int)i;
+            }
+            if (best < 0) { slots.push_back({elems, true}); best = (int)slots.size() - 1; }
+            slots[best].first = std::max(slots[best].first, elems);
+            slots[best].second = true;
+            return best;
         }
-        if (best < 0) { slots.push_back({elems, true}); best = (int)slots.size() - 1; }
-        slots[best].first = std::max(slots[best].first, elems);
-        slots[best].second = true;
+    };
+    // The pool the program runs on, and what it would need with every launch for itself, and with every slot for anybody
+    // on top: a program whose temporaries fit the static scratch area in one of these ways is lowered that way (lower_program).
+    SlotPool pool, pool_apart, pool_packed;
+    size_t apart_bytes = 0, packed_bytes = 0;
+    // A temporary of the region being lowered; what memory it takes is decided when the region's launches stand
+    // (assign_slots), so that two launches only share memory, and depend on one another for it, if they run one after the other.
+    int alloc_temp(int64_t elems, const std::string& name) {
         PlanBuffer b;
         b.kind = PlanBuffer::TEMP;
         b.name = name;
-        b.elems = elems;
-        b.slot = best;
+        b.elems = std::max<int64_t>(elems, 1);
         plan->buffers.push_back(b);
         return (int)plan->buffers.size() - 1;
     }
-    void free_temp(int buf) {
-        const PlanBuffer& b = plan->buffers[buf];
-        if (b.kind == PlanBuffer::TEMP) slots[b.slot].second = false;
+    // Every temporary of a region has a slot from the first launch that names it to the last.
+    void assign_slots(const std::vector<Step>& out, size_t from, SlotPool& p) {
+        std::map<int, std::pair<size_t, size_t>> life;   // buffer -> first and last step
+        for (size_t i = from; i < out.size(); ++i)
+            for (const Arg& a : out[i].launch.args)
+                if (a.kind == Arg::BUF && plan->buffers[(size_t)a.buf].kind == PlanBuffer::TEMP) {
+                    auto it = life.emplace(a.buf, std::make_pair(i, i)).first;
+                    it->second.second = i;
+                }
+        std::vector<std::vector<int>> begin(out.size()), end(out.size());
+        for (auto& kv : life) {
+            begin[kv.second.first].push_back(kv.first);
+            end[kv.second.second].push_back(kv.first);
+        }
+        for (size_t i = from; i < out.size(); ++i) {
+            for (int b : begin[i]) plan->buffers[(size_t)b].slot = p.take(plan->buffers[(size_t)b].elems);
+            for (int b : end[i]) p.slots[(size_t)plan->buffers[(size_t)b].slot].second = false;
+        }
     }
 
     // -----------------------------------------------------------------------------------
@@ -966,7 +995,7 @@ struct Lowerer {
     // Kernels are told apart by their text with the entry name blanked: the per-head kernels of multi-head attention
     // (and the same epilogue generated for two layers) differ in nothing but the position in the program that their
     // name carries, and then share the first one's code object instead of being compiled once each.
-    int add_kernel(const std::string& entry, const std::string& source, const std::string& kind) {
+    int add_kernel(const std::string& entry, const std::string& source, const std::string& kind, size_t shared_bytes = 0) {
         std::string key;
         key.reserve(source.size());
         auto ident = [](char c) { return isalnum((unsigned char)c) || c == '_'; };
@@ -990,6 +1019,7 @@ struct Lowerer {
         d.entry = entry;
         d.source = source;
         d.kind = kind;
+        d.shared_bytes = shared_bytes;
         d.regions.push_back(cur_region);
         plan->kernels.push_back(std::move(d));
         kernel_by_source[key] = (int)plan->kernels.size() - 1;
@@ -1274,7 +1304,6 @@ struct Lowerer {
         std::map<Node*, std::string> home_of;                // wanted node -> id
         std::vector<GroupKernels> gks;                       // per group: generated code
         std::vector<std::map<Node*, bool>> greads;           // per group: reads, for hazard analysis
-        std::vector<int> set_end;                            // per group: last group of the shared launches it runs in
         std::vector<Commit> commits;                         // results computed beside their home buffer, copied in at the end
     };
 
@@ -1294,6 +1323,246 @@ struct Lowerer {
         const size_t first_step = out.size();
         flush_region_launches(live, final_region, out);
         if (opt.fuse && opt.merge_small) merge_single_block_runs(out, first_step);
+        assign_slots(out, first_step, pool_packed);
+        assign_slots(out, first_step, pool_apart);
+        if (opt.fuse && opt.share_independent && !tight() && !opt.unshared_regions.count(cur_region)) share_independent_launches(out, first_step);
+        assign_slots(out, first_step, pool);
+    }
+
+    // The parameters of a kernel's entry behind `guard`, type and name, as they stand in its source (none if it cannot be told),
+    // and where its parameter list begins and ends.
+    struct EntryText {
+        size_t open = std::string::npos, close = std::string::npos;
+        std::vector<std::pair<std::string, std::string>> params;
+    };
+    static EntryText entry_text(const std::string& source, const std::string& entry) {
+        EntryText t;
+        const size_t fn = source.find(" void " + entry + "(");
+        if (fn == std::string::npos) return t;
+        const size_t open = source.find('(', fn), close = source.find(") {", open);
+        if (close == std::string::npos) return t;
+        const std::string list = source.substr(open + 1, close - open - 1);
+        for (size_t pos = 0; pos <= list.size();) {
+            const size_t comma = std::min(list.find(',', pos), list.size());
+            std::string prm = list.substr(pos, comma - pos);
+            pos = comma + 1;
+            while (!prm.empty() && isspace((unsigned char)prm.front())) prm.erase(prm.begin());
+            while (!prm.empty() && isspace((unsigned char)prm.back())) prm.pop_back();
+            const size_t sp = prm.find_last_of(" *");
+            if (sp == std::string::npos || prm.find('#') != std::string::npos) return t;
+            t.params.push_back({prm.substr(0, sp + 1), prm.substr(sp + 1)});
+        }
+        t.params.erase(t.params.begin());   // guard
+        t.open = open;
+        t.close = close;
+        return t;
+    }
+
+    // Launches of one region that do not depend on one another run as one: a launch of a few dozen blocks costs 2-5 us beside its
+    // work and leaves most of the chip idle, and a training step on small tensors has twice as many of them as its longest
+    // chain of dependences (a perceptron: 18 launches, 9 deep; an encoder layer: 35 and 22).  What a launch reads and
+    // writes stands in its arguments and its entry's parameters (`const` or not); from that order, every time, the launch with
+    // the longest way to the end comes next, and takes along what else is ready and fits beside it.  The shared kernel
+    // holds every member's translation unit in a namespace of its own, in which the block's number counts from the member's
+    // first block, and one piece of LDS for all members that ask for a large one.
+    //
+    // Members have at most 512 blocks, all of them together at most 1024, and with a matrix-core product among them, whose
+    // LDS leaves a CU to one block at a time, 512: what is larger fills the chip by itself, and stays where it is.  Kernels
+    // of 1024 threads (128 vector registers a lane) are kept from products and row chains, which need more.
+    // Nothing is taken from further than 64 launches behind the oldest one left: what waits for its readers takes memory.
+    static constexpr int kSharedArgs = 360, kSharedMembers = 12;
+    static constexpr size_t kSharedWindow = 64;
+    // LDS that a kernel has for itself in such a launch (at most)
+    static size_t own_lds(const KernelDef& kd, unsigned threads) {
+        if (kd.kind == "dot_mfma") return kd.shared_bytes ? 0 : 2 * 2 * 16 * 68 * 4;
+        if (kd.kind == "elw_colsum") return 2 * 16 * 64 * 16;
+        return threads > 512 ? 16 * 64 * 16 : 4352;
+    }
+    static bool small_product(const KernelDef& kd) { return kd.shared_bytes > 0 || kd.entry.find("_64") != std::string::npos; }
+    void share_independent_launches(std::vector<Step>& out, size_t from) {
+        for (size_t at = from; at < out.size();) {
+            while (at < out.size() && !can_share(out[at])) ++at;
+            size_t end = at;
+            while (end < out.size() && can_share(out[end]) && out[end].launch.guard == out[at].launch.guard) ++end;
+            at += share_run(out, at, end);
+        }
+    }
+    bool can_share(const Step& st) const {
+        static const std::set<std::string> shareable = {"elw", "reduce_row", "reduce_row_store", "reduce_col", "rowchain", "dot_naive", "dot_mfma", "copy",
+                                                        "sum_slices", "merged", "elw_colsum", "colsum_finalize", "sums_finalize"};
+        if (st.kind != Step::LAUNCH) return false;
+        const Launch& l = st.launch;
+        const KernelDef& kd = plan->kernels[(size_t)l.kernel];
+        for (const Arg& a : l.args)
+            if (a.kind == Arg::FLAG) return false;   // (the loop's last kernel stays its last)
+        return shareable.count(kd.kind) && l.block[1] == 1 && l.block[2] == 1 && l.lds_bytes == 0 && (uint64_t)l.grid[0] * l.grid[1] * l.grid[2] <= 512 &&
+               (kd.kind != "dot_mfma" || small_product(kd));
+    }
+    // A run of such launches; returns how many are left of it.
+    size_t share_run(std::vector<Step>& out, size_t from, size_t to) {
+        const size_t n = to - from;
+        if (n < 2) return n;
+        struct Item {
+            bool ok = false;          // its parameters are known
+            bool product = false;     // on the matrix cores
+            bool chain = false;       // keeps a row in registers
+            int64_t blocks = 0;
+            unsigned threads = 0;
+            size_t own = 0, shared = 0;   // bytes of LDS
+            EntryText text;
+            std::set<int> reads, writes;
+            std::vector<size_t> before;   // what it depends on
+            int height = 0;               // launches on the longest way from it to the run's end
+        };
+        std::vector<Item> items(n);
+        for (size_t i = 0; i < n; ++i) {
+            const Launch& l = out[from + i].launch;
+            const KernelDef& kd = plan->kernels[(size_t)l.kernel];
+            Item& it = items[i];
+            it.text = entry_text(kd.source, kd.entry);
+            it.ok = it.text.open != std::string::npos && it.text.params.size() == l.args.size();
+            for (size_t a = 0; a < l.args.size(); ++a) {
+                if (l.args[a].kind != Arg::BUF) continue;
+                it.reads.insert(l.args[a].buf);
+                if (!it.ok || it.text.params[a].first.find("const") == std::string::npos) it.writes.insert(l.args[a].buf);
+            }
+            it.product = kd.kind == "dot_mfma";
+            it.chain = kd.kind == "rowchain";
+            it.blocks = (int64_t)l.grid[0] * l.grid[1] * l.grid[2];
+            it.threads = l.block[0];
+            it.own = own_lds(kd, it.threads);
+            it.shared = kd.shared_bytes;
+            for (size_t j = 0; j < i; ++j) {
+                auto meet = [](const std::set<int>& x, const std::set<int>& y) {
+                    for (int b : x)
+                        if (y.count(b)) return true;
+                    return false;
+                };
+                if (meet(items[j].writes, it.reads) || meet(items[j].reads, it.writes)) it.before.push_back(j);
+            }
+        }
+        for (size_t i = n; i-- > 0;) {
+            ++items[i].height;
+            for (size_t j : items[i].before) items[j].height = std::max(items[j].height, items[i].height);
+        }
+        std::vector<char> done(n, 0);
+        std::vector<std::vector<size_t>> sets;
+        for (size_t left = n; left > 0;) {
+            std::vector<size_t> ready;
+            const size_t oldest = (size_t)(std::find(done.begin(), done.end(), 0) - done.begin());
+            for (size_t i = oldest; i < std::min(n, oldest + kSharedWindow); ++i)
+                if (!done[i] && std::all_of(items[i].before.begin(), items[i].before.end(), [&](size_t j) { return done[j] != 0; })) ready.push_back(i);
+            std::stable_sort(ready.begin(), ready.end(), [&](size_t x, size_t y) { return items[x].height > items[y].height; });
+            std::vector<size_t> set{ready[0]};
+            Item sum = items[ready[0]];
+            size_t args = out[from + ready[0]].launch.args.size();
+            for (size_t q = 1; q < ready.size() && sum.ok && set.size() < (size_t)kSharedMembers; ++q) {
+                const Item& it = items[ready[q]];
+                const size_t more = out[from + ready[q]].launch.args.size();
+                const bool product = sum.product || it.product;
+                const unsigned threads = std::max(sum.threads, it.threads);
+                const bool mixed = threads != std::min(sum.threads, it.threads), chain = sum.chain || it.chain;
+                if (!it.ok || ((product || chain) && threads > 512) || (mixed && sum.blocks + it.blocks > 512) || sum.blocks + it.blocks > (product ? 512 : 1024) || args + more > (size_t)kSharedArgs ||
+                    sum.own + it.own + std::max(sum.shared, it.shared) > 160 * 1024)
+                    continue;
+                set.push_back(ready[q]);
+                sum.product = product;
+                sum.chain = chain;
+                sum.threads = threads;
+                sum.blocks += it.blocks;
+                sum.own += it.own;
+                sum.shared = std::max(sum.shared, it.shared);
+                args += more;
+            }
+            for (size_t i : set) done[i] = 1;
+            left -= set.size();
+            sets.push_back(std::move(set));
+        }
+        if (sets.size() == n) return n;
+        std::vector<Step> steps;
+        for (std::vector<size_t>& set : sets) {
+            if (set.size() == 1) {
+                steps.push_back(std::move(out[from + set[0]]));
+                continue;
+            }
+            // products first: they take longest
+            std::stable_sort(set.begin(), set.end(), [&](size_t x, size_t y) { return items[x].product > items[y].product; });
+            steps.push_back(shared_launch(out, from, set, items));
+        }
+        out.erase(out.begin() + (std::ptrdiff_t)from, out.begin() + (std::ptrdiff_t)to);
+        out.insert(out.begin() + (std::ptrdiff_t)from, std::make_move_iterator(steps.begin()), std::make_move_iterator(steps.end()));
+        return steps.size();
+    }
+
+    template <class Items>
+    Step shared_launch(const std::vector<Step>& out, size_t from, const std::vector<size_t>& set, const Items& items) {
+        Launch m;
+        m.guard = out[from + set[0]].launch.guard;
+        std::string src, calls, params = "const int* guard";
+        size_t shared = 0;
+        unsigned first = 0;
+        for (size_t i : set) {
+            m.block[0] = std::max(m.block[0], out[from + i].launch.block[0]);
+            shared = std::max(shared, plan->kernels[(size_t)out[from + i].launch.kernel].shared_bytes);
+        }
+        if (shared) src += strf("static __device__ __forceinline__ char* adhip_lds() {\n    __shared__ __attribute__((aligned(16))) char lds[%zu];\n    return lds;\n}\n", shared);
+        for (size_t q = 0; q < set.size(); ++q) {
+            const Launch& l = out[from + set[q]].launch;
+            const KernelDef& kd = plan->kernels[(size_t)l.kernel];
+            std::string body = kd.source;
+            auto replace_all = [&](const std::string& what, const std::string& with) {
+                for (size_t at = body.find(what); at != std::string::npos; at = body.find(what, at + with.size())) body.replace(at, what.size(), with);
+            };
+            replace_all("extern \"C\" __global__", "static __device__ __forceinline__");
+            for (size_t at = body.find("__launch_bounds__("); at != std::string::npos; at = body.find("__launch_bounds__(")) body.erase(at, body.find(')', at) + 1 - at);
+            replace_all("blockIdx", "adhip_block()");
+            if (kd.shared_bytes) {
+                // (the product kernels' one array: "__shared__ __attribute__((aligned(16))) <type> lds[...];")
+                const size_t at = body.find("__shared__ __attribute__((aligned(16))) "), name = body.find(" lds[", at), end = body.find(';', at);
+                ADHIP_CHECK(end != std::string::npos && name < end, "internal: kernel '%s' has no LDS array", kd.entry.c_str());
+                const size_t type = at + strlen("__shared__ __attribute__((aligned(16))) ");
+                const std::string elem = body.substr(type, name - type);
+                body.replace(at, end - at, elem + "* const lds = (" + elem + "*)adhip_lds()");
+            }
+            // macros end with the namespace
+            std::string undef;
+            for (size_t at = body.find("#define "); at != std::string::npos; at = body.find("#define ", at + 8)) {
+                size_t e = at + 8;
+                while (e < body.size() && (isalnum((unsigned char)body[e]) || body[e] == '_')) ++e;
+                undef += "#undef " + body.substr(at + 8, e - at - 8) + "\n";
+            }
+            const unsigned blocks = l.grid[0] * l.grid[1] * l.grid[2];
+            src += strf("namespace part%zu {\nstruct adhip_block_t { unsigned x, y, z; };\nstatic __device__ __forceinline__ adhip_block_t adhip_block() {\n"
+                        "    const unsigned b = blockIdx.x - %uu;\n    return {b %% %uu, b / %uu %% %uu, b / %uu};\n}\n",
+                        q, first, l.grid[0], l.grid[0], l.grid[1], l.grid[0] * l.grid[1]);
+            src += body + "\n}\n" + undef;
+            std::string args;
+            for (size_t a = 0; a < l.args.size(); ++a) {
+                const std::string name = strf("p%zu_%s", q, items[set[q]].text.params[a].second.c_str());
+                params += ", " + items[set[q]].text.params[a].first + name;
+                args += ", " + name;
+            }
+            const bool last = q + 1 == set.size();
+            calls += last ? "    {\n" : strf("    if (blockIdx.x < %uu) {\n", first + blocks);
+            // (wavefronts beyond a member's block end here, and barriers do not wait for them)
+            if (l.block[0] < m.block[0]) calls += strf("        if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= %uu) return;\n", l.block[0]);
+            calls += strf("        part%zu::%s(guard%s);\n        return;\n    }\n", q, kd.entry.c_str(), args.c_str());
+            first += blocks;
+            m.args.insert(m.args.end(), l.args.begin(), l.args.end());
+            m.bytes += l.bytes;
+            m.flops += l.flops;
+        }
+        m.grid[0] = first;
+        const std::string entry = strf("shared%d_%zux", shared_counter++, set.size());
+        src += strf("extern \"C\" __global__ __launch_bounds__(%u) void ", m.block[0]) + entry + "(" + params + ") {\n" + calls + "}\n";
+        m.kernel = add_kernel(entry, src, "shared");
+        m.label = entry;
+        std::vector<size_t> in_order = set;
+        std::sort(in_order.begin(), in_order.end());
+        for (size_t i : in_order) m.parts.push_back(out[from + i].launch);
+        std::vector<Step> one;
+        push_launch(one, m, "shared");
+        return std::move(one[0]);
     }
 
     // Consecutive launches of one region that are a single block each (the kernels of a program on tiny tensors: the
@@ -1332,27 +1601,15 @@ struct Lowerer {
                 for (size_t at = body.find(bounds); at != std::string::npos; at = body.find(bounds)) body.erase(at, body.find(')', at) + 1 - at);
                 // a buffer one phase writes is another phase's input: no parameter may promise that nothing else names its memory
                 for (size_t at = body.find(noalias); at != std::string::npos; at = body.find(noalias)) body.erase(at, noalias.size());
-                const size_t fn = body.find(" void " + kd.entry + "(");
-                const size_t open = fn == std::string::npos ? fn : body.find('(', fn);
-                const size_t close = open == std::string::npos ? open : body.find(") {", open);
-                if (close == std::string::npos) { ok = false; break; }
-                std::string list = body.substr(open + 1, close - open - 1), args;
-                size_t pos = 0, index = 0;
-                while (pos < list.size()) {
-                    size_t comma = list.find(',', pos);
-                    if (comma == std::string::npos) comma = list.size();
-                    std::string prm = list.substr(pos, comma - pos);
-                    pos = comma + 1;
-                    while (!prm.empty() && isspace((unsigned char)prm.front())) prm.erase(prm.begin());
-                    while (!prm.empty() && isspace((unsigned char)prm.back())) prm.pop_back();
-                    if (index++ == 0) continue;  // guard
-                    const size_t sp = prm.find_last_of(" *");
-                    if (sp == std::string::npos) { ok = false; break; }
-                    const std::string name = strf("s%zu_%s", q - i, prm.substr(sp + 1).c_str());
-                    params += ", " + prm.substr(0, sp + 1) + name;
+                const EntryText text = entry_text(body, kd.entry);
+                // the launch must pass exactly the entry's parameters
+                if (text.open == std::string::npos || text.params.size() != l.args.size()) { ok = false; break; }
+                std::string args;
+                for (auto& prm : text.params) {
+                    const std::string name = strf("s%zu_%s", q - i, prm.second.c_str());
+                    params += ", " + prm.first + name;
                     args += ", " + name;
                 }
-                if (index != l.args.size() + 1) ok = false;  // the launch must pass exactly the entry's parameters
                 src += strf("namespace seg%zu {\n", q - i) + body + "\n}\n";
                 calls += strf("    seg%zu::%s(guard%s);\n", q - i, kd.entry.c_str(), args.c_str());
                 if (q + 1 < j) calls += "    __syncthreads();\n";
@@ -2711,24 +2968,8 @@ struct Lowerer {
         auto& groups = rp.groups;
         auto& gks = rp.gks;
         auto& greads = rp.greads;
-        auto& set_end = rp.set_end;
         auto& commits = rp.commits;
         const auto& home_of = rp.home_of;
-        // the last group of the shared launches a group runs in (itself if it runs alone)
-        set_end.assign(groups.size(), 0);
-        for (size_t g = 0; g < groups.size(); ++g) {
-            set_end[g] = (int)g;
-            const int lead = groups[g].lead;
-            if (lead >= 0)
-                for (int q = lead; q <= (int)g; ++q) set_end[q] = (int)g;
-        }
-        std::vector<int> last_use(arena.size() + 16, -1);
-        std::map<Node*, int> last_reader;
-        for (size_t g = 0; g < groups.size(); ++g)
-            if (!groups[g].dead)
-                for (auto& rd : greads[g]) last_reader[rd.first] = (int)g;
-        std::vector<std::vector<Node*>> free_after(groups.size());
-        std::vector<int> scratch_to_free;
         for (size_t g = 0; g < groups.size(); ++g) {
             if (groups[g].dead) continue;
             std::vector<Node*> produced = groups[g].members;
@@ -2781,29 +3022,15 @@ struct Lowerer {
                     else {
                         m->buffer = alloc_temp(numel(m->shape), id + ".new");
                         commits.push_back({hb, m->buffer, numel(m->shape), id});
-                        // released after the commits
                     }
                 } else {
                     m->buffer = alloc_temp(numel(m->shape), m->name + ".tmp");
-                    auto lr = last_reader.find(m);
-                    int when = lr == last_reader.end() ? (int)g : std::max(lr->second, (int)g);
-                    free_after[set_end[when]].push_back(m);  // groups that share launches run at the same time
                 }
             }
-            // partial-sum scratch of chunked reductions lives only inside this group
-            for (Node* e : gks[g].extra_nodes) {
-                if (e->op == Op::COPY) e->buffer = alloc_temp(numel(e->shape), e->name);
-            }
+            // partial sums
             for (Node* e : gks[g].extra_nodes)
-                if (e->op == Op::COPY) scratch_to_free.push_back(e->buffer);
-            for (Node* e : gks[g].row_partials) {
-                e->buffer = alloc_temp(numel(e->shape), e->name);
-                scratch_to_free.push_back(e->buffer);
-            }
-            if (set_end[g] != (int)g) continue;
-            for (int b : scratch_to_free) free_temp(b);
-            scratch_to_free.clear();
-            for (Node* f : free_after[g]) free_temp(f->buffer);
+                if (e->op == Op::COPY) e->buffer = alloc_temp(numel(e->shape), e->name);
+            for (Node* e : gks[g].row_partials) e->buffer = alloc_temp(numel(e->shape), e->name);
         }
     }
 
@@ -2973,7 +3200,6 @@ struct Lowerer {
         }
         if (latch_region && latch_slot >= 0 && commits.empty() && opt.fuse) attach_latch(rp, out);
         for (auto& c : commits) emit_copy(out, c.dst, c.src, c.n, "commit_" + c.id);
-        for (auto& c : commits) free_temp(c.src);
     }
 
     // The region is the last one of a device-predicated loop's body.  When its last launch is the generated kernel
@@ -3234,7 +3460,7 @@ struct Lowerer {
         const std::string entry = small ? "adhip_dot_small_grouped" : dot_kernel_name(cfg) + "_grouped", kind = small ? "dot_naive" : "dot_mfma";
         const int lanes = small_dot_lanes(M, N, K, key0[4] <= key0[3] && key0[5] <= key0[6]);
         Launch l;
-        l.kernel = add_kernel(entry, small ? dot_small_source(entry, nullptr, true) : gemm_source(cfg, entry), kind);
+        l.kernel = add_kernel(entry, small ? dot_small_source(entry, nullptr, true) : gemm_source(cfg, entry), kind, small ? 0 : gemm_shared_bytes(cfg));
         l.block[0] = small ? 256u : gemm_threads(cfg);
         l.grid[0] = (unsigned)(small ? (M * N * lanes + 255) / 256 : ((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile));
         l.grid[1] = (unsigned)cnt;
@@ -3520,9 +3746,9 @@ struct Lowerer {
                 ge.params = epi->params;
                 ge.code = epi->code;
                 ge.store_c = store_c;
-                l.kernel = add_kernel(entry, gemm_source(cfg, entry, &ge), "dot_mfma");
+                l.kernel = add_kernel(entry, gemm_source(cfg, entry, &ge), "dot_mfma", gemm_shared_bytes(cfg));
             } else {
-                l.kernel = add_kernel(entry, gemm_source(cfg, entry), "dot_mfma");
+                l.kernel = add_kernel(entry, gemm_source(cfg, entry), "dot_mfma", gemm_shared_bytes(cfg));
             }
             l.block[0] = gemm_threads(cfg);
             l.grid[0] = (unsigned)(((M + cfg.bm - 1) / cfg.bm) * ((N + bn_tile - 1) / bn_tile));
@@ -3869,7 +4095,19 @@ struct Lowerer {
             r.shape = it->second.shape;
             plan->results[d] = r;
         }
-        for (auto& s : slots) plan->slot_elems.push_back(s.first);
+        for (PlanBuffer& b : plan->buffers)
+            if (b.kind == PlanBuffer::TEMP && b.slot < 0) {   // no launch names it
+                if (pool.slots.empty()) pool.slots.push_back({1, false});
+                b.slot = 0;
+            }
+        auto bytes = [&](const SlotPool& p) {
+            plan->slot_elems.clear();
+            for (auto& s : p.slots) plan->slot_elems.push_back(s.first);
+            return plan->temp_bytes();
+        };
+        apart_bytes = bytes(pool_apart);
+        packed_bytes = bytes(pool_packed);
+        bytes(pool);
         drop_unused_kernels();
         return std::move(plan);
     }
@@ -3883,10 +4121,16 @@ struct Lowerer {
                 if (st.kind == Step::LAUNCH) {
                     if (!assign) {
                         kernel_map[(size_t)st.launch.kernel] = 0;
+                        plan->kernels[(size_t)st.launch.kernel].part_only = false;
                         if (st.launch.stat >= 0) stat_map[(size_t)st.launch.stat] = 0;
                     } else {
                         st.launch.kernel = kernel_map[(size_t)st.launch.kernel];
                         if (st.launch.stat >= 0) st.launch.stat = stat_map[(size_t)st.launch.stat];
+                    }
+                    for (Launch& part : st.launch.parts) {
+                        if (!assign) kernel_map[(size_t)part.kernel] = 0;
+                        else part.kernel = kernel_map[(size_t)part.kernel];
+                        part.stat = -1;
                     }
                 }
                 walk(st.body, assign);
@@ -3894,6 +4138,7 @@ struct Lowerer {
                 walk(st.else_body, assign);
             }
         };
+        for (KernelDef& k : plan->kernels) k.part_only = true;
         walk(plan->steps, false);
         std::vector<KernelDef> kernels;
         for (size_t i = 0; i < plan->kernels.size(); ++i)
@@ -3911,22 +4156,27 @@ struct Lowerer {
     }
 };
 
+void describe_launch(const Launch& l, const Plan& p, const std::string& pad, std::string& o) {
+    o += pad + strf("launch %s [%s] kernel=%s grid=(%u,%u,%u) block=%u bytes=%.0f flops=%.0f args:", l.label.c_str(),
+                    p.kernels[l.kernel].kind.c_str(), p.kernels[l.kernel].entry.c_str(), l.grid[0], l.grid[1], l.grid[2],
+                    l.block[0], l.bytes, l.flops);
+    for (const Arg& a : l.args) {
+        if (a.kind == Arg::BUF) o += " " + p.buffers[a.buf].name + "#" + std::to_string(a.buf) + (a.off ? strf("+%lld", (long long)a.off) : std::string());
+        else if (a.kind == Arg::F32) o += strf(" %g", a.fv);
+        else if (a.kind == Arg::FLAG) o += strf(" flag%lld", (long long)a.iv);
+        else o += strf(" %lld", (long long)a.iv);
+    }
+    o += "\n";
+}
+
 void describe_steps(const std::vector<Step>& steps, const Plan& p, int indent, std::string& o) {
     std::string pad((size_t)indent * 2, ' ');
     for (const Step& s : steps) {
         switch (s.kind) {
         case Step::LAUNCH: {
-            const Launch& l = s.launch;
-            o += pad + strf("launch %s [%s] kernel=%s grid=(%u,%u,%u) block=%u bytes=%.0f flops=%.0f args:", l.label.c_str(),
-                            p.kernels[l.kernel].kind.c_str(), p.kernels[l.kernel].entry.c_str(), l.grid[0], l.grid[1], l.grid[2],
-                            l.block[0], l.bytes, l.flops);
-            for (const Arg& a : l.args) {
-                if (a.kind == Arg::BUF) o += " " + p.buffers[a.buf].name + "#" + std::to_string(a.buf) + (a.off ? strf("+%lld", (long long)a.off) : std::string());
-                else if (a.kind == Arg::F32) o += strf(" %g", a.fv);
-                else if (a.kind == Arg::FLAG) o += strf(" flag%lld", (long long)a.iv);
-                else o += strf(" %lld", (long long)a.iv);
-            }
-            o += "\n";
+            if (s.launch.parts.empty()) describe_launch(s.launch, p, pad, o);
+            else o += pad + strf("%s, one launch of grid=(%u,1,1) block=%u:\n", s.launch.label.c_str(), s.launch.grid[0], s.launch.block[0]);
+            for (const Launch& part : s.launch.parts) describe_launch(part, p, pad, o);
             break;
         }
         case Step::LOOP:
@@ -3958,7 +4208,8 @@ void describe_steps(const std::vector<Step>& steps, const Plan& p, int indent, s
 
 std::string Plan::describe() const {
     std::string o;
-    o += strf("buffers: %zu (temp slots: %zu), kernels: %zu\n", buffers.size(), slot_elems.size(), kernels.size());
+    const size_t own = (size_t)std::count_if(kernels.begin(), kernels.end(), [](const KernelDef& k) { return k.kind != "shared"; });
+    o += strf("buffers: %zu (temp slots: %zu), kernels: %zu\n", buffers.size(), slot_elems.size(), own);
     for (size_t i = 0; i < buffers.size(); ++i) {
         const PlanBuffer& b = buffers[i];
         o += strf("  #%zu %s %s elems=%lld%s%s\n", i, b.kind == PlanBuffer::HOME ? "home" : (b.kind == PlanBuffer::TEMP ? "temp" : "const"),
@@ -3970,7 +4221,7 @@ std::string Plan::describe() const {
 
 std::string lowering_switches() {
     std::string out;
-    for (const char* name : {"ADHIP_GROUP_DOTS", "ADHIP_LAYER_KERNELS", "ADHIP_MERGE_SMALL", "ADHIP_FUSE_ATTENTION", "ADHIP_ROW_CHAINS",
+    for (const char* name : {"ADHIP_GROUP_DOTS", "ADHIP_LAYER_KERNELS", "ADHIP_MERGE_SMALL", "ADHIP_SHARE_INDEPENDENT", "ADHIP_FUSE_ATTENTION", "ADHIP_ROW_CHAINS",
                              "ADHIP_TIGHTEN", "ADHIP_KERNEL_BOUNDS", "ADHIP_DOT_PLAN", "ADHIP_TILED_SHAPE", "ADHIP_GEMM_AHEAD", "ADHIP_GRAPHS"}) {
         const char* e = getenv(name);
         out += e ? e : "";
@@ -3984,6 +4235,7 @@ std::unique_ptr<Plan> lower_program(const Proc& prog, const std::vector<std::str
     if (const char* e = getenv("ADHIP_GROUP_DOTS")) opt.group_dots = opt.group_dots && atoi(e) != 0;
     if (const char* e = getenv("ADHIP_LAYER_KERNELS")) opt.layer_kernels = opt.layer_kernels && atoi(e) != 0;
     if (const char* e = getenv("ADHIP_MERGE_SMALL")) opt.merge_small = opt.merge_small && atoi(e) != 0;
+    if (const char* e = getenv("ADHIP_SHARE_INDEPENDENT")) opt.share_independent = opt.share_independent && atoi(e) != 0;
     if (const char* e = getenv("ADHIP_FUSE_ATTENTION")) opt.fuse_attention = opt.fuse_attention && atoi(e) != 0;
     if (const char* e = getenv("ADHIP_ROW_CHAINS")) opt.row_chains = opt.row_chains && atoi(e) != 0;
     // diagnostic: every region lowered the way a region is after that many kernels of it spilled vector registers
@@ -4000,8 +4252,26 @@ std::unique_ptr<Plan> lower_program(const Proc& prog, const std::vector<std::str
             e = *end == ',' ? end + 1 : end;
         }
     }
-    Lowerer l(prog, dep_ids, opt);
-    return l.run();
+    Lowerer first(prog, dep_ids, opt);
+    std::unique_ptr<Plan> plan = first.run();
+    // Launches that share one run at the same time, and so do not share memory: where that alone keeps a program out of the
+    // static scratch area, they stay apart.
+    constexpr size_t area = ADHIP_STATIC_SCRATCH_BYTES;
+    if (plan->temp_bytes() > area && std::min(first.apart_bytes, first.packed_bytes) <= area) {
+        opt.share_independent = false;
+        opt.pack_slots = first.apart_bytes > area;
+        plan = Lowerer(prog, dep_ids, opt).run();
+    }
+    return plan;
+}
+
+size_t Plan::temp_bytes(std::vector<size_t>* offsets) const {
+    size_t need = 0;
+    for (int64_t elems : slot_elems) {
+        if (offsets) offsets->push_back(need);
+        need += (((size_t)std::max<int64_t>(elems, 1) * sizeof(float)) + 255) & ~size_t(255);
+    }
+    return need + ((((size_t)n_flags * sizeof(int)) + 255) & ~size_t(255));
 }
 
 }  // namespace adhip

@@ -18,6 +18,8 @@ struct LowerOptions {
     bool group_dots = true;  // same-shape independent matrix products share a launch
     bool layer_kernels = true;  // groups that run the same generated kernels on other buffers share their launches
     bool merge_small = true;    // consecutive single-block launches of a region run as phases of one launch
+    bool share_independent = true;  // small launches of a region that do not depend on one another run as one
+    bool pack_slots = false;        // a temporary takes any free slot that fits, however large
     bool fuse_attention = true;  // dot(softmax(scale * dot(Q, K^T)), V) runs as one kernel
     bool row_chains = true;      // row reductions and the element-wise values between them run as one kernel per row
     // Bounds on the size of one generated kernel, in what drives its register pressure: the places it loads from
@@ -34,6 +36,7 @@ struct LowerOptions {
     // there.  A region at shift >= 1 also takes no fused epilogues and no sums riding along.  The runtime raises the
     // shift of a region whose kernel the compiler could only build by spilling vector registers, and lowers again.
     std::map<int, int> region_shift;
+    std::set<int> unshared_regions;  // regions whose small launches stay apart: a kernel that held several of them spilled
     int min_shift = 0;              // diagnostic (ADHIP_TIGHTEN): every region is lowered at this shift at least
 };
 

@@ -22,6 +22,8 @@ struct KernelDef {
     std::string entry;   // symbol name
     std::string source;  // complete HIP C++ translation unit
     std::string kind;    // "elw", "reduce_row", "reduce_col", "dot", ...
+    size_t shared_bytes = 0;  // LDS of a product kernel (its one array `lds`), 0 for all others
+    bool part_only = false;  // only parts of shared launches refer to it: it is described, but never compiled
     std::vector<int> regions;  // the straight-line regions (in lowering order) whose launches use it
 };
 
@@ -43,6 +45,7 @@ struct Launch {
     std::string label;
     double bytes = 0, flops = 0;  // algorithmic work of one launch
     int stat = -1;                // index into Plan::stats
+    std::vector<Launch> parts;    // a shared launch: the launches it does the work of, in the order of the program
 };
 
 struct Step {
@@ -95,6 +98,8 @@ struct Plan {
     std::vector<int64_t> slot_elems;            // physical temp slots
     int n_flags = 0;
     std::string describe() const;
+    // what its temporaries and flags take, every one at a multiple of 256 bytes (`offsets`: where each slot would begin)
+    size_t temp_bytes(std::vector<size_t>* offsets = nullptr) const;
 };
 
 }  // namespace adhip

@@ -433,14 +433,16 @@ template <class Have>
 std::unique_ptr<Plan> lower_and_compile(const Proc& ir, const std::vector<std::string>& deps, const std::string& arch, Have&& have,
                                         std::map<std::string, std::vector<char>>& objects, int* relowered = nullptr) {
     LowerOptions opt;
+    int tightened = 0;
     for (int attempt = 0;; ++attempt) {
         std::unique_ptr<Plan> plan = lower_program(ir, deps, opt);
         std::vector<std::string> missing;
         for (const KernelDef& k : plan->kernels)
-            if (!objects.count(k.source) && !have(k.source)) missing.push_back(k.source);
+            if (!k.part_only && !objects.count(k.source) && !have(k.source)) missing.push_back(k.source);
         for (auto& kv : compile_code_objects(missing, arch)) objects[kv.first] = std::move(kv.second);
         std::set<int> regions;
         std::string report;
+        bool tighter = false;
         for (const KernelDef& k : plan->kernels) {
             auto it = objects.find(k.source);
             if (it == objects.end()) continue;  // loaded before, so accepted before
@@ -449,19 +451,20 @@ std::unique_ptr<Plan> lower_and_compile(const Proc& ir, const std::vector<std::s
                 report += strf("%s%s [%s] (%ld vector, %ld scalar registers spilled, %ld bytes of scratch per lane)", report.empty() ? "" : "; ",
                                ks.name.c_str(), k.kind.c_str(), ks.vector, ks.scalar, ks.scratch_bytes);
                 for (int r : k.regions)
-                    if (r >= 0) regions.insert(r);
+                    if (r >= 0 && k.kind == "shared") tighter = opt.unshared_regions.insert(r).second || tighter;
+                    else if (r >= 0) regions.insert(r);
             }
         }
         if (relowered) *relowered = attempt;
         if (report.empty()) return plan;
-        bool tighter = false;
         for (int r : regions) {
             int& sh = opt.region_shift[r];
             if (sh < 4) { ++sh; tighter = true; }
         }
-        ADHIP_CHECK(tighter && attempt < 4,
+        if (!regions.empty()) ++tightened;
+        ADHIP_CHECK(tighter && tightened <= 4,
                     "refusing to run kernels that spill vector registers to scratch memory (after %d lowerings with tighter bounds): %s",
-                    attempt, report.c_str());
+                    tightened - 1, report.c_str());
     }
 }
 
@@ -524,6 +527,7 @@ adhip_program* program_create(adhip_ctx* ctx, const uint8_t* program, size_t len
     Plan& plan = *p->plan;
     try {
         for (const KernelDef& k : plan.kernels) {
+            if (k.part_only) { p->fn.push_back(nullptr); continue; }
             auto f = fresh.find(k.source);
             auto m = compile_module(ctx, k.source, f != fresh.end() ? &f->second : nullptr);
             p->mods.push_back(m);
@@ -588,14 +592,9 @@ adhip_program* program_create(adhip_ctx* ctx, const uint8_t* program, size_t len
         }
         // where the temporaries and the flags would sit in the static scratch area (256-byte aligned slots)
         {
-            std::vector<size_t> slot_off(plan.slot_elems.size(), 0);
-            size_t need = 0;
-            for (size_t s = 0; s < plan.slot_elems.size(); ++s) {
-                slot_off[s] = need;
-                need += (((size_t)std::max<int64_t>(plan.slot_elems[s], 1) * sizeof(float)) + 255) & ~size_t(255);
-            }
-            const size_t flags_off = need;
-            need += (((size_t)plan.n_flags * sizeof(int)) + 255) & ~size_t(255);
+            std::vector<size_t> slot_off;
+            const size_t need = plan.temp_bytes(&slot_off);
+            const size_t flags_off = need - ((((size_t)plan.n_flags * sizeof(int)) + 255) & ~size_t(255));
             p->static_need = need;
             if (ctx->static_scratch && need <= (size_t)ADHIP_STATIC_SCRATCH_BYTES) {
                 p->static_buf_ptr = p->buf_ptr;
@@ -685,7 +684,7 @@ void launch(adhip_program* p, const Launch& l) {
     // argument block: guard pointer, then the plan's arguments; on the stack, so that a run allocates nothing on the
     // host either
     const void* guard = l.guard >= 0 ? (const void*)(cur_flags(p) + l.guard) : nullptr;
-    constexpr size_t kStackArgs = 192;  // merged launches take at most 160 arguments, shared ones 96 pointers
+    constexpr size_t kStackArgs = 384;  // merged launches take at most 160 arguments, shared ones 360
     void* ptrs[kStackArgs + 1];
     uint64_t vals[kStackArgs];
     ADHIP_CHECK(l.args.size() <= kStackArgs, "internal: launch '%s' takes %zu arguments", l.label.c_str(), l.args.size());
@@ -1248,7 +1247,10 @@ int adhip_compile_check(const uint8_t* program, size_t program_len, const char* 
         std::map<std::string, std::vector<char>> objects;
         int relowered = 0;
         auto plan = lower_and_compile(*ir, dep_vector(dep_ids, n_dep_ids), arch && *arch ? arch : "gfx950", [](const std::string&) { return false; }, objects, &relowered);
+        size_t compiled = 0;
         for (auto& k : plan->kernels) {
+            if (k.part_only) continue;
+            ++compiled;
             const std::vector<char>& code = objects[k.source];
             bytes += code.size();
             if (dump_dir && *dump_dir) {
@@ -1257,10 +1259,11 @@ int adhip_compile_check(const uint8_t* program, size_t program_len, const char* 
                 if (FILE* f = fopen((base + ".hip").c_str(), "wb")) { fwrite(k.source.data(), 1, k.source.size(), f); fclose(f); }
             }
         }
-        text = strf("%zu kernels compiled, %zu bytes of code objects", plan->kernels.size(), bytes);
+        text = strf("%zu kernels compiled, %zu bytes of code objects", compiled, bytes);
         if (relowered) text += strf("; lowered %d more times with tighter kernel bounds", relowered);
         std::string spills;
         for (auto& k : plan->kernels) {
+            if (k.part_only) continue;
             const std::string one = describe_spills(objects[k.source], true);
             if (!one.empty()) spills += (spills.empty() ? "" : "; ") + one;
         }

@@ -1,0 +1,108 @@
+"""Launches of a region that do not depend on one another run as one: what shares, what never does, values under the
+oracle, replays, the static scratch area."""
+import re
+
+import numpy as np
+import pytest
+
+from adhip import ir as IR, workloads as W
+from adhip.device import lower_describe
+from oracle.interp import OracleDevice
+
+
+def _plan(build):
+    proc, deps = build(OracleDevice()).finish()
+    return lower_describe(proc, deps)
+
+
+def _mlp(dev, batch=64, dims=(32, 64, 48, 8), iters=3, seed=1):
+    return W.mlp_train(dev, batch, dims, iters, seed=seed)
+
+
+def _sets(text):
+    """The member launches of every shared launch, by label."""
+    sets, lines = [], text.splitlines()
+    for i, line in enumerate(lines):
+        m = re.match(r"\s*shared\d+_(\d+)x, one launch", line)
+        if m:
+            sets.append([re.match(r"\s*launch (\S+)", lines[i + 1 + j]).group(1) for j in range(int(m.group(1)))])
+    return sets
+
+
+def test_what_does_not_depend_shares_a_launch():
+    sets = _sets(_plan(_mlp))
+    assert sum(map(len, sets)) - len(sets) >= 8, sets   # 17 launches a step and at most nine left
+    # the gradient of a layer's input reads the weights that the layer's update overwrites: never together
+    for s in sets:
+        assert not ({"dot_cf_64x64x48", "dot_ch_64x48x64"} <= set(s) or {"dot_bm_64x48x8", "dot_bo_48x8x64"} <= set(s)), s
+
+
+def _args(text, label):
+    line = re.search(rf"^\s*launch {label} .*args:(.*)$", text, re.M).group(1)
+    return {int(b) for b in re.findall(r"#(\d+)", line)}
+
+
+@pytest.mark.parametrize("build", [_mlp, lambda d: W.encoder_train(d, 64, 32, 4, 64, 2, seed=3), lambda d: W.encoder_train(d, 50, 40, 5, 72, 2, seed=3)],
+                         ids=["perceptron", "encoder", "encoder-odd"])
+def test_members_share_no_memory_that_one_of_them_writes(build):
+    """Temporaries of launches that run at the same time have slots of their own (written ones: those whose slot another
+    member of the set names through another buffer, or names at all and writes)."""
+    text = _plan(build)
+    slot = {int(b): int(s) for b, s in re.findall(r"#(\d+) temp \S+ elems=\d+ slot=(\d+)", text)}
+    sets = _sets(text)
+    assert sets
+    for s in sets:
+        owner = {}
+        for label in s:
+            for b in _args(text, label):
+                if b in slot:
+                    assert owner.setdefault(slot[b], b) == b, (s, label, b)
+
+
+def test_large_launches_stay_apart():
+    text = _plan(lambda d: W.mlp_train(d, 4096, (4096, 4096, 4096, 1024), 2))
+    for s in _sets(text):
+        assert not any(label.startswith("dot") for label in s), s
+
+
+def test_switched_off(monkeypatch):
+    monkeypatch.setenv("ADHIP_SHARE_INDEPENDENT", "0")
+    assert not _sets(_plan(_mlp))
+
+
+@pytest.mark.parametrize("chains", [2, 20])
+def test_a_program_that_fits_the_static_scratch_area_still_fits(chains):
+    """What shares a launch shares no memory: chains of two products, 2 MB between them, of which 20 at a time would be more
+    than the area holds."""
+    cmds, keep = [], set()
+    for i in range(chains):
+        k = 64 + 4 * i   # no two of one shape: those would be one grouped launch
+        cmds += [IR.CreateMat(np.zeros(1000 * k, np.float32), [1000, k], f"x{i}"), IR.CreateMat(np.zeros(k * 512, np.float32), [k, 512], f"v{i}"),
+                 IR.CreateMat(np.zeros(512 * (8 + i), np.float32), [512, 8 + i], f"w{i}"),
+                 IR.DotProduct(a=f"x{i}", b=f"v{i}", res=f"h{i}"), IR.DotProduct(a=f"h{i}", b=f"w{i}", res=f"y{i}")]
+        keep.add(f"y{i}")
+    text = lower_describe(IR.IRProcedure("main", cmds + [IR.EX()]), keep)
+    assert bool(_sets(text)) == (chains == 2), text
+
+
+# ---- on the GPU
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("build", [_mlp, lambda d: _mlp(d, 100, (70, 90, 65, 10), 4), lambda d: _mlp(d, 300, (200, 330, 129, 7), 4),
+                                   lambda d: W.encoder_train(d, 64, 32, 4, 64, 4, seed=3), lambda d: W.encoder_train(d, 130, 80, 5, 200, 4, seed=4)],
+                         ids=["perceptron", "perceptron-odd", "perceptron-products", "encoder", "encoder-products"])
+def test_shared_launches_match_launches_apart(build, hip_device, monkeypatch):
+    """The same kernels, so the same bits, at the first pass (launched one by one) and at replays."""
+    print("[case] shared launches", flush=True)
+    def values(share):
+        monkeypatch.setenv("ADHIP_SHARE_INDEPENDENT", share)
+        out = []
+        for _ in range(3):
+            wl = build(hip_device)
+            out.append({k: np.asarray(v.data, dtype=np.float32) for k, v in wl.run().items()})
+        return out
+    apart, shared = values("0"), values("1")
+    for a, s in zip(apart, shared):
+        for k in a:
+            assert np.array_equal(a[k].view(np.uint32), s[k].view(np.uint32)), k
