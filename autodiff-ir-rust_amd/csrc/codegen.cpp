@@ -749,10 +749,12 @@ ElwBody elw_body(const ElwKernelSpec& spec, const std::set<const Node*>& members
 // three of: results stored, full-size operands read), where a block's closing steps (the sums across the wavefront,
 // the 16 rows through LDS) weigh more against its streaming: two rows per wavefront then, if that still leaves eight
 // blocks per CU.  Measured on 16384 x 4096 with one operand, one result, row and column sums: 103 -> 96 us a step
-// (three and four rows: 98 and 100); on the 3-read + 4-write pass over 8192 x 8192 two rows per wavefront cost 1.5 %
+// (three and four rows: 98 and 100; a pass that stores nothing but its sums takes four, as the stand-alone column sums do);
+// on the 3-read + 4-write pass over 8192 x 8192 two rows per wavefront cost 1.5 %
 // instead.
 static int64_t elw_colsum_rows_per_wave(int64_t rows, int64_t cols, int streams) {
     const int64_t base = std::max<int64_t>(1, (rows + 16 * 1024 - 1) / (16 * 1024));
+    if (base == 1 && streams <= 1 && ((cols / 4 + 63) / 64) * ((rows + 63) / 64) >= 2048) return 4;
     if (base == 1 && streams <= 3 && ((cols / 4 + 63) / 64) * ((rows + 31) / 32) >= 2048) return 2;
     return base;
 }
