@@ -20,19 +20,109 @@
 // With D % 16 == 0 the contraction index of the scores is spread over the lanes in runs of four (in step (S, u) lane
 // group lq supplies element 16 S + 4 lq + u), so a lane's operands for four consecutive steps are one 128-bit LDS
 // read; the weighted values use the same spreading over the keys of a tile.
+//
+// On the bf16 matrix cores (`parts`: heads of 32 to 128 features without a mask, at least 32 keys): every FP32 operand as three
+// bf16 parts, as in gemm_split.cpp, with keys and values split and put into the order of the lanes by a kernel of its own before.
+// A wavefront owns all 64 query rows and every eighth tile of 32 keys, with its own running maxima, sums and accumulators, so
+// that nothing is shared and no barrier stands in the loop; the eight are merged at the end.  It multiplies keys by query
+// rows and values by probabilities, so that a row of the softmax is a lane: its maximum takes one exchange between the
+// lane's halves, its rescaling none, and the probabilities stand in the registers in which the second product wants them.  What
+// does not come out finite -- operands from 2^111 on, infinities, NaN -- is computed again by the kernel described above.
+// 8 heads of 2048 x 2048 x 128: 182 us -> 94 and 8 for the split; the matrix instructions take 50, the merging and the first
+// trips to memory some 15, and what comes from L2 (0.8 GB) the rest: with 32 query rows a wavefront, twice of that, 98.  With keys and
+// values split in the kernel itself, once per row block, it was bound by vector instructions (127 us).  8 heads of 1001 x 1001 x 64:
+// 51 -> 24 + 5.  Errors against 64 bits 7.3e-7 -> 5.5e-7 and 4.9e-7 -> 2.4e-7 of a whole attention layer.
 #include "attention.hpp"
 
+#include <algorithm>
+
 #include "common.hpp"
+#include "gemm.hpp"
 
 namespace adhip {
 
 size_t attention_lds_bytes(const AttentionConfig& cfg) {
     const size_t stage = (size_t)cfg.bn * (size_t)(cfg.d + 4 + cfg.dv + 4);
     const size_t patches = (size_t)4 * cfg.wg * 16 * (size_t)(cfg.bn / cfg.wg + 4);
-    return 4 * (2 * stage + patches);
+    const size_t f32 = 4 * (2 * stage + patches);
+    if (!cfg.parts) return f32;
+    const size_t loop = (size_t)64 * cfg.d * 6, merge = (size_t)4 * 64 * (cfg.dv + 4) * 4;
+    return std::max({f32, loop, merge});
+}
+
+// 128-bit words of a tile of 32 keys in parts: 16 features of the keys, then 16 keys of the values, 64 lanes and three parts each
+static int tile_words(const AttentionConfig& cfg) { return 64 * 3 * (cfg.d / 16 + 2 * (cfg.dv / 32)); }
+int64_t attention_parts_floats(const AttentionConfig& cfg, int64_t sk) { return (sk + 31) / 32 * tile_words(cfg) * 4; }
+
+// K and V of every problem in parts, in the order in which the attention kernel's lanes take them: a block does one tile of one
+// problem, its wavefronts take turns.  Every row block of a problem would split them again otherwise: 13 vector instructions
+// a pair of numbers, 830 of 1180 of a tile, and at five cycles each these, not the matrix instructions, bound the kernel (8 heads
+// of 2048 x 2048 x 128: 127 us; 60 and 9 for this pass).
+std::string attention_split_source(const AttentionConfig& cfg, const std::string& entry) {
+    std::string params, pick;
+    for (int i = 0; i < kAttentionSlots; ++i) {
+        params += strf("const float* k%d, const float* v%d, ", i, i);
+        pick += strf("    case %d: K = k%d; V = v%d; break;\n", i, i, i);
+    }
+    return strf("#define D %d\n#define DV %d\n#define WORDS %d\n#define EDGE 1\n#define NB (DV / 32)\n#define SCALE 65536.0f\n", cfg.d, cfg.dv, tile_words(cfg)) +
+           split_types() + "extern \"C\" __global__ __launch_bounds__(256) void " + entry + "(const int* __restrict__ guard, " + params +
+           "float* parts, long long Sk, long long k_ld, long long v_ld) {\n    if (guard && *guard == 0) return;\n    const float* __restrict__ K;\n"
+           "    const float* __restrict__ V;\n    switch (blockIdx.y) {\n" + pick + "    default: return;\n    }\n" + R"(
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, li = lane & 31u, lh = lane >> 5;
+    const long long kb = min(32ll * blockIdx.x, Sk - 32);
+    uint4_t* to = (uint4_t*)parts + ((long long)blockIdx.y * ((Sk + 31) / 32) + blockIdx.x) * WORDS + lane;
+    auto store8 = [&](const float (&x)[8], int unit) {
+        uint4_t p0, p1, p2;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            unsigned u0, u1, u2;
+            split(x[2 * q], x[2 * q + 1], SCALE, u0, u1, u2);
+            p0[q] = u0;
+            p1[q] = u1;
+            p2[q] = u2;
+        }
+        to[(3 * unit + 0) * 64] = p0;
+        to[(3 * unit + 1) * 64] = p1;
+        to[(3 * unit + 2) * 64] = p2;
+    };
+    for (unsigned u = wave; u < D / 16 + 2; u += 4) {
+        if (u < D / 16) {
+            // key li, features 16 u + 8 lh ..
+            const float* from = K + (kb + li) * k_ld + 16 * u + 8 * lh;
+            float x[8];
+            *(float4_t*)&x[0] = *(const float4_t*)from;
+            *(float4_t*)&x[4] = *(const float4_t*)(from + 4);
+            store8(x, u);
+        } else {
+            // features NB li + i of keys 16 s + 8 (q / 4) + 4 lh + q % 4
+            const unsigned s = u - D / 16;
+            float v[8][NB];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const float* from = V + (kb + 16 * s + 8 * (q >> 2) + 4 * lh + (q & 3)) * v_ld + NB * li;
+#if NB == 4
+                *(float4_t*)v[q] = *(const float4_t*)from;
+#elif NB == 2
+                *(float2_t*)v[q] = *(const float2_t*)from;
+#else
+                v[q][0] = *from;
+#endif
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                float x[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) x[q] = v[q][i];
+                store8(x, D / 16 + s * NB + i);
+            }
+        }
+    }
+}
+)";
 }
 
 std::string attention_kernel_source(const AttentionConfig& cfg, const std::string& entry) {
+    ADHIP_CHECK(!cfg.parts || (!cfg.mask && cfg.wg == 2 && attention_takes_parts(cfg.d, cfg.dv)), "internal: attention of these widths in bf16 parts");
     std::string s;
     std::string params, pick = "switch (problem) {";
     for (int i = 0; i < kAttentionSlots; ++i) {
@@ -41,10 +131,13 @@ std::string attention_kernel_source(const AttentionConfig& cfg, const std::strin
         pick += strf(" case %d: O = o%d; Q = q%d; K = k%d; V = v%d;%s break;", i, i, i, i, i, cfg.mask ? strf(" Mk = m%d;", i).c_str() : "");
     }
     s += "#define GROUP_PARAMS " + params + "\n#define GROUP_PICK " + pick + " default: return; }\n";
-    s += strf("#define KERNEL_NAME %s\n#define D %d\n#define DV %d\n#define BN %d\n#define WG %d\n#define MASK %d\n", entry.c_str(), cfg.d, cfg.dv, cfg.bn,
-              cfg.wg, cfg.mask ? 1 : 0);
+    s += strf("#define KERNEL_NAME %s\n#define D %d\n#define DV %d\n#define BN %d\n#define WG %d\n#define MASK %d\n#define PARTS %d\n#define LDS_FLOATS %zu\n#define WORDS %d\n", entry.c_str(), cfg.d, cfg.dv, cfg.bn,
+              cfg.wg, cfg.mask ? 1 : 0, cfg.parts ? 1 : 0, attention_lds_bytes(cfg) / 4, cfg.parts ? tile_words(cfg) : 0);
+    s += cfg.parts ? "#define PARTS_POINTER const float* __restrict__ parts,\n" : "#define PARTS_POINTER\n";
     s += cfg.mask ? "#define MASK_LD long long m_ld,\n" : "#define MASK_LD\n";
-    s += "typedef float float4_t __attribute__((ext_vector_type(4)));\n";
+    if (cfg.parts) s += "#define EDGE 1\n" + split_types();
+    else
+        s += "typedef float float4_t __attribute__((ext_vector_type(4)));\n";
     s += R"ATTN(
 #define NT (256 * WG)
 #define BNW (BN / WG)
@@ -72,7 +165,7 @@ static __device__ __forceinline__ float row16_sum(float x) {
 }
 
 extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
-    const int* __restrict__ guard, GROUP_PARAMS long long Sq, long long Sk, long long q_ld, long long k_ld, long long v_ld,
+    const int* __restrict__ guard, GROUP_PARAMS PARTS_POINTER long long Sq, long long Sk, long long q_ld, long long k_ld, long long v_ld,
     MASK_LD float scale, int row_blocks, int problems) {
     if (guard && *guard == 0) return;
     // Blocks are handed to the eight XCDs in turn; renumbering them so that an XCD's blocks are consecutive puts the row
@@ -91,12 +184,250 @@ extern "C" __global__ __launch_bounds__(NT) void KERNEL_NAME(
     const float* __restrict__ Mk;
 #endif
     GROUP_PICK
-    __shared__ __attribute__((aligned(16))) float lds[2 * STAGE + 4 * WG * 16 * PLD];
-    float (*Ps)[16][PLD] = (float (*)[16][PLD])(lds + 2 * STAGE);
+    __shared__ __attribute__((aligned(16))) float lds[LDS_FLOATS];
+    const float LOG2E = 1.44269502162933349609375f;  // the float nearest 1 / ln 2
     const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+#if PARTS
+#define SCALE 65536.0f
+#define NB (DV / 32)                    /* blocks of 32 features of the result */
+    {
+        __shared__ int failed;
+        const unsigned li = lane & 31u, lh = lane >> 5, kg = __builtin_amdgcn_readfirstlane(wave);
+        const long long row0 = (long long)row_block * 64;
+        // the block's query rows in parts: [part][eight features][row]
+        uint4_t* Qs = (uint4_t*)lds;
+#pragma unroll
+        for (unsigned u0 = 0; u0 < 64 * D / 8; u0 += NT) {
+            const unsigned u = u0 + tid, row = u / (D / 8), d8 = u % (D / 8);
+            if (64 * D / 8 % NT == 0 || u < 64 * D / 8) {
+                const float* from = Q + min(row0 + (long long)row, Sq - 1) * q_ld + 8 * d8;
+                float x[8];
+                *(float4_t*)&x[0] = *(const float4_t*)from;
+                *(float4_t*)&x[4] = *(const float4_t*)(from + 4);
+                uint4_t p0, p1, p2;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    unsigned u0, u1, u2;
+                    split(x[2 * q], x[2 * q + 1], SCALE, u0, u1, u2);
+                    p0[q] = u0;
+                    p1[q] = u1;
+                    p2[q] = u2;
+                }
+                Qs[(0 * (D / 8) + d8) * 64 + row] = p0;
+                Qs[(1 * (D / 8) + d8) * 64 + row] = p1;
+                Qs[(2 * (D / 8) + d8) * 64 + row] = p2;
+            }
+        }
+        // Keys and values come in parts and in the order of the lanes (see the kernel that splits them): a unit is what six
+        // matrix instructions take of them, first 16 features of the 32 keys at a time, then 16 keys of 32 features of the values
+        // at a time.  Two to four units are on their way; behind its last tile a wavefront fetches the last unit once more.
+#define UNITS (D / 16 + 2 * NB)
+#define RING (NB == 4 ? 2 : UNITS % 4 == 0 ? 4 : UNITS % 3 == 0 ? 3 : 2)
+        const uint4_t* from = (const uint4_t*)parts + (long long)problem * ((Sk + 31) / 32) * WORDS;
+        const unsigned lane_at = 16u * lane;
+        uint4_t ring[RING][3];
+        auto fetch = [&](long long t, int unit) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p) ring[unit % RING][p] = *(const uint4_t*)((const char*)(from + t * WORDS + (3 * unit + p) * 64) + lane_at);
+        };
+        auto split8 = [&](const float (&x)[8], float scale, bf16x8_t (&p)[3]) {
+            uint4_t a, b, c;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                unsigned u0, u1, u2;
+                split(x[2 * q], x[2 * q + 1], scale, u0, u1, u2);
+                a[q] = u0;
+                b[q] = u1;
+                c[q] = u2;
+            }
+            p[0] = __builtin_bit_cast(bf16x8_t, a);
+            p[1] = __builtin_bit_cast(bf16x8_t, b);
+            p[2] = __builtin_bit_cast(bf16x8_t, c);
+        };
+        // of the nine products of parts the six that reach the result's 24 bits, the smallest first
+#define TERM(acc, x, y)                                                                                                  \
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y[0], acc[0], 0, 0, 0);                                     \
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y[1], acc[1], 0, 0, 0);
+#define SIX(acc, x, y)                                                                                                   \
+        TERM(acc, x[2], y[0]) TERM(acc, x[0], y[2]) TERM(acc, x[1], y[1]) TERM(acc, x[1], y[0]) TERM(acc, x[0], y[1]) TERM(acc, x[0], y[0])
+        float16_t o[NB][2];   // o[i][j][4 g + r]: feature NB (8 g + 4 lh + r) + i of query row 32 j + li
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[i][0][r] = o[i][1][r] = 0.0f;
+        float m[2] = {-__builtin_inff(), -__builtin_inff()}, l[2] = {0.0f, 0.0f};   // of query row 32 j + li; the sum over this half's keys
+        const float unscale = scale * (1.0f / SCALE / SCALE);
+        // the matrix cores lose a little towards minus infinity: every other key group weighs with the other sign
+        const float p_scale = kg & 1u ? -SCALE : SCALE;
+        const long long tiles = (Sk + 31) / 32;
+        if (kg < tiles) {
+#pragma unroll
+            for (int u = 0; u < RING; ++u) fetch(kg, u);
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (long long t = kg; t < tiles; t += 8) {
+            const long long t_next = t + 8 < tiles ? t + 8 : t;
+            bf16x8_t f[3];
+            auto next = [&](int unit) {   // takes a unit and asks for the one that will stand in its place
+#pragma unroll
+                for (int p = 0; p < 3; ++p) f[p] = __builtin_bit_cast(bf16x8_t, ring[unit % RING][p]);
+                if (unit + RING < UNITS) fetch(t, unit + RING);
+                else fetch(t_next, unit + RING - UNITS);
+            };
+            // scores, keys by query rows
+            float16_t sc[2];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[0][r] = sc[1][r] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < D / 16; ++u) {
+                bf16x8_t qf[3][2];
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) qf[p][j] = __builtin_bit_cast(bf16x8_t, Qs[(p * (D / 8) + 2 * u + lh) * 64 + 32 * j + li]);
+                next(u);
+                SIX(sc, f, qf)
+                __builtin_amdgcn_sched_barrier(0);   // (operands of later units taken from LDS now are registers that a wide head lacks)
+            }
+            if (32 * t + 32 > Sk) {   // the last tile begins earlier, with keys that the tile before has
+                const int had = (int)(32 * t + 32 - Sk);
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (8 * (r >> 2) + 4 * (int)lh + (r & 3) < had) sc[0][r] = sc[1][r] = -__builtin_inff();
+            }
+            float m_new[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                float mx = -__builtin_inff();
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    sc[j][r] *= unscale;
+                    mx = fmaxf(mx, sc[j][r]);
+                }
+                m_new[j] = fmaxf(m[j], fmaxf(mx, __shfl_xor(mx, 32)));
+            }
+            if (__builtin_amdgcn_ballot_w64(m_new[0] != m[0] || m_new[1] != m[1]) != 0ull) {
+                // some row's maximum grew: what has been accumulated against the old maximum is rescaled
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const float alpha = __builtin_amdgcn_exp2f((m[j] - m_new[j]) * LOG2E);
+                    l[j] *= alpha;
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o[i][j][r] *= alpha;
+                    m[j] = m_new[j];
+                }
+            }
+            // probabilities stand as the second product wants them: a lane's keys are its keys again
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                bf16x8_t pf[3][2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    float p[8];
+                    bf16x8_t parts_of_p[3];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        p[q] = __builtin_amdgcn_exp2f((sc[j][4 * (2 * s + (q >> 2)) + (q & 3)] - m[j]) * LOG2E);
+                        l[j] += p[q];
+                    }
+                    split8(p, p_scale, parts_of_p);
+#pragma unroll
+                    for (int x = 0; x < 3; ++x) pf[x][j] = parts_of_p[x];
+                }
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    next(D / 16 + s * NB + i);
+                    SIX(o[i], f, pf)
+                }
+            }
+        }
+        // half of the key groups hand theirs to the other half, three times
+#pragma unroll
+        for (int half = 4; half >= 1; half >>= 1) {
+            __syncthreads();
+            float* mg = lds + (kg & (half - 1)) * 64 * (32 * NB + 4) + lane * (32 * NB + 4);
+            if ((int)kg >= half && (int)kg < 2 * half) {
+                *(float4_t*)mg = float4_t{m[0], m[1], l[0], l[1]};
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g)
+                            *(float4_t*)(mg + 4 + 32 * i + 16 * j + 4 * g) = float4_t{o[i][j][4 * g], o[i][j][4 * g + 1], o[i][j][4 * g + 2], o[i][j][4 * g + 3]};
+            }
+            __syncthreads();
+            if ((int)kg < half) {
+                const float4_t theirs = *(const float4_t*)mg;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    // (a group without keys has -inf and zeros; one in front of a group with keys has keys)
+                    const float top = fmaxf(m[j], theirs[j]);
+                    const float e0 = m[j] == top ? 1.0f : __builtin_amdgcn_exp2f((m[j] - top) * LOG2E);
+                    const float e1 = theirs[j] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((theirs[j] - top) * LOG2E);
+                    // groups of odd number have the other sign: all of the first round's pairs agree, and so do the second's
+                    const float es = half == 1 ? -e1 : e1;
+                    l[j] = l[j] * e0 + theirs[2 + j] * e1;
+                    m[j] = top;
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const float4_t v = *(const float4_t*)(mg + 4 + 32 * i + 16 * j + 4 * g);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) o[i][j][4 * g + r] = o[i][j][4 * g + r] * e0 + v[r] * es;
+                        }
+                }
+            }
+        }
+        if (kg == 0) {
+            unsigned largest = 0u;
+            float inv[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                l[j] += __shfl_xor(l[j], 32);
+                inv[j] = (1.0f / l[j]) * (1.0f / SCALE / SCALE);
+                largest = max(largest, __builtin_bit_cast(unsigned, l[j]) & 0x7fffffffu);
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const float x = o[i][j][r];
+                        largest = max(largest, __builtin_bit_cast(unsigned, x) & 0x7fffffffu);
+                    }
+            }
+            const bool bad = __builtin_amdgcn_ballot_w64(largest >= 0x7f800000u) != 0ull;
+            if (lane == 0) failed = bad;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const long long row = row0 + 32 * j + li;
+                if (!bad && row < Sq) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            float* to = O + row * DV + NB * (8 * g + 4 * lh + r);
+#if NB == 4
+                            *(float4_t*)to = float4_t{o[0][j][4 * g + r], o[1][j][4 * g + r], o[NB - 2][j][4 * g + r], o[NB - 1][j][4 * g + r]} * inv[j];
+#else
+#pragma unroll
+                            for (int i = 0; i < NB; ++i) to[i] = o[i][j][4 * g + r] * inv[j];
+#endif
+                        }
+                }
+            }
+        }
+        __syncthreads();
+        if (!failed) return;
+        __syncthreads();
+    }
+#endif
+    float (*Ps)[16][PLD] = (float (*)[16][PLD])(lds + 2 * STAGE);
     const unsigned li = lane & 15u, lq = lane >> 4, rw = wave & 3u, kg = wave >> 2;
     const long long row_base = (long long)row_block * 64 + rw * 16;
-    const float LOG2E = 1.44269502162933349609375f;  // the float nearest 1 / ln 2
 
     // this lane's part of the wavefront's 16 query rows
 #if D % 16 == 0

@@ -626,6 +626,7 @@ struct Lowerer {
     // on top: a program whose temporaries fit the static scratch area in one of these ways is lowered that way (lower_program).
     SlotPool pool, pool_apart, pool_packed;
     size_t apart_bytes = 0, packed_bytes = 0;
+    bool has_parts = false;   // keys and values of an attention kernel are kept in parts
     // A temporary of the region being lowered; what memory it takes is decided when the region's launches stand
     // (assign_slots), so that two launches only share memory, and depend on one another for it, if they run one after the other.
     int alloc_temp(int64_t elems, const std::string& name) {
@@ -2853,6 +2854,17 @@ struct Lowerer {
                         gks[g].dot_store = needed;
                     }
                 }
+            } else if (G.kind == Group::ATTN) {
+                AttentionKey key;
+                Affine2D q, kt, v;
+                ADHIP_CHECK(attention_key(G.members[0], key, q, kt, v), "internal: attention node whose operands the kernel cannot read");
+                const AttentionConfig cfg = attention_config(key, (int64_t)G.members.size());
+                if (cfg.parts) {
+                    Node* parts = new_node(Op::COPY, Shape{(int64_t)G.members.size() * attention_parts_floats(cfg, key.sk)}, {}, G.members[0]->name + ".parts", 0.f, false);
+                    parts->root = true;
+                    gks[g].extra_nodes.push_back(parts);
+                    has_parts = true;
+                }
             } else if (G.kind == Group::ROWCHAIN) {
                 // a member is written to memory only if an id holds it or a kernel outside the chain reads it
                 RowChainSpec spec;
@@ -3161,7 +3173,7 @@ struct Lowerer {
                 continue;
             }
             if (G.kind == Group::ATTN) {
-                emit_attention(G.members, out);
+                emit_attention(G.members, out, gks[g].extra_nodes.empty() ? nullptr : gks[g].extra_nodes[0]);
                 continue;
             }
             GeneratedKernel& k = gks[g].k;
@@ -3565,27 +3577,36 @@ struct Lowerer {
         }
     }
 
-    // One launch of the fused attention kernel for up to 16 problems of one shape (block row y works on problem y).
-    void emit_attention(const std::vector<Node*>& atts, std::vector<Step>& out) {
+    AttentionConfig attention_config(const AttentionKey& key, int64_t cnt) const {
+        AttentionConfig cfg;
+        cfg.d = (int)key.d;
+        cfg.dv = (int)key.dv;
+        cfg.mask = key.m_ld > 0;
+        cfg.parts = opt.attention_parts && !cfg.mask && key.sk >= 32 && attention_takes_parts(cfg.d, cfg.dv);
+        // On the FP32 matrix cores a launch with two or more blocks per CU runs blocks of four wavefronts on tiles of 32 keys,
+        // two of which fit a CU's LDS while the heads are not too wide; a smaller launch splits every tile between two groups
+        // of four wavefronts instead, so that a SIMD still has two wavefronts to switch between.  Tiles of 64 keys where two
+        // stages of them fit in LDS.
+        const bool narrow = cfg.d + cfg.dv <= 256;
+        if ((key.sq + 63) / 64 * cnt >= 512 && narrow && !cfg.parts) { cfg.bn = 32; cfg.wg = 1; }
+        else { cfg.bn = narrow ? 64 : 32; cfg.wg = 2; }
+        return cfg;
+    }
+
+    // One launch of the fused attention kernel for up to 16 problems of one shape (block row y works on problem y), behind
+    // one that writes their keys and values in parts (`parts`) where the kernel takes them so.
+    void emit_attention(const std::vector<Node*>& atts, std::vector<Step>& out, Node* parts) {
         const int cnt = (int)atts.size();
         ADHIP_CHECK(cnt >= 1 && cnt <= kAttentionSlots, "internal: attention launch of %d problems", cnt);
         AttentionKey key0;
         Affine2D q0, k0, v0;
         ADHIP_CHECK(attention_key(atts[0], key0, q0, k0, v0), "internal: attention node whose operands the kernel cannot read");
-        AttentionConfig cfg;
-        cfg.d = (int)key0.d;
-        cfg.dv = (int)key0.dv;
-        cfg.mask = key0.m_ld > 0;
+        const AttentionConfig cfg = attention_config(key0, cnt);
         const int64_t row_blocks = (key0.sq + 63) / 64;
-        // A launch with two or more blocks per CU runs blocks of four wavefronts on tiles of 32 keys, two of which fit
-        // a CU's LDS while the heads are not too wide; a smaller launch splits every tile between two groups of four
-        // wavefronts instead, so that a SIMD still has two wavefronts to switch between.  Tiles of 64 keys where two
-        // stages of them fit in LDS.
-        const bool narrow = cfg.d + cfg.dv <= 256;
-        if (row_blocks * cnt >= 512 && narrow) { cfg.bn = 32; cfg.wg = 1; }
-        else { cfg.bn = narrow ? 64 : 32; cfg.wg = 2; }
         ADHIP_CHECK(attention_lds_bytes(cfg) <= 160 * 1024, "internal: attention tiles of %d keys do not fit in LDS", cfg.bn);
-        const std::string entry = strf("adhip_attention_d%d_v%d_k%d_w%d%s", cfg.d, cfg.dv, cfg.bn, cfg.wg, cfg.mask ? "_mask" : "");
+        ADHIP_CHECK(cfg.parts == (parts != nullptr) && (!parts || numel(parts->shape) == cnt * attention_parts_floats(cfg, key0.sk)),
+                    "internal: attention and its keys and values in parts disagree");
+        const std::string entry = strf("adhip_attention_d%d_v%d_k%d_w%d%s%s", cfg.d, cfg.dv, cfg.bn, cfg.wg, cfg.mask ? "_mask" : "", cfg.parts ? "_parts" : "");
         Launch l;
         l.kernel = add_kernel(entry, attention_kernel_source(cfg, entry), "attention");
         l.block[0] = 256u * (unsigned)cfg.wg;
@@ -3610,6 +3631,24 @@ struct Lowerer {
             l.args.push_back(B(kt.base, kt.offset));
             l.args.push_back(B(v.base, v.offset));
             if (cfg.mask) l.args.push_back(B(mk.base, mk.offset));
+        }
+        if (parts) {
+            const std::string split = strf("adhip_attention_split_d%d_v%d", cfg.d, cfg.dv);
+            Launch ls;
+            ls.kernel = add_kernel(split, attention_split_source(cfg, split), "attention_split");
+            ls.block[0] = 256;
+            ls.grid[0] = (unsigned)((key0.sk + 31) / 32);
+            ls.grid[1] = (unsigned)cnt;
+            for (int i = 0; i < kAttentionSlots; ++i) {
+                ls.args.push_back(l.args[(size_t)(4 * i + 2)]);
+                ls.args.push_back(l.args[(size_t)(4 * i + 3)]);
+            }
+            ls.args.push_back(B(parts, 0));
+            for (int64_t v : {key0.sk, key0.k_ld, key0.v_ld}) ls.args.push_back(I(v));
+            ls.label = strf("attention_split_%s_%dx", atts[0]->name.c_str(), cnt);
+            ls.bytes = 4.0 * cnt * (double)key0.sk * (double)(key0.d + key0.dv) + 4.0 * (double)numel(parts->shape);
+            push_launch(out, ls, "attention_split");
+            l.args.push_back(B(parts, 0));
         }
         for (int64_t v : {key0.sq, key0.sk, key0.q_ld, key0.k_ld, key0.v_ld}) l.args.push_back(I(v));
         if (cfg.mask) l.args.push_back(I(key0.m_ld));
@@ -4210,7 +4249,9 @@ struct Lowerer {
 };
 
 void describe_launch(const Launch& l, const Plan& p, const std::string& pad, std::string& o) {
-    o += pad + strf("launch %s [%s] kernel=%s grid=(%u,%u,%u) block=%u bytes=%.0f flops=%.0f args:", l.label.c_str(),
+    // (what only lays the next launch's operands out is not called a launch of the program's)
+    const char* what = p.kernels[l.kernel].kind == "attention_split" ? "lays out" : "launch";
+    o += pad + strf("%s %s [%s] kernel=%s grid=(%u,%u,%u) block=%u bytes=%.0f flops=%.0f args:", what, l.label.c_str(),
                     p.kernels[l.kernel].kind.c_str(), p.kernels[l.kernel].entry.c_str(), l.grid[0], l.grid[1], l.grid[2],
                     l.block[0], l.bytes, l.flops);
     for (const Arg& a : l.args) {
@@ -4314,6 +4355,12 @@ std::unique_ptr<Plan> lower_program(const Proc& prog, const std::vector<std::str
         opt.share_independent = false;
         opt.pack_slots = first.apart_bytes > area;
         plan = Lowerer(prog, dep_ids, opt).run();
+    } else if (plan->temp_bytes() > area && first.has_parts) {
+        // ... and so does attention without its keys and values in parts
+        opt.share_independent = opt.attention_parts = false;
+        opt.pack_slots = true;
+        std::unique_ptr<Plan> smaller = Lowerer(prog, dep_ids, opt).run();
+        if (smaller->temp_bytes() <= area) plan = std::move(smaller);
     }
     return plan;
 }

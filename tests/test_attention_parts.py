@@ -1,0 +1,105 @@
+"""Attention on the bf16 matrix cores: every width of heads it takes compiles without spilled registers, and values at the edges
+of its tiles of 32 keys, its eight key groups and its blocks of 64 rows, and where its parts cannot represent an operand."""
+import math
+
+import numpy as np
+import pytest
+
+from adhip import autodiff, nn
+from adhip.core import ValueData
+from adhip.device import Device, lower_describe
+from parity import RED_RTOL, assert_close
+
+WIDTHS = [(d, dv) for d in (32, 64, 96, 128) for dv in (32, 64, 128)]
+
+
+class Capture(Device):
+    def execute(self, proc, deps):
+        self.proc, self.deps = proc, list(deps)
+
+    def get_tensor(self, id):
+        return ValueData.none()
+
+
+def _program(dev, q, k, v, scale_dim):
+    autodiff.set_device(dev)
+    t = [autodiff.tensor(x.reshape(-1), list(x.shape)) for x in (q, k, v)]
+    o = nn.Attention(t[0], t[1], t[2], scale_dim)
+    o.forward()
+    o.val().keep()
+    autodiff.execute()
+    return o
+
+
+def _zeros(sq, sk, d, dv):
+    return [np.zeros(s, np.float32) for s in ((sq, d), (sk, d), (sk, dv))]
+
+
+@pytest.mark.parametrize("d,dv", WIDTHS)
+def test_every_width_compiles_without_spills(d, dv):
+    from test_library_cpu import _compile_check
+    dev = Capture()
+    _program(dev, *_zeros(100, 200, d, dv), 64)
+    text = lower_describe(dev.proc, dev.deps)
+    assert f"kernel=adhip_attention_d{d}_v{dv}_k" in text and "_parts " in text and "[attention_split]" in text, text
+    rc, msg = _compile_check(dev.proc, dev.deps)
+    assert rc == 0 and "lowered" not in msg, msg
+
+
+@pytest.mark.parametrize("sq,sk,d,dv", [(64, 31, 64, 64), (64, 64, 48, 48), (64, 64, 64, 48), (64, 64, 160, 128)])
+def test_what_it_does_not_take_stays_on_the_fp32_ones(sq, sk, d, dv):
+    dev = Capture()
+    _program(dev, *_zeros(sq, sk, d, dv), 64)
+    text = lower_describe(dev.proc, dev.deps)
+    assert "[attention]" in text and "_parts" not in text, text
+
+
+def test_a_program_that_fits_the_static_scratch_area_without_parts_still_fits():
+    """Keys and values in parts take six bytes a number: 2500 x 64 of eight heads 15 MB, beside 24 MB without them."""
+    from adhip import workloads as W
+    for seq, parts in ((512, True), (2500, False)):
+        dev = Capture()
+        W.attention_forward(dev, seq, 512, 8).run()
+        text = lower_describe(dev.proc, dev.deps)
+        assert ("_parts" in text) == parts, text
+
+
+def _exact(q, k, v, scale_dim):
+    s = q.astype(np.float64) @ k.astype(np.float64).T / math.sqrt(scale_dim)
+    e = np.exp(s - s.max(1, keepdims=True))
+    return (e / e.sum(1, keepdims=True)) @ v.astype(np.float64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,dv", WIDTHS)
+@pytest.mark.parametrize("sq,sk", [(64, 32), (1, 33), (65, 63), (130, 255), (63, 257), (200, 520)])
+def test_values(sq, sk, d, dv, hip_device):
+    print(f"[case] attention in parts {sq}x{sk} d {d} dv {dv}", flush=True)
+    rng = np.random.default_rng(sq + 3 * sk + 7 * d + dv)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((sq, d), (sk, d), (sk, dv)))
+    got = _program(hip_device, q, k, v, 16).val().get()
+    # a score is a sum of d products of size 1, over 4: its error, 2^-24 sqrt(d) sqrt(d) / 4 at most, is the probability's relative one
+    assert_close(got.data, _exact(q, k, v, 16).reshape(-1), RED_RTOL * math.sqrt(max(sk, d)), "o")
+
+
+@pytest.mark.gpu
+def test_operands_that_the_parts_cannot_represent(hip_device):
+    """A value beyond bf16's largest number and an infinite one: their blocks of 64 rows are what the FP32 matrix cores make of
+    them, the others are as before."""
+    print("[case] attention in parts, unrepresentable operands", flush=True)
+    rng = np.random.default_rng(5)
+    sq, sk, d, dv = 190, 140, 64, 64
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((sq, d), (sk, d), (sk, dv)))
+    v[7, 3] = np.finfo(np.float32).max
+    v[9, 5] = np.inf
+    got = np.asarray(_program(hip_device, q, k, v, 16).val().get().data, np.float64).reshape(sq, dv)
+    want = _exact(q, k, v, 16)
+    assert np.all(got[:, 5] == np.inf)
+    cols = [c for c in range(dv) if c != 5]
+    np.testing.assert_allclose(got[:, cols], want[:, cols], rtol=2e-4, atol=2e-4)
+    q[70] = np.nan
+    v[9, 5] = v[7, 3] = 1.0
+    got = np.asarray(_program(hip_device, q, k, v, 16).val().get().data, np.float64).reshape(sq, dv)
+    assert np.all(np.isnan(got[70]))
+    rows = [r for r in range(sq) if r != 70]
+    np.testing.assert_allclose(got[rows], _exact(q, k, v, 16)[rows], rtol=0, atol=2e-5)
