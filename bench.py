@@ -165,7 +165,7 @@ def measure_mlp(dev, iters):
 
 def measure_attention(dev, seq=2048, d_model=1024, heads=8):
     """Multi-head attention forward (inference), [seq, d_model] activations: the fused attention kernel's rate against
-    the FP32 matrix-core peak, and the same program lowered without the fusion beside it."""
+    the bf16 matrix cores' over six (three parts an operand, six products of parts), and the same program lowered without the fusion beside it."""
     from adhip import workloads as W
     out = {}
     for mode in ("fused", "unfused"):
@@ -182,10 +182,10 @@ def measure_attention(dev, seq=2048, d_model=1024, heads=8):
                  "matmul_TFLOPs_whole_step": wl.flops / (ms * 1e-3) / 1e12}
         if mode == "fused":
             for k in ks:
-                if k["kernel"].startswith("attention"):
+                if k["kernel"].startswith("attention:"):
                     tf = wl.attention_flops / (k["avg_ms"] * 1e-3) / 1e12
-                    entry["roofline"] = {"kernel": k["kernel"], "bound": "mfma", "achieved": tf, "peak": FP32_MFMA_PEAK_TFLOPS,
-                                         "unit": "TFLOP/s", "frac": tf / FP32_MFMA_PEAK_TFLOPS, "traffic": None,
+                    entry["roofline"] = {"kernel": k["kernel"], "bound": "mfma", "achieved": tf, "peak": BF16_PARTS_PEAK_TFLOPS,
+                                         "unit": "TFLOP/s", "frac": tf / BF16_PARTS_PEAK_TFLOPS, "traffic": None,
                                          "avg_ms": k["avg_ms"],
                                          "flops_per_launch": wl.attention_flops,
                                          "note": "2 * 2 * seq^2 * head_width flops per head (the two products; the "

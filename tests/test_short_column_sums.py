@@ -7,7 +7,7 @@ import pytest
 from adhip import ir as IR
 from adhip.device import lower_describe
 
-SHAPES = [(33, 24), (64, 64), (65, 1000), (127, 258), (128, 4100), (129, 64), (200, 28)]
+SHAPES = [(33, 256), (64, 64), (65, 1000), (127, 258), (128, 4100), (129, 64), (200, 28)]
 
 
 def _program(rows, cols, x, op):
