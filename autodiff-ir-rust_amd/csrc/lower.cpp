@@ -3377,16 +3377,17 @@ struct Lowerer {
 
     // 0: both operands are 16-byte aligned line by line and k is a multiple of the tile depth (the kernel without
     // bounds checks, if M and N fit the tile as well); 1: not so, but a line of either operand holds at least four
-    // elements (128-bit reads of whatever alignment, single elements on the ragged rim); 2: single elements only
+    // elements (128-bit reads of whatever alignment, single elements on the ragged rim); 2: single elements only.
+    // kLongLines on top, whatever the elements of a line: lines of 2^22 elements and more.  The kernels without bounds
+    // checks, and the one without a staging buffer, address a tile by 32-bit offsets from its corner; such operands take the
+    // checked variant and 64-bit offsets.
+    static constexpr int kLongLines = 4;
     static int dot_alignment(const Affine2D& a, const Affine2D& b, int64_t M, int64_t N, int64_t K) {
         const bool a_k = a.s1 == 1, b_k = b.s0 == 1;
-        const int64_t a_ld = a_k ? a.s0 : a.s1, b_ld = b_k ? b.s1 : b.s0;
-        if ((a_k ? K : M) < 4 || (b_k ? K : N) < 4) return 2;
-        // (the kernel without bounds checks addresses a tile by 32-bit offsets from its corner: lines of 2^22 elements
-        // and more take the checked variant, whose index arithmetic is 64 bits wide)
-        const int64_t widest = int64_t(1) << 22;
-        if (a_ld >= widest || b_ld >= widest) return 3;
-        return ((a.offset % 4) || (b.offset % 4) || (a_ld % 4) || (b_ld % 4) || (K % 16)) ? 1 : 0;
+        const int64_t a_ld = a_k ? a.s0 : a.s1, b_ld = b_k ? b.s1 : b.s0, longest = int64_t(1) << 22;
+        const bool long_lines = a_ld >= longest || b_ld >= longest;
+        const bool aligned = !long_lines && a.offset % 4 == 0 && b.offset % 4 == 0 && a_ld % 4 == 0 && b_ld % 4 == 0 && K % 16 == 0;
+        return ((a_k ? K : M) < 4 || (b_k ? K : N) < 4 ? 2 : aligned ? 0 : 1) + (long_lines ? kLongLines : 0);
     }
 
     template <class ReadsNode, class KeepsEpilogue>
@@ -3708,6 +3709,8 @@ struct Lowerer {
     static DotLaunchPlan plan_product(int64_t M, int64_t N, int64_t K, int64_t cnt, bool a_kcontig, bool b_kcontig, int alignment) {
         DotLaunchPlan pl;
         GemmConfig& cfg = pl.cfg;
+        const bool long_lines = alignment >= kLongLines;
+        alignment %= kLongLines;
         cfg.a_kcontig = a_kcontig;
         cfg.b_kcontig = b_kcontig;
         auto blocks = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * cnt; };
@@ -3775,7 +3778,7 @@ struct Lowerer {
                 }
             cfg.narrow_m = M < cfg.bm;
             cfg.narrow_n = N < cfg.bn;
-            cfg.wide_lines = alignment == 3;
+            cfg.wide_lines = long_lines;
         }
         // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits> forces tile and k ranges of every product with k of 64 and more
         if (const char* e = getenv("ADHIP_DOT_PLAN")) {
