@@ -803,7 +803,10 @@ static GeneratedKernel gen_elw_colsum_kernel(const ElwKernelSpec& spec, const st
     std::string src = kernel_prelude();
     src += strf("extern \"C\" __global__ __launch_bounds__(1024) void %s(%s) {\n", k.entry.c_str(), sig.c_str());
     src += "    if (guard && *guard == 0) return;\n";
-    if (!spec.colsums.empty()) src += "    __shared__ float4_t part[2][16][64];\n";
+    if (!spec.colsums.empty()) {
+        src += "    __shared__ float4_t part[2][16][64];\n";
+        k.lds_bytes = 2 * 16 * 64 * 16;
+    }
     src += "    const unsigned lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;\n";
     src += strf("    const %s %s = (%s)blockIdx.x * 64u + lane;\n", it, (K >= 2 && K <= 4) ? "c1_raw" : "c1", it);
     src += strf("    const bool col_ok = %s < %lld%s;\n", (K >= 2 && K <= 4) ? "c1_raw" : "c1", (long long)(C / 4), sfx);
@@ -974,6 +977,7 @@ static bool gen_elw_tiled_kernel(const ElwKernelSpec& spec, const std::set<const
     src += strf("extern \"C\" __global__ __launch_bounds__(256) void %s(%s) {\n", k.entry.c_str(), sig.c_str());
     src += "    if (guard && *guard == 0) return;\n";
     for (auto& st : g.staged) src += strf("    __shared__ float tile%d[%lld][%lld];\n", st.slot, (long long)TC, (long long)(TR + 1));
+    k.lds_bytes = g.staged.size() * (size_t)(TC * (TR + 1)) * 4;
     src += "    const unsigned tid = threadIdx.x;\n";
     src += strf("    %s bid = blockIdx.x;\n", it);
     src += strf("    const %s col0 = (bid %% %lld%s) * %lldu;\n    bid /= %lld%s;\n", it, (long long)TI, sfx.c_str(), (long long)TC, (long long)TI, sfx.c_str());
@@ -1414,6 +1418,7 @@ GeneratedKernel gen_reduce_kernel(const ReduceKernelSpec& spec, int64_t force_ch
             src += epilogue + "    }\n";
         } else {
             src += strf("    __shared__ float part[4];\n    s = %s(s);\n", wave_comb);
+            k.lds_bytes = 4 * 4;
             src += "    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = s;\n    __syncthreads();\n";
             src += "    if (threadIdx.x == 0 && row_ok) {\n        const float sum_value = " + comb4("part[0]", "part[1]", "part[2]", "part[3]") + ";\n";
             src += strf("        out[(%s)chunk * %lldu + x] = sum_value;\n", g.idx_t(), (long long)V);
@@ -1457,6 +1462,7 @@ GeneratedKernel gen_reduce_kernel(const ReduceKernelSpec& spec, int64_t force_ch
             src += strf("extern \"C\" __global__ __launch_bounds__(1024) void %s(%s) {\n", k.entry.c_str(), sig.c_str());
             src += "    if (guard && *guard == 0) return;\n";
             src += "    __shared__ float4_t part[16][64];\n";
+            k.lds_bytes = 16 * 64 * 16;
             src += "    const unsigned lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;\n";
             src += strf("    const %s xv_raw = (%s)blockIdx.x * 64u + lane;\n", it, it);
             src += strf("    const bool col_ok = xv_raw < %lld%s;\n    const %s xv = col_ok ? xv_raw : %lld%s;\n", (long long)XV, sfx, it, (long long)(XV - 1), sfx);
@@ -1508,6 +1514,7 @@ GeneratedKernel gen_reduce_kernel(const ReduceKernelSpec& spec, int64_t force_ch
         src += strf("extern \"C\" __global__ __launch_bounds__(%d) void %s(%s) {\n", 64 * YG, k.entry.c_str(), sig.c_str());
         src += "    if (guard && *guard == 0) return;\n";
         src += strf("    __shared__ float part[%d][64][%d];\n", YG, vec);
+        k.lds_bytes = (size_t)(YG * 64 * vec) * 4;
         src += "    const unsigned lx = threadIdx.x & 63u, ly = threadIdx.x >> 6;\n";
         src += strf("    const %s xv = (%s)blockIdx.x * 64u + lx;\n", g.idx_t(), g.idx_t());
         src += "    const unsigned chunk = blockIdx.y;\n";
@@ -1722,7 +1729,10 @@ GeneratedKernel gen_rowchain_kernel(const RowChainSpec& spec) {
     std::string src = kernel_prelude();
     src += strf("extern \"C\" __global__ __launch_bounds__(256) void %s(%s) {\n", k.entry.c_str(), sig.c_str());
     src += "    if (guard && *guard == 0) return;\n";
-    if (T == 256 && n_reduce > 0) src += strf("    __shared__ float part[%d][4];\n", n_reduce);
+    if (T == 256 && n_reduce > 0) {
+        src += strf("    __shared__ float part[%d][4];\n", n_reduce);
+        k.lds_bytes = (size_t)n_reduce * 4 * 4;
+    }
     src += strf("    const unsigned lane = threadIdx.x %% %du;\n", T);
     src += strf("    const %s x_raw = (%s)blockIdx.x * %du + threadIdx.x / %du;\n", it_t, it_t, rows_per_block, T);
     // a row beyond the last one works on the last one and stores nothing: no thread leaves early

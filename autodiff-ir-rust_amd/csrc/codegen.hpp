@@ -71,7 +71,7 @@ struct GeneratedKernel {
     std::vector<Node*> buffer_args;  // in signature order (after guard); outputs included
     std::vector<int64_t> int_args;   // trailing integer arguments
     unsigned grid[3] = {1, 1, 1}, block[3] = {1, 1, 1};
-    unsigned lds_bytes = 0;
+    size_t lds_bytes = 0;            // declared in the source
     double bytes = 0, flops = 0;
     // reductions that need a second pass: partial sums [chunks][V] written to `out`, then summed
     // (for element-wise kernels with column sums: the number of row tiles)

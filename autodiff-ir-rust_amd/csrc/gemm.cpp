@@ -27,9 +27,9 @@ unsigned gemm_threads(const GemmConfig& cfg) {
     return 64u * (unsigned)((cfg.bm / (32 * wave_rows(cfg))) * (gemm_tile_columns(cfg) / (32 * wave_columns(cfg))) * cfg.k_waves);
 }
 
-size_t gemm_shared_bytes(const GemmConfig& cfg) {
-    if (!cfg.bf16_parts || cfg.bm > 64) return 0;
+size_t gemm_lds_bytes(const GemmConfig& cfg) {
     const size_t bm = (size_t)cfg.bm, bn = (size_t)gemm_tile_columns(cfg), bk = (size_t)cfg.bk;
+    if (!cfg.bf16_parts) return 4 * 2 * bk * (bm + 4 + bn + 4);
     if (cfg.k_waves != kDirectWaves) return 16 * 2 * 3 * (bk / 8) * (bm + 4 + bn + 4);
     const size_t lines = (cfg.a_kcontig ? bm * bk : 0) + (cfg.b_kcontig ? bn * bk : 0);
     return 4 * kDirectWaves * std::max(lines, bn * (bm + 4));

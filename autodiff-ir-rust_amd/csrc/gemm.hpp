@@ -47,8 +47,8 @@ std::string gemm_tile_head(const GemmConfig& cfg);
 std::string gemm_entry(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue, unsigned threads, const char* more = "");
 int gemm_tile_columns(const GemmConfig& cfg);
 unsigned gemm_threads(const GemmConfig& cfg);
-// LDS of a block of at most 64x64 on the bf16 matrix cores, which is one array that kernels in one launch can share; 0 for others
-size_t gemm_shared_bytes(const GemmConfig& cfg);
+// LDS of a block: on the bf16 matrix cores one array `lds`
+size_t gemm_lds_bytes(const GemmConfig& cfg);
 
 std::string gemm_kernel_source(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr);
 // The same product on the bf16 matrix cores, every operand split into three bf16 parts (gemm_split.cpp).

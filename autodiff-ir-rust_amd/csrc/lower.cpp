@@ -18,6 +18,9 @@
 
 namespace adhip {
 
+// LDS of the kernels below that have any
+constexpr size_t kTransposeLds = 64 * 65 * 4, kFinalizeLds = 64 * 16 * 16;
+
 const char* fixed_kernels_source() {
     return R"(
 extern "C" __global__ __launch_bounds__(256) void adhip_copy(const int* __restrict__ guard, float* __restrict__ dst,
@@ -996,7 +999,7 @@ struct Lowerer {
     // Kernels are told apart by their text with the entry name blanked: the per-head kernels of multi-head attention
     // (and the same epilogue generated for two layers) differ in nothing but the position in the program that their
     // name carries, and then share the first one's code object instead of being compiled once each.
-    int add_kernel(const std::string& entry, const std::string& source, const std::string& kind, size_t shared_bytes = 0) {
+    int add_kernel(const std::string& entry, const std::string& source, const std::string& kind, size_t lds_bytes = 0, const GemmConfig* product = nullptr) {
         std::string key;
         key.reserve(source.size());
         auto ident = [](char c) { return isalnum((unsigned char)c) || c == '_'; };
@@ -1020,11 +1023,18 @@ struct Lowerer {
         d.entry = entry;
         d.source = source;
         d.kind = kind;
-        d.shared_bytes = shared_bytes;
+        d.lds_bytes = lds_bytes;
+        d.one_array = product && product->bf16_parts;
+        d.tile_rows = product ? product->bm : 0;
         d.regions.push_back(cur_region);
         plan->kernels.push_back(std::move(d));
         kernel_by_source[key] = (int)plan->kernels.size() - 1;
         return (int)plan->kernels.size() - 1;
+    }
+
+    int add_kernel(const GeneratedKernel& k) { return add_kernel(k.entry, k.source, k.kind, k.lds_bytes); }
+    int add_product(const GemmConfig& cfg, const std::string& entry, const GemmEpilogue* epilogue = nullptr) {
+        return add_kernel(entry, gemm_source(cfg, entry, epilogue), "dot_mfma", gemm_lds_bytes(cfg), &cfg);
     }
 
     // The variant of a generated kernel that runs `cnt` instances of it in one launch: the kernel becomes a device
@@ -1077,7 +1087,7 @@ struct Lowerer {
         out += "    default: return;\n    }\n    " + base.entry + "_one(guard";
         for (auto& pr : params) out += ", " + pr.second;
         out += ");\n}\n";
-        const int idx = add_kernel(entry, out, base.kind);
+        const int idx = add_kernel(entry, out, base.kind, base.lds_bytes);
         layered_kernels[{kernel, cnt}] = idx;
         return idx;
     }
@@ -1373,13 +1383,7 @@ struct Lowerer {
     // Nothing is taken from further than 64 launches behind the oldest one left: what waits for its readers takes memory.
     static constexpr int kSharedArgs = 360, kSharedMembers = 12;
     static constexpr size_t kSharedWindow = 64;
-    // LDS that a kernel has for itself in such a launch (at most)
-    static size_t own_lds(const KernelDef& kd, unsigned threads) {
-        if (kd.kind == "dot_mfma") return kd.shared_bytes ? 0 : 2 * 2 * 16 * 68 * 4;
-        if (kd.kind == "elw_colsum") return 2 * 16 * 64 * 16;
-        return threads > 512 ? 16 * 64 * 16 : 4352;
-    }
-    static bool small_product(const KernelDef& kd) { return kd.shared_bytes > 0 || kd.entry.find("_64") != std::string::npos; }
+    static constexpr size_t kLds = 160 * 1024;   // bytes of a CU's LDS
     void share_independent_launches(std::vector<Step>& out, size_t from) {
         for (size_t at = from; at < out.size();) {
             while (at < out.size() && !can_share(out[at])) ++at;
@@ -1396,8 +1400,8 @@ struct Lowerer {
         const KernelDef& kd = plan->kernels[(size_t)l.kernel];
         for (const Arg& a : l.args)
             if (a.kind == Arg::FLAG) return false;   // (the loop's last kernel stays its last)
-        return shareable.count(kd.kind) && l.block[1] == 1 && l.block[2] == 1 && l.lds_bytes == 0 && (uint64_t)l.grid[0] * l.grid[1] * l.grid[2] <= 512 &&
-               (kd.kind != "dot_mfma" || small_product(kd));
+        return shareable.count(kd.kind) && l.block[1] == 1 && l.block[2] == 1 && (uint64_t)l.grid[0] * l.grid[1] * l.grid[2] <= 512 &&
+               kd.tile_rows <= 64;
     }
     // A run of such launches; returns how many are left of it.
     size_t share_run(std::vector<Step>& out, size_t from, size_t to) {
@@ -1431,8 +1435,7 @@ struct Lowerer {
             it.chain = kd.kind == "rowchain";
             it.blocks = (int64_t)l.grid[0] * l.grid[1] * l.grid[2];
             it.threads = l.block[0];
-            it.own = own_lds(kd, it.threads);
-            it.shared = kd.shared_bytes;
+            (kd.one_array ? it.shared : it.own) = kd.lds_bytes;
             for (size_t j = 0; j < i; ++j) {
                 auto meet = [](const std::set<int>& x, const std::set<int>& y) {
                     for (int b : x)
@@ -1464,7 +1467,7 @@ struct Lowerer {
                 const unsigned threads = std::max(sum.threads, it.threads);
                 const bool mixed = threads != std::min(sum.threads, it.threads), chain = sum.chain || it.chain;
                 if (!it.ok || ((product || chain) && threads > 512) || (mixed && sum.blocks + it.blocks > 512) || sum.blocks + it.blocks > (product ? 512 : 1024) || args + more > (size_t)kSharedArgs ||
-                    sum.own + it.own + std::max(sum.shared, it.shared) > 160 * 1024)
+                    sum.own + it.own + std::max(sum.shared, it.shared) > kLds)
                     continue;
                 set.push_back(ready[q]);
                 sum.product = product;
@@ -1504,7 +1507,8 @@ struct Lowerer {
         unsigned first = 0;
         for (size_t i : set) {
             m.block[0] = std::max(m.block[0], out[from + i].launch.block[0]);
-            shared = std::max(shared, plan->kernels[(size_t)out[from + i].launch.kernel].shared_bytes);
+            const KernelDef& kd = plan->kernels[(size_t)out[from + i].launch.kernel];
+            if (kd.one_array) shared = std::max(shared, kd.lds_bytes);
         }
         if (shared) src += strf("static __device__ __forceinline__ char* adhip_lds() {\n    __shared__ __attribute__((aligned(16))) char lds[%zu];\n    return lds;\n}\n", shared);
         for (size_t q = 0; q < set.size(); ++q) {
@@ -1517,7 +1521,7 @@ struct Lowerer {
             replace_all("extern \"C\" __global__", "static __device__ __forceinline__");
             for (size_t at = body.find("__launch_bounds__("); at != std::string::npos; at = body.find("__launch_bounds__(")) body.erase(at, body.find(')', at) + 1 - at);
             replace_all("blockIdx", "adhip_block()");
-            if (kd.shared_bytes) {
+            if (kd.one_array) {
                 // (the product kernels' one array: "__shared__ __attribute__((aligned(16))) <type> lds[...];")
                 const size_t at = body.find("__shared__ __attribute__((aligned(16))) "), name = body.find(" lds[", at), end = body.find(';', at);
                 ADHIP_CHECK(end != std::string::npos && name < end, "internal: kernel '%s' has no LDS array", kd.entry.c_str());
@@ -1576,7 +1580,7 @@ struct Lowerer {
         auto single_block = [&](const Step& st) {
             if (st.kind != Step::LAUNCH) return false;
             const Launch& l = st.launch;
-            if (l.grid[0] != 1 || l.grid[1] != 1 || l.grid[2] != 1 || l.block[0] != 256 || l.block[1] != 1 || l.block[2] != 1 || l.lds_bytes != 0) return false;
+            if (l.grid[0] != 1 || l.grid[1] != 1 || l.grid[2] != 1 || l.block[0] != 256 || l.block[1] != 1 || l.block[2] != 1) return false;
             return mergeable.count(plan->kernels[(size_t)l.kernel].kind) > 0;
         };
         for (size_t i = from; i < out.size(); ++i) {
@@ -1593,10 +1597,12 @@ struct Lowerer {
             merged.block[0] = 256;
             merged.guard = out[i].launch.guard;
             bool ok = true;
+            size_t lds = 0;   // phases have theirs side by side (1 KB for a column sum, and 80 of those have the arguments)
             for (size_t q = i; q < j && ok; ++q) {
                 const Launch& l = out[q].launch;
                 const KernelDef& kd = plan->kernels[(size_t)l.kernel];
                 std::string body = kd.source;
+                lds += kd.lds_bytes;
                 const std::string head = "extern \"C\" __global__", bounds = "__launch_bounds__(", noalias = "__restrict__";
                 for (size_t at = body.find(head); at != std::string::npos; at = body.find(head)) body.replace(at, head.size(), "static __device__");
                 for (size_t at = body.find(bounds); at != std::string::npos; at = body.find(bounds)) body.erase(at, body.find(')', at) + 1 - at);
@@ -1621,7 +1627,7 @@ struct Lowerer {
             if (!ok) continue;
             const std::string entry = strf("run%d_%s_x%zu", kernel_counter++, out[i].launch.label.c_str(), j - i);
             src += "extern \"C\" __global__ __launch_bounds__(256) void " + entry + "(" + params + ") {\n" + calls + "}\n";
-            merged.kernel = add_kernel(entry, src, "merged");
+            merged.kernel = add_kernel(entry, src, "merged", lds);
             merged.label = entry;
             KernelStat st;
             st.label = entry;
@@ -2956,9 +2962,8 @@ struct Lowerer {
             bool ok = true;
             auto add = [&](const GeneratedKernel& k) {
                 if (k.source.find("blockIdx.z") != std::string::npos || !k.int_args.empty()) ok = false;
-                sig.push_back(add_kernel(k.entry, k.source, k.kind));
+                sig.push_back(add_kernel(k));
                 for (int d = 0; d < 3; ++d) { sig.push_back(k.grid[d]); sig.push_back(k.block[d]); }
-                sig.push_back(k.lds_bytes);
                 sig.push_back((int64_t)k.buffer_args.size());
                 sig.push_back(k.chunks);
             };
@@ -3113,10 +3118,9 @@ struct Lowerer {
         };
         auto launch_generated = [&](GeneratedKernel& gk) {
             Launch l2;
-            l2.kernel = add_kernel(gk.entry, gk.source, gk.kind);
+            l2.kernel = add_kernel(gk);
             memcpy(l2.grid, gk.grid, sizeof l2.grid);
             memcpy(l2.block, gk.block, sizeof l2.block);
-            l2.lds_bytes = gk.lds_bytes;
             l2.label = gk.entry;
             l2.bytes = gk.bytes;
             l2.flops = gk.flops;
@@ -3129,10 +3133,9 @@ struct Lowerer {
             GeneratedKernel& k = gks[g].k;
             std::vector<std::pair<Launch, std::string>> ls;
             Launch l;
-            l.kernel = add_kernel(k.entry, k.source, k.kind);
+            l.kernel = add_kernel(k);
             memcpy(l.grid, k.grid, sizeof l.grid);
             memcpy(l.block, k.block, sizeof l.block);
-            l.lds_bytes = k.lds_bytes;
             l.label = k.entry;
             l.bytes = k.bytes;
             l.flops = k.flops;
@@ -3145,7 +3148,7 @@ struct Lowerer {
                 ls.push_back({l, k.kind});
                 GeneratedKernel& k2 = gks[g].extra[0];
                 Launch l2;
-                l2.kernel = add_kernel(k2.entry, k2.source, k2.kind);
+                l2.kernel = add_kernel(k2);
                 memcpy(l2.grid, k2.grid, sizeof l2.grid);
                 memcpy(l2.block, k2.block, sizeof l2.block);
                 l2.label = k2.entry;
@@ -3190,7 +3193,7 @@ struct Lowerer {
                     const size_t nc = std::min<size_t>(4, G.colsums.size() - cols_done);
                     const int64_t runs = elw_rowsum_runs(G.cs_cols);
                     const int64_t col_blocks = nc ? (G.cs_cols + 63) / 64 : 0, row_blocks = (G.cs_rows + 1023) / 1024;
-                    if (fixed_sums_finalize < 0) fixed_sums_finalize = add_kernel("adhip_sums_finalize", fixed_kernels_source(), "sums_finalize");
+                    if (fixed_sums_finalize < 0) fixed_sums_finalize = add_kernel("adhip_sums_finalize", fixed_kernels_source(), "sums_finalize", kFinalizeLds);
                     Launch lf;
                     lf.kernel = fixed_sums_finalize;
                     lf.block[0] = 1024;
@@ -3215,7 +3218,7 @@ struct Lowerer {
                     cols_done += nc;
                 }
                 // the column sums that are left: one launch of the fixed second-pass kernel per four sums
-                if (cols_done < G.colsums.size() && fixed_finalize < 0) fixed_finalize = add_kernel("adhip_colsum_finalize", fixed_kernels_source(), "colsum_finalize");
+                if (cols_done < G.colsums.size() && fixed_finalize < 0) fixed_finalize = add_kernel("adhip_colsum_finalize", fixed_kernels_source(), "colsum_finalize", kFinalizeLds);
                 for (size_t i0 = cols_done; i0 < G.colsums.size(); i0 += 4) {
                     const size_t cnt = std::min<size_t>(4, G.colsums.size() - i0);
                     Launch lf;
@@ -3302,7 +3305,7 @@ struct Lowerer {
         }
         Launch& l = out.back().launch;
         if (!nk.latch_done || l.label != gk.k.entry || nk.buffer_args.size() != gk.k.buffer_args.size()) return;
-        l.kernel = add_kernel(nk.entry, nk.source, nk.kind);
+        l.kernel = add_kernel(nk);
         l.label = nk.entry;
         plan->stats[(size_t)l.stat].label = nk.entry;
         plan->stats[(size_t)l.stat].kernel = l.kernel;
@@ -3336,8 +3339,8 @@ struct Lowerer {
         ADHIP_CHECK(st.offset >= 0 && hi < numel(pc.src.node->shape), "internal: transposing copy reads outside its source");
         bool v4 = (U % 4 == 0) && (V % 4 == 0) && (st.offset % 4 == 0) && (st.stride[last] % 4 == 0) && (dense[u] % 4 == 0);
         for (int q = 0; q < 3; ++q) v4 = v4 && (ib[q] % 4 == 0) && (ob[q] % 4 == 0);
-        if (fixed_transpose < 0) fixed_transpose = add_kernel("adhip_transpose_copy", fixed_kernels_source(), "transpose");
-        if (fixed_transpose4 < 0) fixed_transpose4 = add_kernel("adhip_transpose_copy4", fixed_kernels_source(), "transpose");
+        if (fixed_transpose < 0) fixed_transpose = add_kernel("adhip_transpose_copy", fixed_kernels_source(), "transpose", kTransposeLds);
+        if (fixed_transpose4 < 0) fixed_transpose4 = add_kernel("adhip_transpose_copy4", fixed_kernels_source(), "transpose", kTransposeLds);
         Launch l;
         l.kernel = v4 ? fixed_transpose4 : fixed_transpose;
         l.block[0] = 256;
@@ -3526,7 +3529,7 @@ struct Lowerer {
         const std::string entry = small ? "adhip_dot_small_grouped" : dot_kernel_name(cfg) + "_grouped", kind = small ? "dot_naive" : "dot_mfma";
         const int lanes = small_dot_lanes(M, N, K, key0[4] <= key0[3] && key0[5] <= key0[6]);
         Launch l;
-        l.kernel = add_kernel(entry, small ? dot_small_source(entry, nullptr, true) : gemm_source(cfg, entry), kind, small ? 0 : gemm_shared_bytes(cfg));
+        l.kernel = small ? add_kernel(entry, dot_small_source(entry, nullptr, true), kind) : add_product(cfg, entry);
         l.block[0] = small ? 256u : gemm_threads(cfg);
         l.grid[0] = (unsigned)(small ? (M * N * lanes + 255) / 256 : ((M + cfg.bm - 1) / cfg.bm) * ((N + pl.bn_tile - 1) / pl.bn_tile));
         l.grid[1] = (unsigned)cnt;
@@ -3604,12 +3607,12 @@ struct Lowerer {
         ADHIP_CHECK(attention_key(atts[0], key0, q0, k0, v0), "internal: attention node whose operands the kernel cannot read");
         const AttentionConfig cfg = attention_config(key0, cnt);
         const int64_t row_blocks = (key0.sq + 63) / 64;
-        ADHIP_CHECK(attention_lds_bytes(cfg) <= 160 * 1024, "internal: attention tiles of %d keys do not fit in LDS", cfg.bn);
+        ADHIP_CHECK(attention_lds_bytes(cfg) <= kLds, "internal: attention tiles of %d keys do not fit in LDS", cfg.bn);
         ADHIP_CHECK(cfg.parts == (parts != nullptr) && (!parts || numel(parts->shape) == cnt * attention_parts_floats(cfg, key0.sk)),
                     "internal: attention and its keys and values in parts disagree");
         const std::string entry = strf("adhip_attention_d%d_v%d_k%d_w%d%s%s", cfg.d, cfg.dv, cfg.bn, cfg.wg, cfg.mask ? "_mask" : "", cfg.parts ? "_parts" : "");
         Launch l;
-        l.kernel = add_kernel(entry, attention_kernel_source(cfg, entry), "attention");
+        l.kernel = add_kernel(entry, attention_kernel_source(cfg, entry), "attention", attention_lds_bytes(cfg) + (cfg.parts ? 4 : 0));
         l.block[0] = 256u * (unsigned)cfg.wg;
         ADHIP_CHECK(row_blocks * cnt <= 0x7fffffff, "internal: attention grid too large");
         l.grid[0] = (unsigned)(row_blocks * cnt);
@@ -3841,9 +3844,9 @@ struct Lowerer {
                 ge.params = epi->params;
                 ge.code = epi->code;
                 ge.store_c = store_c;
-                l.kernel = add_kernel(entry, gemm_source(cfg, entry, &ge), "dot_mfma", gemm_shared_bytes(cfg));
+                l.kernel = add_product(cfg, entry, &ge);
             } else {
-                l.kernel = add_kernel(entry, gemm_source(cfg, entry), "dot_mfma", gemm_shared_bytes(cfg));
+                l.kernel = add_product(cfg, entry);
             }
             l.block[0] = gemm_threads(cfg);
             l.grid[0] = (unsigned)(((M + cfg.bm - 1) / cfg.bm) * ((N + bn_tile - 1) / bn_tile));

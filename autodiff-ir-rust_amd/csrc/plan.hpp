@@ -22,7 +22,9 @@ struct KernelDef {
     std::string entry;   // symbol name
     std::string source;  // complete HIP C++ translation unit
     std::string kind;    // "elw", "reduce_row", "reduce_col", "dot", ...
-    size_t shared_bytes = 0;  // LDS of a product kernel (its one array `lds`), 0 for all others
+    size_t lds_bytes = 0;     // static LDS of a block
+    bool one_array = false;   // ... is one array `lds`, which the kernels of one launch can share
+    int tile_rows = 0;        // of a product on the matrix cores
     bool part_only = false;  // only parts of shared launches refer to it: it is described, but never compiled
     std::vector<int> regions;  // the straight-line regions (in lowering order) whose launches use it
 };
@@ -39,7 +41,6 @@ struct Launch {
     int kernel = -1;  // index into Plan::kernels
     unsigned grid[3] = {1, 1, 1};
     unsigned block[3] = {1, 1, 1};
-    unsigned lds_bytes = 0;
     std::vector<Arg> args;  // after the leading guard pointer
     int guard = -1;         // flag slot or -1
     std::string label;

@@ -325,7 +325,7 @@ std::vector<char> compile_code_object_uncached(const std::string& source, const 
 // Code objects of several sources at once: hipRTC takes a few hundred milliseconds per kernel and a program can
 // have dozens of them, so the ones that are not cached are compiled on several host threads
 // (ADHIP_COMPILE_THREADS, default 8; 1 compiles one after the other).
-std::map<std::string, std::vector<char>> compile_code_objects(const std::vector<std::string>& sources, const std::string& arch) {
+std::map<std::string, std::vector<char>> compile_code_objects(const std::vector<std::string>& sources, const std::string& arch, std::map<std::string, std::string>& errors) {
     std::map<std::string, std::vector<char>> out;
     std::vector<const std::string*> todo;
     for (const std::string& src : sources)
@@ -333,28 +333,30 @@ std::map<std::string, std::vector<char>> compile_code_objects(const std::vector<
     int threads = 8;
     if (const char* e = getenv("ADHIP_COMPILE_THREADS")) threads = std::max(1, atoi(e));
     threads = (int)std::min<size_t>((size_t)threads, todo.size());
-    if (threads <= 1) {
-        for (const std::string* src : todo) out[*src] = compile_code_object(*src, arch);
-        return out;
-    }
     std::atomic<size_t> next{0};
-    std::vector<std::string> errors((size_t)threads);
-    std::vector<std::thread> pool;
-    for (int t = 0; t < threads; ++t)
-        pool.emplace_back([&, t] {
+    std::vector<std::string> failed(todo.size());
+    auto work = [&] {
+        for (size_t i = next.fetch_add(1); i < todo.size(); i = next.fetch_add(1)) {
             try {
-                for (size_t i = next.fetch_add(1); i < todo.size(); i = next.fetch_add(1)) {
-                    std::vector<char> code = compile_code_object(*todo[i], arch);
-                    out.find(*todo[i])->second = std::move(code);   // distinct keys: no two threads touch one entry
-                }
+                std::vector<char> code = compile_code_object(*todo[i], arch);
+                out.find(*todo[i])->second = std::move(code);   // distinct keys: no two threads touch one entry
             } catch (const std::exception& e) {
-                errors[(size_t)t] = e.what();
-                next.store(todo.size());
+                failed[i] = e.what();
             }
-        });
-    for (auto& th : pool) th.join();
-    for (auto& e : errors)
-        if (!e.empty()) throw Error(e);
+        }
+    };
+    if (threads <= 1) work();
+    else {
+        std::vector<std::thread> pool;
+        for (int t = 0; t < threads; ++t) pool.emplace_back(work);
+        for (auto& th : pool) th.join();
+    }
+    for (size_t i = 0; i < todo.size(); ++i)
+        if (!failed[i].empty()) {
+            const std::string src = *todo[i];
+            errors[src] = failed[i];
+            out.erase(src);
+        }
     return out;
 }
 
@@ -428,7 +430,8 @@ std::string describe_spills(const std::vector<char>& code, bool everything) {
 // that the compiler could only build by spilling vector registers to scratch memory is never accepted: the regions
 // it belongs to are lowered again with their kernel-size bounds halved (LowerOptions::region_shift), up to four
 // times, and if a kernel still spills then -- or is not one the lowering can cut: a hand-written one -- the program
-// is refused.  `relowered` receives the number of extra lowerings.
+// is refused.  A launch that several small ones share runs apart in a region where its kernel spills or does not compile.
+// `relowered` receives the number of extra lowerings.
 template <class Have>
 std::unique_ptr<Plan> lower_and_compile(const Proc& ir, const std::vector<std::string>& deps, const std::string& arch, Have&& have,
                                         std::map<std::string, std::vector<char>>& objects, int* relowered = nullptr) {
@@ -439,10 +442,22 @@ std::unique_ptr<Plan> lower_and_compile(const Proc& ir, const std::vector<std::s
         std::vector<std::string> missing;
         for (const KernelDef& k : plan->kernels)
             if (!k.part_only && !objects.count(k.source) && !have(k.source)) missing.push_back(k.source);
-        for (auto& kv : compile_code_objects(missing, arch)) objects[kv.first] = std::move(kv.second);
+        std::map<std::string, std::string> errors;
+        for (auto& kv : compile_code_objects(missing, arch, errors)) objects[kv.first] = std::move(kv.second);
         std::set<int> regions;
         std::string report;
         bool tighter = false;
+        for (const KernelDef& k : plan->kernels) {
+            // a shared launch that does not compile: its launches run apart
+            auto it = errors.find(k.source);
+            if (k.part_only || it == errors.end()) continue;
+            bool apart = false;
+            if (k.kind == "shared")
+                for (int r : k.regions) apart = (r >= 0 && opt.unshared_regions.insert(r).second) || apart;
+            if (!apart) throw Error(it->second);
+            tighter = true;
+            report += (report.empty() ? "" : "; ") + it->second;
+        }
         for (const KernelDef& k : plan->kernels) {
             auto it = objects.find(k.source);
             if (it == objects.end()) continue;  // loaded before, so accepted before
@@ -713,18 +728,18 @@ void launch(adhip_program* p, const Launch& l) {
                        gz = (uint64_t)l.grid[2] * l.block[2];
         if (gx <= 0xffffffffull && gy <= 0xffffffffull && gz <= 0xffffffffull) {
             HIP_OK(hipExtModuleLaunchKernel(p->fn[l.kernel], (uint32_t)gx, (uint32_t)gy, (uint32_t)gz, l.block[0], l.block[1],
-                                            l.block[2], l.lds_bytes, ctx->stream, ptrs, nullptr, e0, e1, 0));
+                                            l.block[2], 0, ctx->stream, ptrs, nullptr, e0, e1, 0));
         } else {
             HIP_OK(hipEventRecord(e0, ctx->stream));
             HIP_OK(hipModuleLaunchKernel(p->fn[l.kernel], l.grid[0], l.grid[1], l.grid[2], l.block[0], l.block[1], l.block[2],
-                                         l.lds_bytes, ctx->stream, ptrs, nullptr));
+                                         0, ctx->stream, ptrs, nullptr));
             HIP_OK(hipEventRecord(e1, ctx->stream));
         }
         p->pending.push_back({l.stat, {e0, e1}});
         if (p->pending.size() > 4096) drain_events(p);
     } else {
         HIP_OK(hipModuleLaunchKernel(p->fn[l.kernel], l.grid[0], l.grid[1], l.grid[2], l.block[0], l.block[1], l.block[2],
-                                     l.lds_bytes, ctx->stream, ptrs, nullptr));
+                                     0, ctx->stream, ptrs, nullptr));
     }
     p->plan->stats[l.stat].launches++;
 }
