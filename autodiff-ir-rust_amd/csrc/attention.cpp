@@ -21,8 +21,8 @@
 // group lq supplies element 16 S + 4 lq + u), so a lane's operands for four consecutive steps are one 128-bit LDS
 // read; the weighted values use the same spreading over the keys of a tile.
 //
-// On the bf16 matrix cores (`parts`: heads of 32 to 128 features without a mask, at least 32 keys): every FP32 operand as three
-// bf16 parts, as in gemm_split.cpp, with keys and values split and put into the order of the lanes by a kernel of its own before.
+// On the bf16 matrix cores (`parts`: keys of 32, 64, 96 or 128 features, values of 32, 64 or 128, no mask, and as many keys as the
+// lowering asks for, at least 32): every FP32 operand as three bf16 parts, as in gemm_split.cpp, with keys and values split and put into the order of the lanes by a kernel of its own before.
 // A wavefront owns all 64 query rows and every eighth tile of 32 keys, with its own running maxima, sums and accumulators, so
 // that nothing is shared and no barrier stands in the loop; the eight are merged at the end.  It multiplies keys by query
 // rows and values by probabilities, so that a row of the softmax is a lane: its maximum takes one exchange between the

@@ -3586,7 +3586,13 @@ struct Lowerer {
         cfg.d = (int)key.d;
         cfg.dv = (int)key.dv;
         cfg.mask = key.m_ld > 0;
-        cfg.parts = opt.attention_parts && !cfg.mask && key.sk >= 32 && attention_takes_parts(cfg.d, cfg.dv);
+        // Parts from 256 keys on, from 384 where a value has more features than a key.  Below, the kernel that writes them and
+        // the merging of eight key groups (of which 160 keys fill five) weigh more than the products (heads x rows x keys x
+        // features, FP32 matrix cores and parts, in us): 8x2048x64x64 8.2, 12.9; 16x4096x64x32 11.7, 24.2; 8x192x192x64 12.8, 13.4;
+        // 16x4096x192x64 39.1, 41.3; 16x4096x224x128 78.4, 80.9; 8x256x256x64 15.7, 13.9; 16x4096x256x32 30.5, 29.4;
+        // 16x4096x256x128 88.1, 84.1; 8x384x384x64 21.1, 16.1; keys of 32 and values of 128 features 8x2048x256 19.4, 20.7, x384 26.1, 24.4.
+        const int64_t parts_from = opt.attention_parts_from ? opt.attention_parts_from : cfg.dv > cfg.d ? 384 : 256;
+        cfg.parts = opt.attention_parts && !cfg.mask && key.sk >= std::max<int64_t>(parts_from, 32) && attention_takes_parts(cfg.d, cfg.dv);
         // On the FP32 matrix cores a launch with two or more blocks per CU runs blocks of four wavefronts on tiles of 32 keys,
         // two of which fit a CU's LDS while the heads are not too wide; a smaller launch splits every tile between two groups
         // of four wavefronts instead, so that a SIMD still has two wavefronts to switch between.  Tiles of 64 keys where two
@@ -4321,7 +4327,7 @@ std::string Plan::describe() const {
 
 std::string lowering_switches() {
     std::string out;
-    for (const char* name : {"ADHIP_GROUP_DOTS", "ADHIP_LAYER_KERNELS", "ADHIP_MERGE_SMALL", "ADHIP_SHARE_INDEPENDENT", "ADHIP_FUSE_ATTENTION", "ADHIP_ROW_CHAINS",
+    for (const char* name : {"ADHIP_GROUP_DOTS", "ADHIP_LAYER_KERNELS", "ADHIP_MERGE_SMALL", "ADHIP_SHARE_INDEPENDENT", "ADHIP_FUSE_ATTENTION", "ADHIP_ATTENTION_PARTS", "ADHIP_ROW_CHAINS",
                              "ADHIP_TIGHTEN", "ADHIP_KERNEL_BOUNDS", "ADHIP_DOT_PLAN", "ADHIP_TILED_SHAPE", "ADHIP_GEMM_AHEAD", "ADHIP_GRAPHS"}) {
         const char* e = getenv(name);
         out += e ? e : "";
@@ -4337,6 +4343,10 @@ std::unique_ptr<Plan> lower_program(const Proc& prog, const std::vector<std::str
     if (const char* e = getenv("ADHIP_MERGE_SMALL")) opt.merge_small = opt.merge_small && atoi(e) != 0;
     if (const char* e = getenv("ADHIP_SHARE_INDEPENDENT")) opt.share_independent = opt.share_independent && atoi(e) != 0;
     if (const char* e = getenv("ADHIP_FUSE_ATTENTION")) opt.fuse_attention = opt.fuse_attention && atoi(e) != 0;
+    if (const char* e = getenv("ADHIP_ATTENTION_PARTS")) {
+        opt.attention_parts = opt.attention_parts && atoi(e) > 0;
+        opt.attention_parts_from = std::max(atoi(e), 0);
+    }
     if (const char* e = getenv("ADHIP_ROW_CHAINS")) opt.row_chains = opt.row_chains && atoi(e) != 0;
     // diagnostic: every region lowered the way a region is after that many kernels of it spilled vector registers
     if (const char* e = getenv("ADHIP_TIGHTEN")) opt.min_shift = std::max(0, std::min(atoi(e), 4));

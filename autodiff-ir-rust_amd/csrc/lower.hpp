@@ -21,6 +21,7 @@ struct LowerOptions {
     bool share_independent = true;  // small launches of a region that do not depend on one another run as one
     bool pack_slots = false;        // a temporary takes any free slot that fits, however large
     bool attention_parts = true;    // attention on the bf16 matrix cores, with keys and values split beforehand
+    int64_t attention_parts_from = 0;  // ... from that many keys on (0: where it is the faster one)
     bool fuse_attention = true;  // dot(softmax(scale * dot(Q, K^T)), V) runs as one kernel
     bool row_chains = true;      // row reductions and the element-wise values between them run as one kernel per row
     // Bounds on the size of one generated kernel, in what drives its register pressure: the places it loads from

@@ -39,19 +39,32 @@ def _zeros(sq, sk, d, dv):
 def test_every_width_compiles_without_spills(d, dv):
     from test_library_cpu import _compile_check
     dev = Capture()
-    _program(dev, *_zeros(100, 200, d, dv), 64)
+    _program(dev, *_zeros(100, 400, d, dv), 64)
     text = lower_describe(dev.proc, dev.deps)
     assert f"kernel=adhip_attention_d{d}_v{dv}_k" in text and "_parts " in text and "[attention_split]" in text, text
     rc, msg = _compile_check(dev.proc, dev.deps)
     assert rc == 0 and "lowered" not in msg, msg
 
 
-@pytest.mark.parametrize("sq,sk,d,dv", [(64, 31, 64, 64), (64, 64, 48, 48), (64, 64, 64, 48), (64, 64, 160, 128)])
+@pytest.mark.parametrize("sq,sk,d,dv", [(64, 31, 64, 64), (64, 400, 48, 48), (64, 400, 64, 48), (64, 400, 160, 128),
+                                        (2048, 255, 64, 64), (64, 32, 32, 32), (300, 300, 32, 64), (64, 383, 64, 128)])
 def test_what_it_does_not_take_stays_on_the_fp32_ones(sq, sk, d, dv):
     dev = Capture()
     _program(dev, *_zeros(sq, sk, d, dv), 64)
     text = lower_describe(dev.proc, dev.deps)
     assert "[attention]" in text and "_parts" not in text, text
+
+
+@pytest.mark.parametrize("sq,sk,d,dv", [(64, 256, 64, 64), (1, 256, 128, 32), (64, 384, 64, 128)])
+def test_what_it_takes(sq, sk, d, dv, monkeypatch):
+    dev = Capture()
+    _program(dev, *_zeros(sq, sk, d, dv), 64)
+    assert "_parts" in lower_describe(dev.proc, dev.deps)
+    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "0")
+    assert "_parts" not in lower_describe(dev.proc, dev.deps)
+    _program(dev, *_zeros(sq, 32, d, dv), 64)
+    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")
+    assert "_parts" in lower_describe(dev.proc, dev.deps)
 
 
 def test_a_program_that_fits_the_static_scratch_area_without_parts_still_fits():
@@ -73,7 +86,8 @@ def _exact(q, k, v, scale_dim):
 @pytest.mark.gpu
 @pytest.mark.parametrize("d,dv", WIDTHS)
 @pytest.mark.parametrize("sq,sk", [(64, 32), (1, 33), (65, 63), (130, 255), (63, 257), (200, 520)])
-def test_values(sq, sk, d, dv, hip_device):
+def test_values(sq, sk, d, dv, hip_device, monkeypatch):
+    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")   # also where the other kernel is the faster one
     print(f"[case] attention in parts {sq}x{sk} d {d} dv {dv}", flush=True)
     rng = np.random.default_rng(sq + 3 * sk + 7 * d + dv)
     q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((sq, d), (sk, d), (sk, dv)))
@@ -83,10 +97,11 @@ def test_values(sq, sk, d, dv, hip_device):
 
 
 @pytest.mark.gpu
-def test_operands_that_the_parts_cannot_represent(hip_device):
+def test_operands_that_the_parts_cannot_represent(hip_device, monkeypatch):
     """A value beyond bf16's largest number and an infinite one: their blocks of 64 rows are what the FP32 matrix cores make of
     them, the others are as before."""
     print("[case] attention in parts, unrepresentable operands", flush=True)
+    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")
     rng = np.random.default_rng(5)
     sq, sk, d, dv = 190, 140, 64, 64
     q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((sq, d), (sk, d), (sk, dv)))
