@@ -640,23 +640,31 @@ struct Lowerer {
         plan->buffers.push_back(b);
         return (int)plan->buffers.size() - 1;
     }
-    // Every temporary of a region has a slot from the first launch that names it to the last.
+    // Every temporary of a region has a slot from the first launch that names it to the last, of a run of phases from the first
+    // phase to the last: a barrier stands between two of them (the README's training step, eleven phases: three slots, five
+    // with the run as one).
     void assign_slots(const std::vector<Step>& out, size_t from, SlotPool& p) {
-        std::map<int, std::pair<size_t, size_t>> life;   // buffer -> first and last step
-        for (size_t i = from; i < out.size(); ++i)
-            for (const Arg& a : out[i].launch.args)
-                if (a.kind == Arg::BUF && plan->buffers[(size_t)a.buf].kind == PlanBuffer::TEMP) {
-                    auto it = life.emplace(a.buf, std::make_pair(i, i)).first;
-                    it->second.second = i;
-                }
-        std::vector<std::vector<int>> begin(out.size()), end(out.size());
+        std::map<int, std::pair<size_t, size_t>> life;   // buffer -> first and last launch or phase
+        size_t now = 0;
+        for (size_t i = from; i < out.size(); ++i) {
+            const Launch& l = out[i].launch;
+            size_t phase = 0;
+            for (size_t a = 0; a < l.args.size(); ++a) {
+                while (phase < l.phase_ends.size() && a >= l.phase_ends[phase]) ++phase;
+                if (l.args[a].kind != Arg::BUF || plan->buffers[(size_t)l.args[a].buf].kind != PlanBuffer::TEMP) continue;
+                auto it = life.emplace(l.args[a].buf, std::make_pair(now + phase, now + phase)).first;
+                it->second.second = now + phase;
+            }
+            now += std::max<size_t>(l.phase_ends.size(), 1);
+        }
+        std::vector<std::vector<int>> begin(now), end(now);
         for (auto& kv : life) {
             begin[kv.second.first].push_back(kv.first);
             end[kv.second.second].push_back(kv.first);
         }
-        for (size_t i = from; i < out.size(); ++i) {
-            for (int b : begin[i]) plan->buffers[(size_t)b].slot = p.take(plan->buffers[(size_t)b].elems);
-            for (int b : end[i]) p.slots[(size_t)plan->buffers[(size_t)b].slot].second = false;
+        for (size_t t = 0; t < now; ++t) {
+            for (int b : begin[t]) plan->buffers[(size_t)b].slot = p.take(plan->buffers[(size_t)b].elems);
+            for (int b : end[t]) p.slots[(size_t)plan->buffers[(size_t)b].slot].second = false;
         }
     }
 
@@ -1621,6 +1629,7 @@ struct Lowerer {
                 calls += strf("    seg%zu::%s(guard%s);\n", q - i, kd.entry.c_str(), args.c_str());
                 if (q + 1 < j) calls += "    __syncthreads();\n";
                 merged.args.insert(merged.args.end(), l.args.begin(), l.args.end());
+                merged.phase_ends.push_back(merged.args.size());
                 merged.bytes += l.bytes;
                 merged.flops += l.flops;
             }

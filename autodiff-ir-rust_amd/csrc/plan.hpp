@@ -46,6 +46,7 @@ struct Launch {
     std::string label;
     double bytes = 0, flops = 0;  // algorithmic work of one launch
     int stat = -1;                // index into Plan::stats
+    std::vector<size_t> phase_ends;  // a run of phases: where the arguments of each end
     std::vector<Launch> parts;    // a shared launch: the launches it does the work of, in the order of the program
 };
 

@@ -59,6 +59,17 @@ def test_members_share_no_memory_that_one_of_them_writes(build):
                     assert owner.setdefault(slot[b], b) == b, (s, label, b)
 
 
+@pytest.mark.parametrize("build", [W.readme_mlp, lambda d: W.mlp_train(d, 3, (5, 4, 4, 2), 2)], ids=["readme", "perceptron"])
+def test_phases_of_one_launch_share_memory_as_launches_do(build, monkeypatch):
+    """A temporary whose last phase is over is memory for the phases behind it."""
+    monkeypatch.setenv("ADHIP_SHARE_INDEPENDENT", "0")
+    slots = lambda: int(re.search(r"temp slots: (\d+)", _plan(build)).group(1))  # noqa: E731
+    together, text = slots(), _plan(build)
+    assert "[merged]" in text
+    monkeypatch.setenv("ADHIP_MERGE_SMALL", "0")
+    assert together <= slots(), text
+
+
 def test_large_launches_stay_apart():
     text = _plan(lambda d: W.mlp_train(d, 4096, (4096, 4096, 4096, 1024), 2))
     for s in _sets(text):
