@@ -4270,9 +4270,7 @@ struct Lowerer {
 };
 
 void describe_launch(const Launch& l, const Plan& p, const std::string& pad, std::string& o) {
-    // (what only lays the next launch's operands out is not called a launch of the program's)
-    const char* what = p.kernels[l.kernel].kind == "attention_split" ? "lays out" : "launch";
-    o += pad + strf("%s %s [%s] kernel=%s grid=(%u,%u,%u) block=%u bytes=%.0f flops=%.0f args:", what, l.label.c_str(),
+    o += pad + strf("launch %s [%s] kernel=%s grid=(%u,%u,%u) block=%u bytes=%.0f flops=%.0f args:", l.label.c_str(),
                     p.kernels[l.kernel].kind.c_str(), p.kernels[l.kernel].entry.c_str(), l.grid[0], l.grid[1], l.grid[2],
                     l.block[0], l.bytes, l.flops);
     for (const Arg& a : l.args) {
@@ -4323,8 +4321,12 @@ void describe_steps(const std::vector<Step>& steps, const Plan& p, int indent, s
 
 std::string Plan::describe() const {
     std::string o;
-    const size_t own = (size_t)std::count_if(kernels.begin(), kernels.end(), [](const KernelDef& k) { return k.kind != "shared"; });
-    o += strf("buffers: %zu (temp slots: %zu), kernels: %zu\n", buffers.size(), slot_elems.size(), own);
+    size_t shared = 0, parts = 0;
+    for (const KernelDef& k : kernels) {
+        shared += k.kind == "shared";
+        parts += k.part_only;
+    }
+    o += strf("buffers: %zu (temp slots: %zu), kernels: %zu (shared: %zu, parts of shared ones only: %zu)\n", buffers.size(), slot_elems.size(), kernels.size(), shared, parts);
     for (size_t i = 0; i < buffers.size(); ++i) {
         const PlanBuffer& b = buffers[i];
         o += strf("  #%zu %s %s elems=%lld%s%s\n", i, b.kind == PlanBuffer::HOME ? "home" : (b.kind == PlanBuffer::TEMP ? "temp" : "const"),
