@@ -3794,20 +3794,24 @@ struct Lowerer {
                         tile(bm, bn, 32, kDirectWaves);
                     }
                 }
-            cfg.narrow_m = M < cfg.bm;
-            cfg.narrow_n = N < cfg.bn;
-            cfg.wide_lines = long_lines;
         }
-        // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits> forces tile and k ranges of every product with k of 64 and more
+        // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits>[,8] forces tile and k ranges of every product with k of 64 and more; tiles
+        // with 32 in them, and with an 8 behind it 64x64, are those without a staging buffer
         if (const char* e = getenv("ADHIP_DOT_PLAN")) {
-            long fbm = 0, fbn = 0, fs = 0;
-            if (sscanf(e, "%ld,%ld,%ld", &fbm, &fbn, &fs) == 3 && K >= 64 && fs >= 1) {
-                const bool known = (fbm == 256 && fbn == 256) || (fbm == 128 && (fbn == 128 || fbn == 64)) || (fbm == 64 && fbn == 64);
+            long fbm = 0, fbn = 0, fs = 0, waves = 0;
+            if (sscanf(e, "%ld,%ld,%ld,%ld", &fbm, &fbn, &fs, &waves) >= 3 && K >= 64 && fs >= 1) {
+                const bool direct = (fbm == 32 || fbm == 64) && (fbn == 32 || fbn == 64) && (fbm + fbn < 128 || waves == kDirectWaves);
+                const bool known = direct || (fbm == 256 && fbn == 256) || (fbm == 128 && (fbn == 128 || fbn == 64)) || (fbm == 64 && fbn == 64);
                 if (known) {
-                    tile((int)fbm, (int)fbn, fbm == 256 ? 16 : 32, fbm == 128 && fbn == 128 ? 2 : 1);
+                    tile((int)fbm, (int)fbn, fbm == 256 ? 16 : 32, direct ? kDirectWaves : fbm == 128 && fbn == 128 ? 2 : 1);
                     want = std::min<int64_t>(fs, K / 64);
                 }
             }
+        }
+        if (cfg.k_waves == kDirectWaves) {
+            cfg.narrow_m = M < cfg.bm;
+            cfg.narrow_n = N < cfg.bn;
+            cfg.wide_lines = long_lines;
         }
         pl.bn_tile = cfg.bn;
         if (want > 1) {
@@ -3821,11 +3825,13 @@ struct Lowerer {
     }
 
     static std::string dot_kernel_name(const GemmConfig& cfg) {
-        std::string s = strf("adhip_gemm_%c%c_%d", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', std::max(cfg.bm, 64));
-        if (cfg.bm > 64 && gemm_tile_columns(cfg) == 64) s += "x64";
+        const bool direct = cfg.k_waves == kDirectWaves;
+        std::string s = strf("adhip_gemm_%c%c_%d", cfg.a_kcontig ? 'k' : 'm', cfg.b_kcontig ? 'k' : 'n', cfg.bm);
+        if (direct || (cfg.bm > 64 && gemm_tile_columns(cfg) == 64)) s += strf("x%d", gemm_tile_columns(cfg));
         if (cfg.edge) s += cfg.bf16_parts || cfg.edge_vec ? "_rim" : "_edge";
         if (cfg.split_k) s += "_splitk";
-        else if (cfg.k_waves > 1) s += "_pair";
+        else if (cfg.k_waves == 2) s += "_pair";
+        if (direct) s += "_direct";
         if (!cfg.bf16_parts) s += "_f32";
         return s;
     }

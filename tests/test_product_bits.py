@@ -20,8 +20,8 @@ from adhip.device import lower_describe
 TILES = [  # m, n, k, kernel
     (4096, 4096, 64, "256"), (3990, 4011, 277, "256_rim"), (2048, 4096, 96, "128"), (4100, 3900, 48, "128_rim"),
     (2048, 2048, 512, "128_pair"), (2100, 2000, 530, "128_rim_pair"), (1024, 1024, 2048, "128_splitk"), (1000, 1100, 2050, "128_rim_splitk"),
-    (2048, 2048, 128, "128x64"), (2100, 2100, 260, "128x64_rim"), (1024, 2048, 64, "64"), (1500, 1100, 40, "64_rim"), (128, 128, 128, "64_pair"),
-    (65, 63, 65, "64_rim_pair"), (64, 64, 2048, "64_splitk"), (100, 130, 1500, "64_rim_splitk"),
+    (2048, 2048, 128, "128x64"), (2100, 2100, 260, "128x64_rim"), (1024, 2048, 64, "64"), (1500, 1100, 40, "64_rim"), (128, 128, 128, "32x32_direct"),
+    (65, 63, 65, "32x32_rim_direct"), (64, 64, 2048, "32x32_splitk_direct"), (100, 130, 1500, "32x32_rim_splitk_direct"),
     # k below 32: the FP32 matrix cores
     (4096, 4096, 16, "256_f32"), (3072, 3072, 16, "128_f32"), (2900, 3000, 16, "128_rim_f32"), (4096, 4096, 31, "128_rim_f32"), (2048, 2048, 16, "128x64_f32"),
     (2100, 2100, 7, "128x64_rim_f32"), (128, 128, 16, "64_f32"), (96, 100, 31, "64_rim_f32")]
@@ -130,7 +130,7 @@ def test_exact_products(tile, layout, hip_device):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["kn", "kk", "mn", "mk"])
-@pytest.mark.parametrize("tile", [t for t in TILES if t[3] in ("256_rim", "128_rim_pair", "64_rim_pair", "128_rim_f32")], ids=lambda t: f"{t[3]}-{t[0]}x{t[1]}x{t[2]}")
+@pytest.mark.parametrize("tile", [t for t in TILES if t[3] in ("256_rim", "128_rim_pair", "32x32_rim_direct", "128_rim_f32")], ids=lambda t: f"{t[3]}-{t[0]}x{t[1]}x{t[2]}")
 def test_exact_products_added_in_place(tile, layout, hip_device):
     """w += a b on the accumulators: one FP32 addition to an exact product."""
     m, n, k, kernel = tile
@@ -155,7 +155,7 @@ def test_error_of_sums(tile, layout, hip_device):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("count,m,n,k,kernel", [(16, 2048, 512, 16, "kn_256_f32"), (5, 500, 500, 64, "kn_64_rim"), (5, 500, 64, 500, "kn_64_rim_pair"),
+@pytest.mark.parametrize("count,m,n,k,kernel", [(16, 2048, 512, 16, "kn_256_f32"), (5, 500, 500, 64, "kn_64_rim"), (5, 500, 64, 500, "kn_32x32_rim_direct"),
                                                 (8, 2048, 128, 1024, "kn_64"), (8, 2048, 128, 2048, "kn_128_splitk"), (4, 1000, 132, 2050, "kn_128_rim_splitk"), (8, 2000, 132, 2050, "kn_128_rim_pair"), (6, 1536, 1536, 96, "kn_256"),
                                                 (7, 1500, 1500, 50, "kn_256_rim"), (16, 100, 100, 31, "kn_64_rim_f32")])
 def test_exact_products_grouped(count, m, n, k, kernel, hip_device):
