@@ -1,6 +1,7 @@
 """Attention on the bf16 matrix cores: every width of heads it takes compiles without spilled registers, and values at the edges
 of its tiles of 32 keys, its eight key groups and its blocks of 64 rows, and where its parts cannot represent an operand."""
 import math
+import re
 
 import numpy as np
 import pytest
@@ -94,6 +95,46 @@ def test_values(sq, sk, d, dv, hip_device, monkeypatch):
     got = _program(hip_device, q, k, v, 16).val().get()
     # a score is a sum of d products of size 1, over 4: its error, 2^-24 sqrt(d) sqrt(d) / 4 at most, is the probability's relative one
     assert_close(got.data, _exact(q, k, v, 16).reshape(-1), RED_RTOL * math.sqrt(max(sk, d)), "o")
+
+
+def _heads_in_one_matrix(dev, q, w, heads, d, dv):
+    """Every head's query, keys and values are columns of wider matrices, keys and values of one."""
+    autodiff.set_device(dev)
+    Q, KV = (autodiff.tensor(x.reshape(-1), list(x.shape)) for x in (q, w))
+    out = []
+    for h in range(heads):
+        k0, v0 = 4 + h * d, 4 + heads * d + h * dv
+        out.append(nn.Attention(Q.r(range(h * d, (h + 1) * d), 1), KV.r(range(k0, k0 + d), 1), KV.r(range(v0, v0 + dv), 1), 16))
+        out[-1].forward()
+        out[-1].val().keep()
+    autodiff.execute()
+    return out
+
+
+@pytest.mark.parametrize("d,dv", [(64, 32), (128, 128)])
+def test_strided_operands_are_read_where_they_are(d, dv):
+    dev, heads, sk = Capture(), 3, 400
+    width = heads * (d + dv) + 8
+    _heads_in_one_matrix(dev, np.zeros((65, heads * d), np.float32), np.zeros((sk, width), np.float32), heads, d, dv)
+    text = lower_describe(dev.proc, dev.deps)
+    assert text.count("[attention_split]") == 1 and "[copy]" not in text and "[elw]" not in text, text
+    assert re.search(rf"\.parts#\d+ {sk} {width} {width}\n", text) and f" 65 {sk} {heads * d} {width} {width} " in text, text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,dv", WIDTHS)
+@pytest.mark.parametrize("sq,sk", [(65, 385), (130, 512)])
+def test_strided_operands(sq, sk, d, dv, hip_device):
+    """The columns that belong to no head are NaN."""
+    heads = 3
+    print(f"[case] attention in parts {sq}x{sk} d {d} dv {dv}, {heads} heads in one matrix", flush=True)
+    rng = np.random.default_rng(sq + 3 * sk + 7 * d + dv)
+    q, w = rng.standard_normal((sq, heads * d)).astype(np.float32), rng.standard_normal((sk, heads * (d + dv) + 8)).astype(np.float32)
+    w[:, :4] = w[:, -4:] = np.nan
+    for h, o in enumerate(_heads_in_one_matrix(hip_device, q, w, heads, d, dv)):
+        k0, v0 = 4 + h * d, 4 + heads * d + h * dv
+        want = _exact(q[:, h * d:(h + 1) * d], w[:, k0:k0 + d], w[:, v0:v0 + dv], 16)
+        assert_close(o.val().get().data, want.reshape(-1), RED_RTOL * math.sqrt(max(sk, d)), f"o{h}")   # (as above)
 
 
 @pytest.mark.gpu
