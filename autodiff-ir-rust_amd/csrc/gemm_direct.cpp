@@ -310,7 +310,7 @@ std::string gemm_direct_kernel_source(const GemmConfig& cfg, const std::string& 
     }
     if ((int)wave < steps) multiply(1);
 #if A_KCONTIG || B_KCONTIG
-    __syncthreads();   // partial results overwrite other wavefronts' lines
+    __syncthreads();   // (a wavefront's partial result takes the place of its own lines, which it has read by then)
 #endif
     // Partial results go to LDS column by column (part[i][j][4 g + r] is row 8 g + 4 lh + r of block i, column li of
     // block j), and a wavefront for each 32x32 block adds them up.

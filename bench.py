@@ -4,8 +4,8 @@
 A step is one pass of the hot path (every kernel of the lowered program, to EX) over one batch of
 synthetic input that is already resident in HBM; the timed steps are queued back to back on the
 device's stream (`adhip_program_enqueue`) between two waits (`adhip_program_sync`).  The headline workload is
-BASELINE.json configs[1]: fused element-wise + broadcast, forward and backward, 8192x8192 f32.
-The other configs are measured too (shorter) and reported under "extra".
+fused element-wise + broadcast, forward and backward, 8192x8192 f32.
+The other workloads are measured too (shorter) and reported under "extra".
 
 Prints ONE JSON line.
 """
@@ -21,7 +21,6 @@ for p in (ROOT, os.path.join(ROOT, "autodiff-ir-rust_amd")):
         sys.path.insert(0, p)
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, published
-FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix, published (the attention kernel, products with k below 32)
 # FP32 products on the bf16 matrix cores: six products of bf16 parts each (dense bf16, published, over six)
 BF16_PARTS_PEAK_TFLOPS = 2500.0 / 6
 # Bytes per launch between the L2 caches and the memory fabric, from rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by a plain
@@ -30,14 +29,14 @@ BF16_PARTS_PEAK_TFLOPS = 2500.0 / 6
 TRAFFIC_BYTES = {
     # 2 x 393277.1 KiB fetched + 1081785.4 KiB written (the 4 outputs and two [512][8192] partial column-sum buffers)
     "fused_elw": {"elw_colsum": int((2 * 393277.1 + 1081785.4) * 1024)},
-    # the one pass of configs[2] (dx with row and column sums riding along): 2 x 131353.0 KiB fetched + 278577.4 KiB
+    # the one pass of the reductions (dx with row and column sums riding along): 2 x 131353.0 KiB fetched + 278577.4 KiB
     # written (dx, the [512][4096] partial column sums, one run sum per row and 256 columns)
     "reductions": {"elw_colsum": int((2 * 131353.0 + 278577.4) * 1024)},
     # the stand-alone reductions (profiles/reductions_forward_and_row_chains.hbm_traffic_pmc.txt), by kernel kind and
     # tensors per launch: fetched x 2 + written (the column reduction writes a row of partial sums per 64 rows)
     "reductions_forward": {("reduce_row", 1): int((2 * 131085.5 + 512.0) * 1024), ("reduce_col", 1): int((2 * 131088.5 + 4096.0) * 1024),
                            ("reduce_row", 3): int((2 * 393230.0 + 1536.4) * 1024), ("reduce_col", 3): int((2 * 393233.5 + 12288.0) * 1024)},
-    # gather stage of configs[4] (one tiled element-wise launch): 2 x 73777.4 KiB fetched + 294912.0 KiB written
+    # gather stage of the manipulation program (one tiled element-wise launch): 2 x 73777.4 KiB fetched + 294912.0 KiB written
     "manip_loop": {"gather_stage": int((2 * 73777.4 + 294912.0) * 1024)},
 }
 
@@ -117,7 +116,7 @@ def cpu_baseline_fused_elw(rows, cols):
            "kind": "port", "sample": f"fused_elw forward+backward on {rows}x{cols} f32 ({rows}/8192 of the rows), "
            f"{dt:.2f} s wall; rate on the same {wl.algorithmic_bytes:.0f} bytes as the GPU figure (the port itself stores "
            f"every intermediate, as the reference does)", "seconds": dt}
-    # the other two rooflines, on bounded samples: configs[2] whole, and one 2048^3 product of configs[3]'s kind
+    # the other two rooflines, on bounded samples: the reductions whole, and one 2048^3 product
     import numpy as np
     from oracle.interp import ref_dot
     wl3 = W.reductions(OracleDevice(), 16384, 4096, seed=0)
@@ -135,7 +134,7 @@ def cpu_baseline_fused_elw(rows, cols):
 
 
 def measure_mlp(dev, iters):
-    """`iters` training steps inside one resident program run."""
+    """A perceptron of 4096-4096-4096-1024, batch 4096: `iters` training steps inside one resident program run."""
     from adhip import workloads as W
     wl4 = W.mlp_train(dev, 4096, (4096, 4096, 4096, 1024), iters, seed=0)
     p4 = compile_resident(dev, wl4)
@@ -198,8 +197,8 @@ def measure_attention(dev, seq=2048, d_model=1024, heads=8):
 
 def measure_reductions_forward(dev, rows=16384, cols=4096):
     """The stand-alone reduction kernels at HBM size (what a forward-only `x.pow(2).sum(1)` / `x.sum(0)` runs: in the
-    forward + backward step of configs[2] the sums ride on the element-wise pass instead).  Three programs: configs[2]
-    without its backward pass; row sums of three different 256 MiB tensors; column sums of the same three.  With three
+    forward + backward step of the reductions the sums ride on the element-wise pass instead).  Three programs: the
+    reductions without their backward pass; row sums of three different 256 MiB tensors; column sums of the same three.  With three
     tensors in turn no launch finds its operand in the 256 MiB last-level cache."""
     import numpy as np
     from adhip import autodiff
@@ -244,7 +243,7 @@ def measure_reductions_forward(dev, rows=16384, cols=4096):
 
 
 def measure_last_layer_products(dev):
-    """The three products of configs[3]'s last layer (4096 -> 1024, batch 4096) on their own, without epilogues:
+    """The three products of the perceptron's last layer (4096 -> 1024, batch 4096) on their own, without epilogues:
     y = x W (A rows contiguous), dW = x^T dy (A columns contiguous), dx = dy W^T (both along k).  With
     ADHIP_DOT_PLAN=<bm>,<bn>,<splits> in the environment the library launches them with that tile and that many ranges
     of k instead of its own choice, which is how alternative tiles are timed."""
@@ -308,9 +307,9 @@ def main():
                          "the known-size reference that hardware byte counters are scaled by; "
                          "'streammix': only a bare 3-reads + 4-writes kernel over 8192x8192 f32 (the stream mix of the "
                          "headline pass with trivial arithmetic and no column sums: what the memory system gives that mix); "
-                         "'reductions': only configs[2]; 'reductions_forward': only the stand-alone row and column reduction "
+                         "'reductions': only the reductions over 16384x4096; 'reductions_forward': only the stand-alone row and column reduction "
                          "kernels on 256 MiB tensors; 'last_layer_products': the three 4096x1024x4096-shaped products of "
-                         "configs[3]'s last layer on their own (honours ADHIP_DOT_PLAN); 'mlp': only configs[3]; 'manip': only configs[4] (one run: its "
+                         "the perceptron's last layer on their own (honours ADHIP_DOT_PLAN); 'mlp': only its training; 'manip': only the gather with its loop (one run: the "
                          "loop consumes its counter); 'attention': only multi-head attention forward; 'encoder': only the encoder "
                          "layer, with its per-kernel list")
     args = ap.parse_args()
