@@ -2995,7 +2995,7 @@ struct Lowerer {
         for (auto* set : sets) {
             auto& kv = *set;
             if (kv.second.size() < 2) continue;
-            const size_t n_buf = (size_t)kv.first[8];
+            const size_t n_buf = gks[kv.second[0]].k.buffer_args.size();
             const size_t cap = std::max<size_t>(1, std::min<size_t>(16, 96 / std::max<size_t>(1, n_buf)));
             std::vector<size_t> leads;
             for (size_t f : kv.second) {
