@@ -3598,12 +3598,14 @@ struct Lowerer {
         cfg.d = (int)key.d;
         cfg.dv = (int)key.dv;
         cfg.mask = key.m_ld > 0;
-        // Parts from 256 keys on, from 384 where a value has more features than a key.  Below, the kernel that writes them and
-        // the merging of eight key groups (of which 160 keys fill five) weigh more than the products (heads x rows x keys x
-        // features, FP32 matrix cores and parts, in us): 8x2048x64x64 8.2, 12.9; 16x4096x64x32 11.7, 24.2; 8x192x192x64 12.8, 13.4;
-        // 16x4096x192x64 39.1, 41.3; 16x4096x224x128 78.4, 80.9; 8x256x256x64 15.7, 13.9; 16x4096x256x32 30.5, 29.4;
-        // 16x4096x256x128 88.1, 84.1; 8x384x384x64 21.1, 16.1; keys of 32 and values of 128 features 8x2048x256 19.4, 20.7, x384 26.1, 24.4.
-        const int64_t parts_from = opt.attention_parts_from ? opt.attention_parts_from : cfg.dv > cfg.d ? 384 : 256;
+        // Parts from 256 keys on; keys of 32 features, and of 64 with values of 128, from 321 on; keys of 64 and fewer than 64 query
+        // rows from 257 on.  Below, the kernel that writes the parts and the merging of eight key groups weigh more than the
+        // products.  Heads x rows x keys x features, FP32 matrix cores and parts, in us a run: 8x2048x64x64 8.2, 12.9;
+        // 8x192x192x64 12.8, 13.4; 8x64x256x32 11.1, 12.1, x320 12.8, 13.1, x352 14.6, 13.1; values of 128 beside keys of 64: 8x1x320
+        // 0.96 of the time, x352 1.08; 8x1x256x64 0.97, x257 1.03, 8x64x256x64 1.03, 16x4096x256x64 1.16; of 96 and 128 features 1.02 to
+        // 1.22 at 256 keys, 1.2 to 1.4 at 384, of 1 to 16 heads and 1 to 4096 rows.
+        const int64_t narrow_from = cfg.d == 64 && key.sq < 64 ? 257 : 256;
+        const int64_t parts_from = opt.attention_parts_from ? opt.attention_parts_from : cfg.d == 32 || (cfg.d == 64 && cfg.dv == 128) ? 321 : narrow_from;
         cfg.parts = opt.attention_parts && !cfg.mask && key.sk >= std::max<int64_t>(parts_from, 32) && attention_takes_parts(cfg.d, cfg.dv);
         // On the FP32 matrix cores a launch with two or more blocks per CU runs blocks of four wavefronts on tiles of 32 keys,
         // two of which fit a CU's LDS while the heads are not too wide; a smaller launch splits every tile between two groups

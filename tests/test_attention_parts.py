@@ -48,7 +48,8 @@ def test_every_width_compiles_without_spills(d, dv):
 
 
 @pytest.mark.parametrize("sq,sk,d,dv", [(64, 31, 64, 64), (64, 400, 48, 48), (64, 400, 64, 48), (64, 400, 160, 128),
-                                        (2048, 255, 64, 64), (64, 32, 32, 32), (300, 300, 32, 64), (64, 383, 64, 128)])
+                                        (2048, 255, 64, 64), (64, 32, 32, 32), (300, 300, 32, 64), (2048, 320, 32, 32), (64, 320, 64, 128),
+                                        (63, 256, 64, 64), (1, 256, 64, 32)])
 def test_what_it_does_not_take_stays_on_the_fp32_ones(sq, sk, d, dv):
     dev = Capture()
     _program(dev, *_zeros(sq, sk, d, dv), 64)
@@ -56,7 +57,7 @@ def test_what_it_does_not_take_stays_on_the_fp32_ones(sq, sk, d, dv):
     assert "[attention]" in text and "_parts" not in text, text
 
 
-@pytest.mark.parametrize("sq,sk,d,dv", [(64, 256, 64, 64), (1, 256, 128, 32), (64, 384, 64, 128)])
+@pytest.mark.parametrize("sq,sk,d,dv", [(64, 256, 64, 64), (1, 257, 64, 64), (1, 256, 128, 32), (1, 256, 96, 128), (64, 321, 64, 128), (1, 321, 32, 32)])
 def test_what_it_takes(sq, sk, d, dv, monkeypatch):
     dev = Capture()
     _program(dev, *_zeros(sq, sk, d, dv), 64)
