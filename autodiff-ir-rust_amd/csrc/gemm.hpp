@@ -15,7 +15,7 @@ struct GemmConfig {
     int bn = 0;             // its columns; 0 = the FP32 kernel's for bm (128, or 64 for bm 64)
     bool bf16_parts = false;  // the kernel on the bf16 matrix cores (gemm_split.cpp); needs K >= bk
     bool split_k = false;   // of that kernel: blockIdx.y picks a range of k (extra argument k_chunk); slice y of the product goes to C + y*M*N
-    int bk = 16;            // k depth of a tile: 16 or 32, on the FP32 matrix cores 16
+    int bk = 16;            // k depth of a tile: 16, 32 or 64, on the FP32 matrix cores 16
     // of that kernel: 2 = a tile's k is shared between two sets of wavefronts, whose sums are added at the end; kDirectWaves =
     // the kernel without a staging buffer (gemm_direct.cpp), whose eight wavefronts share k in steps of 32
     int k_waves = 1;

@@ -21,7 +21,8 @@
 //   128x128x16  4 wavefronts of 64x64, two blocks per CU: 710-770 us
 //   128x128x32  8 wavefronts, two per 64x64 sub-tile with half of the k-tile each: one block per CU does what two of
 //               the former do (4096 x 1024 x 4096: 181-188 us against 326 on 128x64 FP32 tiles)
-//   128x64x32, 64x64x32: outputs of a few hundred blocks with a short k (smaller ones: gemm_direct.cpp)
+//   128x64x32, 64x64x32, 64x64x64 (two sets): outputs of a few hundred blocks with a short k, or a long one in ranges (other
+//               small ones: gemm_direct.cpp)
 // Ragged sizes cost little: rows beyond the product repeat its last row, and the last k-tile starts inside the one
 // before it, with zeros for the k it shares (4000 x 4011 x 4001: 615-665 us against 1567).
 #include "gemm.hpp"

@@ -3799,9 +3799,21 @@ struct Lowerer {
                         tile(bm, bn, 32, kDirectWaves);
                     }
                 }
+            // Where that is 64x64, staging through LDS is faster from k = 128 to 448 (eight steps of 32 have a wavefront each, a ninth
+            // makes one of them wait; without and with a staging buffer 169 x 428 x 156 of eight 8.6 us, 7.4; 640 x 1344 x 256 9.0,
+            // 7.8; 192 x 640 x 448 of eight 15.2, 12.5; but 1234 x 496 x 87 6.2, 6.7; 508 x 663 x 461 of two 12.4, 13.1; 1415 x 139 x 616 of
+            // three 13.7, 14.9), with a k of one tile of 64 beside all but the smallest (160 x 1024 of five 6.2, 5.0; 174 x 529 of
+            // five 5.1, 4.7), and with ranges of k, two blocks to a CU (320 x 256 x 3264 14.3, 13.3; 436 x 64 x 2367 of three 14.7,
+            // 13.6; 155 x 76 x 2292 of five 16.6, 13.8).
+            if (cfg.bm == 64 && cfg.bn == 64 && want > 1) {
+                tile(64, 64, 32, 1);
+                want = std::max<int64_t>(std::min<int64_t>((512 + blocks64 - 1) / blocks64, max_splits), 1);
+            } else if ((K == 64 && cfg.bm + cfg.bn > 64) || (cfg.bm + cfg.bn == 128 && K >= 128 && K <= 448)) {
+                tile(64, 64, 64, 2);
+            }
         }
-        // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits>[,8] forces tile and k ranges of every product with k of 64 and more; tiles
-        // with 32 in them, and with an 8 behind it 64x64, are those without a staging buffer
+        // diagnostic: ADHIP_DOT_PLAN=<bm>,<bn>,<splits>[,<waves>] forces tile and k ranges of every product with k of 64 and more;
+        // tiles with 32 in them, and with an 8 behind it 64x64, are those without a staging buffer, 64x64 with a 2 is the one whose k two sets of wavefronts share
         if (const char* e = getenv("ADHIP_DOT_PLAN")) {
             long fbm = 0, fbn = 0, fs = 0, waves = 0;
             if (sscanf(e, "%ld,%ld,%ld,%ld", &fbm, &fbn, &fs, &waves) >= 3 && K >= 64 && fs >= 1) {
@@ -3809,6 +3821,7 @@ struct Lowerer {
                 const bool known = direct || (fbm == 256 && fbn == 256) || (fbm == 128 && (fbn == 128 || fbn == 64)) || (fbm == 64 && fbn == 64);
                 if (known) {
                     tile((int)fbm, (int)fbn, fbm == 256 ? 16 : 32, direct ? kDirectWaves : fbm == 128 && fbn == 128 ? 2 : 1);
+                    if (fbm == 64 && fbn == 64 && waves == 2) tile(64, 64, 64, 2);
                     want = std::min<int64_t>(fs, K / 64);
                 }
             }

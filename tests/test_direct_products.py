@@ -1,11 +1,13 @@
 """The kernel without a staging buffer addresses a step by 32-bit byte offsets unless an operand's lines are long: which of
 the two a product gets, read from the generated source (no tensor of these sizes is ever touched)."""
 import math
+import re
 
 import numpy as np
 import pytest
 
 from adhip import ir as IR
+from adhip.device import lower_describe
 from parity import RED_RTOL, assert_close
 from test_library_cpu import _compile_check
 
@@ -31,6 +33,17 @@ def _program(m, n, k, layout, long_a, long_b, products, values=None):
         cmds += ca + cb + [IR.DotProduct(a=a, b=b, res=f"c{i}")]
         keep.add(f"c{i}")
     return IR.IRProcedure("main", cmds + [IR.EX()]), keep
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (544, 1017, 64, "64_rim_pair"), (544, 1017, 65, "64x64_rim_direct"), (544, 1017, 127, "64x64_rim_direct"), (544, 1017, 128, "64_rim_pair"),
+    (544, 1017, 448, "64_rim_pair"), (544, 1017, 449, "64x64_rim_direct"),
+    (300, 300, 64, "32x32_rim_direct"), (600, 600, 64, "64_rim_pair"), (1000, 500, 128, "32x64_rim_direct"),
+    (320, 256, 3264, "64_splitk"), (128, 128, 3264, "32x32_splitk_direct")])
+def test_where_staging_is_the_faster(m, n, k, kernel):
+    """Sizes beside the lines between the kernels with and without a staging buffer."""
+    text = lower_describe(*_program(m, n, k, "kn", 0, 0, 1))
+    assert re.findall(r"kernel=adhip_gemm_kn_(\w+)", text) == [kernel], text
 
 
 LONG, MIDDLE = 36_000_000, 1 << 21

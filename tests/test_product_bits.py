@@ -22,6 +22,8 @@ TILES = [  # m, n, k, kernel
     (2048, 2048, 512, "128_pair"), (2100, 2000, 530, "128_rim_pair"), (1024, 1024, 2048, "128_splitk"), (1000, 1100, 2050, "128_rim_splitk"),
     (2048, 2048, 128, "128x64"), (2100, 2100, 260, "128x64_rim"), (1024, 2048, 64, "64"), (1500, 1100, 40, "64_rim"), (128, 128, 128, "32x32_direct"),
     (65, 63, 65, "32x32_rim_direct"), (64, 64, 2048, "32x32_splitk_direct"), (100, 130, 1500, "32x32_rim_splitk_direct"),
+    (640, 1344, 256, "64_pair"), (544, 1017, 129, "64_rim_pair"), (1000, 900, 448, "64_rim_pair"), (576, 1024, 64, "64_pair"), (320, 256, 3264, "64_splitk"),
+    (157, 506, 2807, "64_rim_splitk"),
     # k below 32: the FP32 matrix cores
     (4096, 4096, 16, "256_f32"), (3072, 3072, 16, "128_f32"), (2900, 3000, 16, "128_rim_f32"), (4096, 4096, 31, "128_rim_f32"), (2048, 2048, 16, "128x64_f32"),
     (2100, 2100, 7, "128x64_rim_f32"), (128, 128, 16, "64_f32"), (96, 100, 31, "64_rim_f32")]
