@@ -4350,7 +4350,8 @@ std::string Plan::describe() const {
         shared += k.kind == "shared";
         parts += k.part_only;
     }
-    o += strf("buffers: %zu (temp slots: %zu), kernels: %zu (shared: %zu, parts of shared ones only: %zu)\n", buffers.size(), slot_elems.size(), kernels.size(), shared, parts);
+    o += strf("buffers: %zu (temp slots: %zu), kernels: %zu and %zu that run several of them as one launch, never compiled by themselves: %zu\n", buffers.size(),
+              slot_elems.size(), kernels.size() - shared, shared, parts);
     for (size_t i = 0; i < buffers.size(); ++i) {
         const PlanBuffer& b = buffers[i];
         o += strf("  #%zu %s %s elems=%lld%s%s\n", i, b.kind == PlanBuffer::HOME ? "home" : (b.kind == PlanBuffer::TEMP ? "temp" : "const"),

@@ -37,6 +37,28 @@ def test_what_does_not_depend_shares_a_launch():
         assert not ({"dot_cf_64x64x48", "dot_ch_64x48x64"} <= set(s) or {"dot_bm_64x48x8", "dot_bo_48x8x64"} <= set(s)), s
 
 
+def _args(text, label):
+    line = re.search(rf"^\s*launch {label} .*args:(.*)$", text, re.M).group(1)
+    return {int(b) for b in re.findall(r"#(\d+)", line)}
+
+
+@pytest.mark.parametrize("build", [_mlp, lambda d: W.encoder_train(d, 64, 32, 4, 64, 2, seed=3), lambda d: W.encoder_train(d, 50, 40, 5, 72, 2, seed=3)],
+                         ids=["perceptron", "encoder", "encoder-odd"])
+def test_members_share_no_memory_that_one_of_them_writes(build):
+    """Temporaries of launches that run at the same time have slots of their own (written ones: those whose slot another
+    member of the set names through another buffer, or names at all and writes)."""
+    text = _plan(build)
+    slot = {int(b): int(s) for b, s in re.findall(r"#(\d+) temp \S+ elems=\d+ slot=(\d+)", text)}
+    sets = _sets(text)
+    assert sets
+    for s in sets:
+        owner = {}
+        for label in s:
+            for b in _args(text, label):
+                if b in slot:
+                    assert owner.setdefault(slot[b], b) == b, (s, label, b)
+
+
 def _memory(text, written):
     """Per launch of a plan, in its order: (label, step, memory it names, memory it writes, buffers it names, buffers it writes);
     memory is a home buffer or a temporary's slot.  Members of a shared launch have one step.  `written`: per kernel, which of its
@@ -71,7 +93,7 @@ def _hazards(launches, any_of, writes):
 
 @pytest.mark.parametrize("build", [_mlp, lambda d: _mlp(d, 300, (200, 330, 129, 7)), lambda d: W.encoder_train(d, 64, 32, 4, 64, 2, seed=3),
                                    lambda d: W.encoder_train(d, 50, 40, 5, 72, 2, seed=3)], ids=["perceptron", "perceptron-products", "encoder", "encoder-odd"])
-def test_members_share_no_memory_that_one_of_them_writes(build, tmp_path, monkeypatch):
+def test_members_name_no_memory_that_another_one_writes(build, tmp_path, monkeypatch):
     """What a launch writes is read from its kernel's parameters.  No member of a shared launch names memory (a home buffer, or a
     temporary's slot) that another one writes; and two launches that depend on one another when each runs by itself are
     in the same order when some share."""
@@ -109,6 +131,12 @@ def test_phases_of_one_launch_share_memory_as_launches_do(build, monkeypatch):
     assert "[merged]" in text
     monkeypatch.setenv("ADHIP_MERGE_SMALL", "0")
     assert together <= slots(), text
+
+
+def test_kernels_of_shared_launches_are_counted():
+    text = _plan(_mlp)
+    own, shared, parts = map(int, re.search(r"kernels: (\d+) and (\d+) that run several of them as one launch, never compiled by themselves: (\d+)", text).groups())
+    assert 0 < shared <= len(re.findall(r"^\s*shared\w+, one launch", text, re.M)) and parts <= own
 
 
 def test_large_launches_stay_apart():
