@@ -47,7 +47,8 @@ def test_every_width_compiles_without_spills(d, dv):
     assert rc == 0 and "lowered" not in msg, msg
 
 
-@pytest.mark.parametrize("sq,sk,d,dv", [(64, 31, 64, 64), (64, 400, 48, 48), (64, 400, 64, 48), (64, 400, 160, 128),
+@pytest.mark.parametrize("sq,sk,d,dv", [(64, 31, 64, 64), (64, 64, 48, 48), (64, 64, 64, 48), (64, 64, 160, 128),
+                                                        (64, 400, 48, 48), (64, 400, 64, 48), (64, 400, 160, 128),
                                         (2048, 255, 64, 64), (64, 32, 32, 32), (300, 300, 32, 64), (2048, 320, 32, 32), (64, 320, 64, 128),
                                         (63, 256, 64, 64), (1, 256, 64, 32)])
 def test_what_it_does_not_take_stays_on_the_fp32_ones(sq, sk, d, dv):
@@ -88,8 +89,7 @@ def _exact(q, k, v, scale_dim):
 @pytest.mark.gpu
 @pytest.mark.parametrize("d,dv", WIDTHS)
 @pytest.mark.parametrize("sq,sk", [(64, 32), (1, 33), (65, 63), (130, 255), (63, 257), (200, 520)])
-def test_values(sq, sk, d, dv, hip_device, monkeypatch):
-    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")   # also where the other kernel is the faster one
+def test_values(sq, sk, d, dv, hip_device):
     print(f"[case] attention in parts {sq}x{sk} d {d} dv {dv}", flush=True)
     rng = np.random.default_rng(sq + 3 * sk + 7 * d + dv)
     q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((sq, d), (sk, d), (sk, dv)))
@@ -139,11 +139,18 @@ def test_strided_operands(sq, sk, d, dv, hip_device):
 
 
 @pytest.mark.gpu
-def test_operands_that_the_parts_cannot_represent(hip_device, monkeypatch):
+@pytest.mark.parametrize("d,dv", WIDTHS)
+@pytest.mark.parametrize("sq,sk", [(64, 32), (1, 33), (65, 63), (130, 255), (63, 257)])
+def test_values_in_parts_where_the_other_kernel_is_faster(sq, sk, d, dv, hip_device, monkeypatch):
+    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")
+    test_values(sq, sk, d, dv, hip_device)
+
+
+@pytest.mark.gpu
+def test_operands_that_the_parts_cannot_represent(hip_device):
     """A value beyond bf16's largest number and an infinite one: their blocks of 64 rows are what the FP32 matrix cores make of
     them, the others are as before."""
     print("[case] attention in parts, unrepresentable operands", flush=True)
-    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")
     rng = np.random.default_rng(5)
     sq, sk, d, dv = 190, 140, 64, 64
     q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((sq, d), (sk, d), (sk, dv)))
@@ -160,3 +167,9 @@ def test_operands_that_the_parts_cannot_represent(hip_device, monkeypatch):
     assert np.all(np.isnan(got[70]))
     rows = [r for r in range(sq) if r != 70]
     np.testing.assert_allclose(got[rows], _exact(q, k, v, 16)[rows], rtol=0, atol=2e-5)
+
+
+@pytest.mark.gpu
+def test_operands_that_the_parts_cannot_represent_in_parts(hip_device, monkeypatch):
+    monkeypatch.setenv("ADHIP_ATTENTION_PARTS", "32")
+    test_operands_that_the_parts_cannot_represent(hip_device)

@@ -178,7 +178,7 @@ _FUSED_SHAPES = [
 
 
 @pytest.mark.parametrize("sq,sk,d,dv", _FUSED_SHAPES)
-def test_attention_lowers_to_the_fused_kernel(sq, sk, d, dv):
+def test_attention_lowers_to_one_kernel(sq, sk, d, dv):
     from adhip.core import ValueData
     from adhip.device import Device, lower_describe
 
