@@ -484,7 +484,7 @@ def main():
         p5.close()
         # config 4: dense MLP training
         extra["mlp_train"] = measure_mlp(dev, args.mlp_iters)
-        # beyond BASELINE.json's configs: one transformer encoder layer (the caller side's attention modules),
+        # beside these: one transformer encoder layer (the caller side's attention modules),
         # forward + backward, [2048, 1024] activations, 8 heads, feed-forward width 4096
         extra["encoder_layer"] = measure_encoder(dev)
         extra["attention_forward"] = measure_attention(dev)
